@@ -37,6 +37,12 @@ constexpr uint32_t kLevelTile = kLevelBlock * kLevelElems;  // 8192 points
 constexpr int kFinishBlock = 512;      // threads per LDS subtree of the deep tree
 constexpr uint32_t kFinishTile = 2048;  // max points per LDS subtree
 constexpr int kForestBlock = 256;       // threads per forest tree
+// Levels of the forest trees that k_forest_reg builds (pst_forest_build.hip):
+// trees of 31 to 511 points, a wave each (2.99 -> 0.174 ms for 16.7M points
+// in trees of 127). Smaller trees leave most of a wave's lanes to tree ends;
+// trees of 1023 points would need 16 points per lane, whose sort keys alone
+// fill a lane's registers.
+constexpr uint32_t kForestRegMin = 5, kForestRegMax = 9;
 
 template <typename I>
 struct IdStore {
@@ -814,8 +820,9 @@ __host__ __device__ constexpr size_t forest_lds_bytes(uint32_t N) {
 
 template <typename T, typename I>
 __global__ __launch_bounds__(kForestBlock) void k_forest_build(const Point<T, I>* __restrict__ pts, uint64_t n,
-                                                               uint32_t St, uint32_t L, uint32_t N,
-                                                               Node<T, typename IdStore<I>::type>* __restrict__ nodes,
+                                                               uint64_t tree0, uint32_t St, uint32_t L, uint32_t N,
+                                                               Node<T, typename IdStore<I>::type>* nodes, T* submin,
+                                                               typename IdStore<I>::type* ids, T* bounds,
                                                                int* __restrict__ nan_flag) {
   using IS = typename IdStore<I>::type;
   extern __shared__ __align__(16) unsigned char lds[];
@@ -829,7 +836,7 @@ __global__ __launch_bounds__(kForestBlock) void k_forest_build(const Point<T, I>
   uint16_t* o1 = reinterpret_cast<uint16_t*>(bufB + N);
   uint16_t* o2 = o1 + N;
 
-  const uint64_t c = blockIdx.x;
+  const uint64_t c = tree0 + blockIdx.x;
   const uint64_t first = c * St;
   const uint32_t m = static_cast<uint32_t>(n - first < St ? n - first : St);
   for (uint32_t x = threadIdx.x; x < N; x += blockDim.x) {
@@ -867,12 +874,42 @@ __global__ __launch_bounds__(kForestBlock) void k_forest_build(const Point<T, I>
     if (kid[a] != kid[b]) return kid[a] > kid[b];
     return a > b;
   });
+  if (threadIdx.x == 0) {  // the tree's dim1 range
+    bounds[2 * c] = pts[first + o1[0]].dim1_val;
+    bounds[2 * c + 1] = pts[first + o1[m - 1]].dim1_val;
+  }
   for (uint32_t r = threadIdx.x; r < m; r += blockDim.x) bufB[o2[r]] = r;
   __syncthreads();
   for (uint32_t x = threadIdx.x; x < m; x += blockDim.x) bufA[x] = bufB[o1[x]];
   __syncthreads();
+  nodes += c << L;
   lds_build<T, IS>(bufA, bufB, sres, wred, m, 0, reinterpret_cast<const Point<T, IS>*>(pts), LocalPerm{o2, first},
-                   nodes + (c << L));
+                   nodes);
+  // subtree minima of dim2 and the ID array, bottom level first (what
+  // k_submin_level computes), from the records this workgroup wrote
+  submin += c << L;
+  const uint64_t Mp = static_cast<uint64_t>(m) + 1;
+  for (int u = 31 - __clz(static_cast<int>(m)); u >= 0; u--) {
+    for (uint32_t k = threadIdx.x; k < (1u << u); k += blockDim.x) {
+      const int64_t ms = level_size(Mp, u, k);
+      if (ms < 1) continue;
+      const uint32_t s = (1u << u) - 1 + k;
+      T v = nodes[s].dim2;
+      if constexpr (has_id_v<I>) {
+        if (ids) ids[(c << L) + s] = nodes[s].id;
+      }
+      if (ms >= 2) {
+        const T b = submin[2 * s + 1];
+        v = b < v ? b : v;
+      }
+      if (ms >= 3) {
+        const T b = submin[2 * s + 2];
+        v = b < v ? b : v;
+      }
+      submin[s] = v;
+    }
+    __syncthreads();
+  }
 }
 
 // Forest export: per tree the reference's layout for its own slot count,
@@ -1234,7 +1271,8 @@ Status export_typed(size_t n, const void* nodes, void* blob, size_t o1, size_t o
 }
 
 template <typename T, typename I>
-Status forest_build_typed(const void* pts_v, size_t n, size_t St, void* nodes_v, hipStream_t s) {
+Status forest_build_typed(int dtype, int id_dtype, const void* pts_v, size_t n, size_t St, void* nodes_v,
+                          void* submin_v, void* ids_v, void* bounds_v, hipStream_t s) {
   using IS = typename IdStore<I>::type;
   if (n == 0) return Status{};
   uint32_t L = 0;
@@ -1252,9 +1290,19 @@ Status forest_build_typed(const void* pts_v, size_t n, size_t St, void* nodes_v,
   e = flag.alloc(sizeof(int));
   if (e == hipSuccess) e = hipMemsetAsync(flag.p, 0, sizeof(int), s);
   if (e != hipSuccess) return hip_status(e, "Error in allocating construction flag");
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(ntrees)), dim3(kForestBlock), lds, s,
-                     static_cast<const Point<T, I>*>(pts_v), static_cast<uint64_t>(n), static_cast<uint32_t>(St), L,
-                     N, static_cast<Node<T, IS>*>(nodes_v), flag.as<int>());
+  // full trees of kForestRegMin..kForestRegMax levels a wave each, in
+  // registers; a partial last tree and other sizes a workgroup each
+  size_t done = 0;
+  if (L >= kForestRegMin && L <= kForestRegMax && n >= St) {
+    done = n / St;
+    Status st = build_forest_full(dtype, id_dtype, L, pts_v, done, nodes_v, submin_v, ids_v, bounds_v, flag.as<int>(), s);
+    if (!st.ok()) return st;
+  }
+  if (done < ntrees)
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(ntrees - done)), dim3(kForestBlock), lds, s,
+                       static_cast<const Point<T, I>*>(pts_v), static_cast<uint64_t>(n), static_cast<uint64_t>(done),
+                       static_cast<uint32_t>(St), L, N, static_cast<Node<T, IS>*>(nodes_v), static_cast<T*>(submin_v),
+                       static_cast<IS*>(ids_v), static_cast<T*>(bounds_v), flag.as<int>());
   e = hipGetLastError();
   if (e != hipSuccess) return hip_status(e, "Error in launching forest construction");
   int hflag = 0;
@@ -1346,10 +1394,11 @@ Status export_tree(int dtype, int id_dtype, size_t n, const void* nodes_d, void*
 namespace pst {
 
 Status build_forest(int dtype, int id_dtype, const void* pts_d, size_t n, size_t slots_per_tree, void* nodes_d,
-                    hipStream_t stream) {
+                    void* submin_d, void* ids_d, void* bounds_d, hipStream_t stream) {
   return with_t(dtype, [&](auto t) {
     return with_id(id_dtype, [&](auto i) {
-      return forest_build_typed<decltype(t), decltype(i)>(pts_d, n, slots_per_tree, nodes_d, stream);
+      return forest_build_typed<decltype(t), decltype(i)>(dtype, id_dtype, pts_d, n, slots_per_tree, nodes_d, submin_d,
+                                                          ids_d, bounds_d, stream);
     });
   });
 }

@@ -438,12 +438,8 @@ int pst_gpu_arr_create(const void* pt_arr_d, size_t n, int dtype, int id_dtype, 
     pst_gpu_destroy(t);
     return fail(PST_ERR_HIP, m);
   }
-  Status st = pst::build_forest(dtype, id_dtype, pt_arr_d, n, t->slots_per_tree, t->nodes, t->stream);
-  if (st.ok())
-    st = pst::build_submin(dtype, id_dtype, n, t->slots_per_tree, t->nodes, t->submin, t->ids, t->stream);
-  if (st.ok())
-    st = pst::build_forest_bounds(dtype, id_dtype, n, t->slots_per_tree, t->nodes, t->tree_bounds, t->stream);
-  if (st.ok()) st = pst::hip_status(hipStreamSynchronize(t->stream), "Error in synchronising after construction");
+  Status st = pst::build_forest(dtype, id_dtype, pt_arr_d, n, t->slots_per_tree, t->nodes, t->submin, t->ids,
+                                t->tree_bounds, t->stream);
   if (!st.ok()) {
     pst_gpu_destroy(t);
     return fail(st);

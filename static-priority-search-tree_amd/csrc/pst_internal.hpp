@@ -71,8 +71,14 @@ Status export_tree(int dtype, int id_dtype, size_t n, const void* nodes_d, void*
 // ---- forest of shallow trees (pst_build.hip) ----
 // Tree c holds points [c*St, min(n, (c+1)*St)), St = 2^L - 1 <= 2047; its
 // records start at slot c << L of `nodes` (ceil(n/St) << L records).
+// With them the subtree minima, the IDs per slot (null: none) and each
+// tree's dim1 range (what build_submin and build_forest_bounds give).
 Status build_forest(int dtype, int id_dtype, const void* pts_d, size_t n, size_t slots_per_tree, void* nodes_d,
-                    hipStream_t stream);
+                    void* submin_d, void* ids_d, void* bounds_d, hipStream_t stream);
+// The first `ntrees` trees of a forest of full trees of 2^log_n - 1 points,
+// log_n = 5..9 (pst_forest_build.hip); *nan_flag_d is set on a NaN value.
+Status build_forest_full(int dtype, int id_dtype, uint32_t log_n, const void* pts_d, size_t ntrees, void* nodes_d,
+                         void* submin_d, void* ids_d, void* bounds_d, int* nan_flag_d, hipStream_t s);
 // Per-tree reference layouts, trees concatenated: tree c at position c*St
 // of each array; total_slots = (trees - 1)*St + S(last tree's points).
 Status export_forest(int dtype, int id_dtype, size_t n, size_t slots_per_tree, const void* nodes_d, void* blob_d,

@@ -977,10 +977,10 @@ __global__ void k_export(const Node<T, IS>* __restrict__ nodes, uint64_t S,
 // ---------------------------------------------------------------------------
 struct DevBuf {
   void* p = nullptr;
-  ~DevBuf() { release(); }
-  hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1); }
-  void release() {
-    if (p) (void)hipFree(p);
+  ~DevBuf() { (void)dev_free(p); }  // early returns: queued kernels may still use it
+  hipError_t alloc(size_t bytes) { return dev_alloc(&p, bytes); }
+  void release_idle() {  // after the caller has waited for every use
+    (void)dev_free_idle(p);
     p = nullptr;
   }
   template <typename U>
@@ -1239,8 +1239,8 @@ Status build_typed(const void* pts_v, size_t n64, BuildOut& out, hipStream_t s, 
   PST_TRY(hipMemcpyAsync(hflag, flags, sizeof(hflag), hipMemcpyDeviceToHost, s),
           "Error in reading construction flag");
   PST_TRY(hipStreamSynchronize(s), "Error in synchronising after construction");
-  arena_b.release();
-  arena_a.release();
+  arena_b.release_idle();
+  arena_a.release_idle();
   if (times) {
     hipEventElapsedTime(&times->sort_ms, ev[0], ev[1]);
     hipEventElapsedTime(&times->levels_ms, ev[1], ev[2]);
@@ -1309,6 +1309,7 @@ Status forest_build_typed(int dtype, int id_dtype, const void* pts_v, size_t n, 
   e = hipMemcpyAsync(&hflag, flag.p, sizeof(int), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hip_status(e, "Error in synchronising after forest construction");
+  flag.release_idle();
   if (hflag) return Status{3, "Error: input contains NaN values, which have no order"};
   return Status{};
 }
@@ -1368,16 +1369,21 @@ Status build_tree(int dtype, int id_dtype, const void* pts_d, size_t n, void* no
   return build_tree(dtype, id_dtype, pts_d, n, out, stream, times);
 }
 
-size_t build_scratch_bytes(int dtype, int id_dtype, size_t n) {
-  size_t bytes = 0;
-  Status st = with_t(dtype, [&](auto t) {
+namespace {
+BuildLayout layout_of(int dtype, int id_dtype, size_t n) {
+  BuildLayout L{};
+  (void)with_t(dtype, [&](auto t) {
     return with_id(id_dtype, [&](auto i) {
-      bytes = build_layout<BuildKey<decltype(t), decltype(i)>>(n).total;
+      L = build_layout<BuildKey<decltype(t), decltype(i)>>(n);
       return Status{};
     });
   });
-  return st.ok() ? bytes : 0;
+  return L;
 }
+}  // namespace
+
+size_t build_scratch_bytes(int dtype, int id_dtype, size_t n) { return layout_of(dtype, id_dtype, n).total; }
+size_t build_arena_bytes(int dtype, int id_dtype, size_t n) { return layout_of(dtype, id_dtype, n).total_a; }
 
 Status export_tree(int dtype, int id_dtype, size_t n, const void* nodes_d, void* blob_d,
                    size_t o1, size_t o2, size_t om, size_t oi, size_t ob, hipStream_t stream) {

@@ -183,13 +183,13 @@ int blocking_search(pst_tree* t, int kind, int ret, size_t* num, void** res, con
   hipSetDevice(t->device);
   const size_t rec = ret == PST_RET_POINT ? pst_point_size(t->dtype, t->id_dtype) : id_size(t->id_dtype);
   void* out = nullptr;
-  hipError_t e = hipMalloc(&out, t->n * rec);
+  hipError_t e = pst::dev_alloc(&out, t->n * rec);
   if (e != hipSuccess)
     return fail(PST_ERR_HIP, "Error in allocating array to store PointStruct search result" +
                                  dev_suffix(t->dev_ind, t->num_devs) + hipGetErrorString(e));
   int rc = single_search(t, kind, ret, a, b, c, out, t->n, num, t->stream);
   if (rc != PST_OK) {
-    hipFree(out);
+    pst::dev_free(out);
     *res = nullptr;
     return rc;
   }
@@ -211,10 +211,10 @@ Status forest_seg_reserve(pst_tree* t, size_t nq) {
   const size_t need = std::max<size_t>(pst::forest_dense_scratch_bytes(t->n, t->slots_per_tree, nq, cus), 16);
   if (t->sc.fseg_bytes >= need) return Status{};
   if (t->sc.pinned) return Status{1, pst::kPinnedScratchMsg};
-  if (t->sc.fseg) hipFree(t->sc.fseg);
+  if (t->sc.fseg) pst::dev_free(t->sc.fseg);
   t->sc.fseg = nullptr;
   t->sc.fseg_bytes = 0;
-  Status st = pst::hip_status(hipMalloc(&t->sc.fseg, need), "Error in allocating forest search buffers");
+  Status st = pst::hip_status(pst::dev_alloc(&t->sc.fseg, need), "Error in allocating forest search buffers");
   if (st.ok()) t->sc.fseg_bytes = need;
   return st;
 }
@@ -320,7 +320,7 @@ size_t pst_point_size(int dtype, int id_dtype) {
 
 int pst_free(void* p) {
   if (!p) return PST_OK;
-  hipError_t e = hipFree(p);
+  hipError_t e = pst::dev_free(p);
   if (e != hipSuccess) return fail(pst::hip_status(e, "Error in freeing search result array"));
   return PST_OK;
 }
@@ -353,9 +353,9 @@ int pst_gpu_create(const void* pt_arr_d, size_t n, int dtype, int id_dtype, int 
   // so that the allocation overlaps them
   pst::BuildOut bo;
   bo.alloc = [&](pst::BuildOut& o) {
-    hipError_t e = hipMalloc(&t->nodes, t->S * pst::node_size(dtype, id_dtype));
-    if (e == hipSuccess) e = hipMalloc(&t->submin, t->S * pst::dtype_size(dtype));
-    if (e == hipSuccess && id_size(id_dtype) > 0) e = hipMalloc(&t->ids, t->S * id_size(id_dtype));
+    hipError_t e = pst::dev_alloc(&t->nodes, t->S * pst::node_size(dtype, id_dtype));
+    if (e == hipSuccess) e = pst::dev_alloc(&t->submin, t->S * pst::dtype_size(dtype));
+    if (e == hipSuccess && id_size(id_dtype) > 0) e = pst::dev_alloc(&t->ids, t->S * id_size(id_dtype));
     if (e != hipSuccess)
       return Status{PST_ERR_HIP, "Error in allocating priority search tree storage array" +
                                      dev_suffix(dev_ind, num_devs) + hipGetErrorString(e)};
@@ -377,24 +377,15 @@ int pst_gpu_destroy(pst_tree* t) {
   if (!t) return PST_OK;
   if (t->graphs > 0)
     return fail(PST_ERR_INVALID, "Error: the tree still has batch graphs; destroy them before the tree");
-  hipError_t e = hipSuccess;
-  if (t->nodes) e = hipFree(t->nodes);
-  if (t->submin) {
-    hipError_t e2 = hipFree(t->submin);
+  // one wait for the device's work, then every array goes back
+  hipError_t e = t->nodes ? pst::dev_wait(t->nodes) : hipSuccess;
+  const bool idle = e == hipSuccess;
+  for (void* p : {t->nodes, t->submin, t->ids, t->tree_bounds, t->lv_key, t->lv_id}) {
+    const hipError_t e2 = idle ? pst::dev_free_idle(p) : pst::dev_free(p);
     if (e == hipSuccess) e = e2;
   }
-  if (t->ids) {
-    hipError_t e2 = hipFree(t->ids);
-    if (e == hipSuccess) e = e2;
-  }
-  if (t->tree_bounds) {
-    hipError_t e2 = hipFree(t->tree_bounds);
-    if (e == hipSuccess) e = e2;
-  }
-  pst::scratch_release(t->sc);
-  if (t->lv_key) hipFree(t->lv_key);
-  if (t->lv_id) hipFree(t->lv_id);
-  pst::level_scratch_release(t->lsc);
+  pst::scratch_release(t->sc, idle);
+  pst::level_scratch_release(t->lsc, idle);
   const int di = t->dev_ind, nd = t->num_devs;
   delete t;
   if (e != hipSuccess)
@@ -428,10 +419,10 @@ int pst_gpu_arr_create(const void* pt_arr_d, size_t n, int dtype, int id_dtype, 
     *out = t;
     return PST_OK;
   }
-  hipError_t e = hipMalloc(&t->nodes, t->S * pst::node_size(dtype, id_dtype));
-  if (e == hipSuccess) e = hipMalloc(&t->submin, t->S * pst::dtype_size(dtype));
-  if (e == hipSuccess && id_size(id_dtype) > 0) e = hipMalloc(&t->ids, t->S * id_size(id_dtype));
-  if (e == hipSuccess) e = hipMalloc(&t->tree_bounds, pst::forest_bounds_bytes(dtype, n, t->slots_per_tree));
+  hipError_t e = pst::dev_alloc(&t->nodes, t->S * pst::node_size(dtype, id_dtype));
+  if (e == hipSuccess) e = pst::dev_alloc(&t->submin, t->S * pst::dtype_size(dtype));
+  if (e == hipSuccess && id_size(id_dtype) > 0) e = pst::dev_alloc(&t->ids, t->S * id_size(id_dtype));
+  if (e == hipSuccess) e = pst::dev_alloc(&t->tree_bounds, pst::forest_bounds_bytes(dtype, n, t->slots_per_tree));
   if (e != hipSuccess) {
     std::string m = "Error in allocating array of PSTs on device " + std::to_string(dev_ind + 1) +
                     " (1-indexed) of " + std::to_string(num_devs) + ": " + hipGetErrorString(e);
@@ -478,11 +469,11 @@ int pst_gpu_load(const char* path, int dev_ind, int num_devs, pst_stream_t strea
     *out = t;
     return PST_OK;
   }
-  hipError_t e = hipMalloc(&t->nodes, t->S * pst::node_size(t->dtype, t->id_dtype));
-  if (e == hipSuccess) e = hipMalloc(&t->submin, t->S * pst::dtype_size(t->dtype));
-  if (e == hipSuccess && id_size(t->id_dtype) > 0) e = hipMalloc(&t->ids, t->S * id_size(t->id_dtype));
+  hipError_t e = pst::dev_alloc(&t->nodes, t->S * pst::node_size(t->dtype, t->id_dtype));
+  if (e == hipSuccess) e = pst::dev_alloc(&t->submin, t->S * pst::dtype_size(t->dtype));
+  if (e == hipSuccess && id_size(t->id_dtype) > 0) e = pst::dev_alloc(&t->ids, t->S * id_size(t->id_dtype));
   if (e == hipSuccess && t->slots_per_tree)
-    e = hipMalloc(&t->tree_bounds, pst::forest_bounds_bytes(t->dtype, t->n, t->slots_per_tree));
+    e = pst::dev_alloc(&t->tree_bounds, pst::forest_bounds_bytes(t->dtype, t->n, t->slots_per_tree));
   if (e != hipSuccess) {
     std::string m = "Error in allocating priority search tree storage array" + dev_suffix(dev_ind, num_devs) +
                     hipGetErrorString(e);
@@ -561,7 +552,7 @@ size_t pst_gpu_calc_global_mem_needed(size_t n, int dtype, int id_dtype) {
   const size_t S = slots_for(n);
   // resident: node records, subtree minima and the per-slot ID array
   const size_t tree = S * (pst::node_size(dtype, id_dtype) + pst::dtype_size(dtype) + id_size(id_dtype));
-  // construction's buffers, freed when it ends
+  // construction's buffers, kept for the next construction of this size
   const size_t construct = pst::build_scratch_bytes(dtype, id_dtype, n);
   // one blocking search: the handle's search buffers (kept) and a result
   // array of n points (the reference's allocation, pst/static-pst-gpu.tu:563)
@@ -569,7 +560,7 @@ size_t pst_gpu_calc_global_mem_needed(size_t n, int dtype, int id_dtype) {
   hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
   const size_t search = pst::search_scratch_bytes(n, dtype, cus) + n * pst::point_size(dtype, id_dtype);
-  return tree + (construct > search ? construct : search);
+  return tree + construct + search;
 }
 
 size_t pst_gpu_arr_calc_global_mem_needed(size_t n, unsigned threads_per_block, int dtype, int id_dtype) {
@@ -629,7 +620,7 @@ int pst_gpu_export_tree(pst_tree* t, void* host_blob, size_t blob_bytes, size_t*
   if (blob_bytes < need) return fail(PST_ERR_INVALID, "Error: export buffer too small");
   if (t->n == 0) return PST_OK;
   void* d = nullptr;
-  hipError_t e = hipMalloc(&d, need);
+  hipError_t e = pst::dev_alloc(&d, need);
   if (e != hipSuccess) return fail(pst::hip_status(e, "Error in allocating tree export buffer"));
   Status st = t->slots_per_tree
                   ? pst::export_forest(t->dtype, t->id_dtype, t->n, t->slots_per_tree, t->nodes, d, S, off6[0],
@@ -639,7 +630,7 @@ int pst_gpu_export_tree(pst_tree* t, void* host_blob, size_t blob_bytes, size_t*
   if (st.ok()) st = pst::hip_status(hipMemcpyAsync(host_blob, d, need, hipMemcpyDeviceToHost, t->stream),
                                     "Error in copying tree export");
   if (st.ok()) st = pst::hip_status(hipStreamSynchronize(t->stream), "Error in synchronising tree export");
-  hipFree(d);
+  pst::dev_free(d);
   if (!st.ok()) return fail(st);
   return PST_OK;
 }
@@ -798,14 +789,14 @@ int pst_gpu_autotune(pst_tree* t, const void* queries_d, size_t nq, int ret, pst
   void* out = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   auto cleanup = [&]() {
-    if (counts) hipFree(counts);
-    if (offs) hipFree(offs);
-    if (out) hipFree(out);
+    if (counts) pst::dev_free(counts);
+    if (offs) pst::dev_free(offs);
+    if (out) pst::dev_free(out);
     if (e0) hipEventDestroy(e0);
     if (e1) hipEventDestroy(e1);
   };
-  hipError_t e = hipMalloc(&counts, nq * 8);
-  if (e == hipSuccess) e = hipMalloc(&offs, (nq + 1) * 8);
+  hipError_t e = pst::dev_alloc(&counts, nq * 8);
+  if (e == hipSuccess) e = pst::dev_alloc(&offs, (nq + 1) * 8);
   if (e == hipSuccess) e = hipEventCreate(&e0);
   if (e == hipSuccess) e = hipEventCreate(&e1);
   if (e != hipSuccess) {
@@ -822,7 +813,7 @@ int pst_gpu_autotune(pst_tree* t, const void* queries_d, size_t nq, int ret, pst
   if (st.ok()) st = pst::hip_status(hipMemcpyAsync(&total, offs + nq, 8, hipMemcpyDeviceToHost, s), "Error in reading the batch total");
   if (st.ok()) st = pst::hip_status(hipStreamSynchronize(s), "Error in synchronising");
   const size_t rec = ret == PST_RET_POINT ? pst::point_size(t->dtype, t->id_dtype) : id_size(t->id_dtype);
-  if (st.ok()) st = pst::hip_status(hipMalloc(&out, std::max<size_t>(total * rec, 1)), "Error in allocating autotuning output");
+  if (st.ok()) st = pst::hip_status(pst::dev_alloc(&out, std::max<size_t>(total * rec, 1)), "Error in allocating autotuning output");
   if (!st.ok()) {
     cleanup();
     return fail(st);
@@ -957,8 +948,8 @@ int pst_gpu_set_level_index(pst_tree* t, int on) {
     if (t->graphs > 0 && t->lv_key)
       return fail(PST_ERR_INVALID, "Error: a batch graph of this tree uses its level index; destroy the graph first");
     hipSetDevice(t->device);
-    if (t->lv_key) hipFree(t->lv_key);
-    if (t->lv_id) hipFree(t->lv_id);
+    if (t->lv_key) pst::dev_free(t->lv_key);
+    if (t->lv_id) pst::dev_free(t->lv_id);
     t->lv_key = t->lv_id = nullptr;
     pst::level_scratch_release(t->lsc);
     return PST_OK;
@@ -971,13 +962,13 @@ int pst_gpu_set_level_index(pst_tree* t, int on) {
   const size_t elems = pst::level_index_bytes(t->dtype, t->id_dtype, t->n) /
                        (pst::dtype_size(t->dtype) + id_size(t->id_dtype));
   void *k = nullptr, *i = nullptr;
-  hipError_t e = hipMalloc(&k, elems * pst::dtype_size(t->dtype));
-  if (e == hipSuccess) e = hipMalloc(&i, elems * id_size(t->id_dtype));
+  hipError_t e = pst::dev_alloc(&k, elems * pst::dtype_size(t->dtype));
+  if (e == hipSuccess) e = pst::dev_alloc(&i, elems * id_size(t->id_dtype));
   Status st = pst::hip_status(e, "Error in allocating the level index" + dev_suffix(t->dev_ind, t->num_devs));
   if (st.ok()) st = pst::build_level_index(t->dtype, t->id_dtype, t->n, t->nodes, t->ids, k, i, t->stream);
   if (!st.ok()) {
-    if (k) hipFree(k);
-    if (i) hipFree(i);
+    if (k) pst::dev_free(k);
+    if (i) pst::dev_free(i);
     return fail(st);
   }
   t->lv_key = k;
@@ -1152,7 +1143,7 @@ int surface_blocking(IsoCountFn cfn, IsoWriteFn wfn, const void* vertex_arr_d, i
   unsigned long long* err = device_counter(dev);
   if (!err) return fail(PST_ERR_HIP, "Error in allocating a device counter");
   unsigned long long* counts = nullptr;  // counts, then offsets (num_ids + 1)
-  hipError_t e = hipMalloc(&counts, (2 * num_ids + 1) * sizeof(unsigned long long));
+  hipError_t e = pst::dev_alloc(&counts, (2 * num_ids + 1) * sizeof(unsigned long long));
   if (e != hipSuccess) return fail(PST_ERR_HIP, std::string("Error in allocating isosurface counts: ") + hipGetErrorString(e));
   unsigned long long* offsets = counts + num_ids;
   Status st = pst::hip_status(hipMemsetAsync(err, 0, 8, nullptr), "Error in clearing the error flag");
@@ -1166,13 +1157,13 @@ int surface_blocking(IsoCountFn cfn, IsoWriteFn wfn, const void* vertex_arr_d, i
   if (st.ok() && bad) st = Status{PST_ERR_INVALID, "Error: a metacell ID lies past the metacell grid"};
   float* tri = nullptr;
   if (st.ok() && total)
-    st = pst::hip_status(hipMalloc(&tri, total * 9 * sizeof(float)), "Error in allocating the triangle array");
+    st = pst::hip_status(pst::dev_alloc(&tri, total * 9 * sizeof(float)), "Error in allocating the triangle array");
   if (st.ok() && total)
     st = wfn(dtype, id_dtype, vertex_arr_d, p32, m32, metacell_ids_d, num_ids, isovalue, offsets, total, tri, nullptr);
   if (st.ok()) st = pst::hip_status(hipStreamSynchronize(nullptr), "Error in synchronising after isosurface extraction");
-  hipFree(counts);
+  pst::dev_free(counts);
   if (!st.ok()) {
-    if (tri) hipFree(tri);
+    if (tri) pst::dev_free(tri);
     return fail(st);
   }
   *triangles_d = tri;
@@ -1233,7 +1224,7 @@ int pst_form_metacell_tags(const void* vertex_arr_d, int dtype, int id_dtype, co
   const size_t nm = pst_calc_num_metacells(pt_grid_dims, metacell_dims, nullptr);
   if (nm == 0) return fail(PST_ERR_INVALID, "Error: empty metacell grid");
   void* out = nullptr;
-  hipError_t e = hipMalloc(&out, nm * pst::point_size(dtype, id_dtype));
+  hipError_t e = pst::dev_alloc(&out, nm * pst::point_size(dtype, id_dtype));
   if (e != hipSuccess)
     return fail(PST_ERR_HIP, "Error in allocating metacell tag storage array" + dev_suffix(dev_ind, num_devs) +
                                  hipGetErrorString(e));
@@ -1241,7 +1232,7 @@ int pst_form_metacell_tags(const void* vertex_arr_d, int dtype, int id_dtype, co
   if (rc == PST_OK && hipStreamSynchronize(nullptr) != hipSuccess)
     rc = fail(PST_ERR_HIP, "Error in synchronising after metacell formation");
   if (rc != PST_OK) {
-    hipFree(out);
+    pst::dev_free(out);
     return rc;
   }
   *metacell_arr_d = out;
@@ -1273,7 +1264,7 @@ int pst_interval_parallel_search(const void* pt_arr_d, size_t n, int dtype, int 
     return fail(PST_ERR_INVALID, "Error: IDs requested from points without IDs");
   const size_t rec = ret == PST_RET_POINT ? pst::point_size(dtype, id_dtype) : id_size(id_dtype);
   void* out = nullptr;
-  hipError_t e = hipMalloc(&out, (n ? n : 1) * rec);
+  hipError_t e = pst::dev_alloc(&out, (n ? n : 1) * rec);
   if (e != hipSuccess)
     return fail(PST_ERR_HIP, "Error in allocating array to store PointStruct search result" +
                                  dev_suffix(dev_ind, num_devs) + hipGetErrorString(e));
@@ -1281,12 +1272,12 @@ int pst_interval_parallel_search(const void* pt_arr_d, size_t n, int dtype, int 
   hipGetDevice(&dev);
   unsigned long long* ctr = device_counter(dev);
   if (!ctr) {
-    hipFree(out);
+    pst::dev_free(out);
     return fail(PST_ERR_HIP, "Error in allocating global result array index" + dev_suffix(dev_ind, num_devs));
   }
   e = hipMemsetAsync(ctr, 0, 8, nullptr);
   if (e != hipSuccess) {
-    hipFree(out);
+    pst::dev_free(out);
     return fail(PST_ERR_HIP, "Error in initialising global result array index to 0" +
                                  dev_suffix(dev_ind, num_devs) + hipGetErrorString(e));
   }
@@ -1295,7 +1286,7 @@ int pst_interval_parallel_search(const void* pt_arr_d, size_t n, int dtype, int 
   if (st.ok()) st = pst::hip_status(hipMemcpy(&h, ctr, 8, hipMemcpyDeviceToHost),
                                     "Error in copying global result array final index from device");
   if (!st.ok()) {
-    hipFree(out);
+    pst::dev_free(out);
     return fail(st);
   }
   *num = h;

@@ -56,8 +56,10 @@ struct BuildOut {
 Status build_tree(int dtype, int id_dtype, const void* pts_d, size_t n, BuildOut& out, hipStream_t stream,
                   BuildTimes* times = nullptr);
 
-// Device bytes one construction of n points allocates (freed when it ends).
+// Device bytes one construction of n points allocates (freed when it ends),
+// and those of the first of its two blocks (at least 8 B per point).
 size_t build_scratch_bytes(int dtype, int id_dtype, size_t n);
+size_t build_arena_bytes(int dtype, int id_dtype, size_t n);
 // Device bytes a handle keeps for one search of a deep tree of n points
 // (work lists, copy tasks, the overflow stacks of the default grid on a GPU
 // with `cus` compute units), allocated at its first search.
@@ -91,6 +93,24 @@ Status export_forest(int dtype, int id_dtype, size_t n, size_t slots_per_tree, c
 Status build_submin(int dtype, int id_dtype, size_t n, size_t slots_per_tree, const void* nodes_d, void* submin_d,
                     void* ids_d, hipStream_t stream);
 
+// ---- device memory (pst_memory.cpp) ----
+// hipMalloc on the current device through the library's bounded cache of
+// freed blocks (contents undefined).
+hipError_t dev_alloc_bytes(void** p, size_t bytes);
+template <typename U>
+hipError_t dev_alloc(U** p, size_t bytes) {
+  void* v = nullptr;
+  const hipError_t e = dev_alloc_bytes(&v, bytes);
+  *p = static_cast<U*>(v);
+  return e;
+}
+// Waits for the work of the block's device, then frees it (null: nothing).
+hipError_t dev_free(void* p);
+// The same without waiting: the caller has waited for every use of p.
+hipError_t dev_free_idle(void* p);
+// Waits for the work of the device that holds the block p.
+hipError_t dev_wait(const void* p);
+
 // ---- searches on one deep tree (pst_search.hip) ----
 constexpr int kGroup = 8;  // queries per group walk in batched searches
 struct SearchScratch {
@@ -118,7 +138,7 @@ struct SearchScratch {
 extern const char* const kPinnedScratchMsg;
 // Work lists for nq queries whose walks start from `roots` root items.
 Status scratch_reserve(SearchScratch& sc, size_t nq, size_t roots, hipStream_t stream);
-void scratch_release(SearchScratch& sc);
+void scratch_release(SearchScratch& sc, bool idle = false);
 
 // mode 0: count into counts_d[q]; mode 1: write results for query q at
 // out + offsets_d[q] (offsets_d may be null: all offsets 0), at most
@@ -193,7 +213,7 @@ struct LevelScratch {
   int external = 0;                    // the buffers belong to the caller (never freed or grown here)
 };
 Status level_scratch_reserve(LevelScratch& sc, size_t nq);
-void level_scratch_release(LevelScratch& sc);
+void level_scratch_release(LevelScratch& sc, bool idle = false);
 // Batched count (a.mode 0) or ID write (a.mode 1) with the semantics of
 // run_search, through the level index (asynchronous). plan 1 (count): also
 // keep the batch's ranges in the scratch; plan 2 (write): write from the

@@ -658,12 +658,22 @@ Status build_level_index(int dtype, int id_dtype, size_t n, const void* nodes_d,
       hipError_t e = sizeof(K) == 4
                          ? radix_sort_u32(nullptr, tmp_bytes, nullptr, nullptr, nullptr, nullptr, n, s)
                          : radix_sort_u64(nullptr, tmp_bytes, nullptr, nullptr, nullptr, nullptr, n, s);
-      if (e == hipSuccess) e = hipMalloc(&kin, n * sizeof(K));
-      if (e == hipSuccess) e = hipMalloc(&sa, n * 4);
-      if (e == hipSuccess) e = hipMalloc(&sb, n * 4);
-      if (e == hipSuccess) e = hipMalloc(&agg, (ntiles + 1) * 8ull);
-      if (e == hipSuccess) e = hipMalloc(&pre, (ntiles + 1) * 8ull);
-      if (e == hipSuccess) e = hipMalloc(&tmp, std::max<size_t>(tmp_bytes, 16));
+      // The slot arrays take the block that construction of a tree of this
+      // size used and gave back. The sort of level 0 works in the key array's
+      // deeper levels, which are written after it, where they hold it.
+      const size_t slots = build_arena_bytes(dtype, id_dtype, n);
+      const bool inside = H >= 2 && ns * sizeof(K) * (H - 2) >= tmp_bytes && n * 8 <= slots;
+      uint32_t* slot_block = nullptr;
+      void* sort_block = nullptr;
+      if (e == hipSuccess) e = dev_alloc(&slot_block, std::max(slots, n * 8));
+      if (e == hipSuccess) e = dev_alloc(&agg, (ntiles + 1) * 8ull);
+      if (e == hipSuccess) e = dev_alloc(&pre, (ntiles + 1) * 8ull);
+      const size_t kin_bytes = (n * sizeof(K) + 255) & ~size_t{255};
+      if (e == hipSuccess && !inside) e = dev_alloc(&sort_block, kin_bytes + std::max<size_t>(tmp_bytes, 16));
+      sa = slot_block;
+      sb = slot_block + n;
+      kin = inside ? key + ns : static_cast<K*>(sort_block);
+      tmp = inside ? static_cast<void*>(key + 2 * ns) : static_cast<unsigned char*>(sort_block) + kin_bytes;
       Status st = hip_status(e, "Error in allocating level index construction buffers");
       if (st.ok()) {
         const unsigned blocks = (n32 + kLvBlock - 1) / kLvBlock;
@@ -694,12 +704,8 @@ Status build_level_index(int dtype, int id_dtype, size_t n, const void* nodes_d,
         if (st.ok()) st = hip_status(hipGetLastError(), "Error in launching level index construction");
         if (st.ok()) st = hip_status(hipStreamSynchronize(s), "Error in building the level index");
       }
-      if (kin) hipFree(kin);
-      if (sa) hipFree(sa);
-      if (sb) hipFree(sb);
-      if (agg) hipFree(agg);
-      if (pre) hipFree(pre);
-      if (tmp) hipFree(tmp);
+      for (void* p : {static_cast<void*>(slot_block), sort_block, static_cast<void*>(agg), static_cast<void*>(pre)})
+        (void)(st.ok() ? dev_free_idle(p) : dev_free(p));
       return st;
     });
   });
@@ -711,12 +717,12 @@ Status level_scratch_reserve(LevelScratch& sc, size_t nq) {
   if (sc.pinned) return Status{1, kPinnedScratchMsg};
   level_scratch_release(sc);
   const size_t cap = std::max<size_t>(nq, 64);
-  hipError_t e = hipMalloc(&sc.tsrc, cap * kTaskCap * 8);
-  if (e == hipSuccess) e = hipMalloc(&sc.tpre, cap * kTaskCap * 4);
-  if (e == hipSuccess) e = hipMalloc(&sc.ntask, cap * 4);
-  if (e == hipSuccess) e = hipMalloc(&sc.wq, cap * 8);
-  if (e == hipSuccess) e = hipMalloc(&sc.woff, (cap + 1) * 8);
-  if (e == hipSuccess) e = hipMalloc(&sc.chunk_task, kChunkCap * 4);
+  hipError_t e = dev_alloc(&sc.tsrc, cap * kTaskCap * 8);
+  if (e == hipSuccess) e = dev_alloc(&sc.tpre, cap * kTaskCap * 4);
+  if (e == hipSuccess) e = dev_alloc(&sc.ntask, cap * 4);
+  if (e == hipSuccess) e = dev_alloc(&sc.wq, cap * 8);
+  if (e == hipSuccess) e = dev_alloc(&sc.woff, (cap + 1) * 8);
+  if (e == hipSuccess) e = dev_alloc(&sc.chunk_task, kChunkCap * 4);
   if (e != hipSuccess) {
     level_scratch_release(sc);
     return hip_status(e, "Error in allocating level search buffers");
@@ -725,17 +731,14 @@ Status level_scratch_reserve(LevelScratch& sc, size_t nq) {
   return Status{};
 }
 
-void level_scratch_release(LevelScratch& sc) {
+void level_scratch_release(LevelScratch& sc, bool idle) {
   if (sc.external) {
     sc = LevelScratch{};
     return;
   }
-  if (sc.tsrc) hipFree(sc.tsrc);
-  if (sc.tpre) hipFree(sc.tpre);
-  if (sc.ntask) hipFree(sc.ntask);
-  if (sc.wq) hipFree(sc.wq);
-  if (sc.woff) hipFree(sc.woff);
-  if (sc.chunk_task) hipFree(sc.chunk_task);
+  for (void* p : {static_cast<void*>(sc.tsrc), static_cast<void*>(sc.tpre), static_cast<void*>(sc.ntask),
+                  static_cast<void*>(sc.wq), static_cast<void*>(sc.woff), static_cast<void*>(sc.chunk_task)})
+    (void)(idle ? dev_free_idle(p) : dev_free(p));
   sc = LevelScratch{};
 }
 

@@ -173,11 +173,11 @@ struct Staging {
   void* dev = nullptr;
   ~Staging() {
     if (host) hipHostFree(host);
-    if (dev) hipFree(dev);
+    if (dev) dev_free(dev);
   }
   Status alloc(size_t bytes) {
     hipError_t e = hipHostMalloc(&host, bytes, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMalloc(&dev, bytes);
+    if (e == hipSuccess) e = dev_alloc(&dev, bytes);
     return hip_status(e, "Error in allocating tree file staging buffers");
   }
 };

@@ -998,10 +998,10 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
   const size_t gbytes = static_cast<size_t>(grid) * P.gcap * sizeof(Items::type);
   if (sc.gstack_bytes < gbytes) {
     if (sc.pinned) return Status{1, kPinnedScratchMsg};
-    if (sc.gstack) hipFree(sc.gstack);
+    if (sc.gstack) dev_free(sc.gstack);
     sc.gstack = nullptr;
     sc.gstack_bytes = 0;
-    e = hipMalloc(&sc.gstack, gbytes);
+    e = dev_alloc(&sc.gstack, gbytes);
     if (e != hipSuccess) return hip_status(e, "Error in allocating search overflow stacks");
     sc.gstack_bytes = gbytes;
   }
@@ -1010,10 +1010,10 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
     const size_t want = a.copy_tasks > 0 ? std::min(a.copy_tasks, kCopyTaskCap) : kCopyTaskCap;
     if (sc.task_cap < want) {
       if (sc.pinned) return Status{1, kPinnedScratchMsg};
-      if (sc.tasks) hipFree(sc.tasks);
+      if (sc.tasks) dev_free(sc.tasks);
       sc.tasks = nullptr;
       sc.task_cap = 0;
-      e = hipMalloc(&sc.tasks, want * sizeof(CopyTask));
+      e = dev_alloc(&sc.tasks, want * sizeof(CopyTask));
       if (e != hipSuccess) return hip_status(e, "Error in allocating the copy task list");
       sc.task_cap = want;
     }
@@ -1116,58 +1116,51 @@ Status scratch_reserve(SearchScratch& sc, size_t nq, size_t roots, hipStream_t) 
                     (nq > 1 && sc.gcap < nq);
   if (grow && sc.pinned) return Status{1, kPinnedScratchMsg};
   if (sc.list_cap < need) {
-    if (sc.list[0]) hipFree(sc.list[0]);
-    if (sc.list[1]) hipFree(sc.list[1]);
+    if (sc.list[0]) dev_free(sc.list[0]);
+    if (sc.list[1]) dev_free(sc.list[1]);
     sc.list[0] = sc.list[1] = nullptr;
     sc.list_cap = 0;
-    hipError_t e = hipMalloc(&sc.list[0], need * sizeof(Entry));
-    if (e == hipSuccess) e = hipMalloc(&sc.list[1], need * sizeof(Entry));
+    hipError_t e = dev_alloc(&sc.list[0], need * sizeof(Entry));
+    if (e == hipSuccess) e = dev_alloc(&sc.list[1], need * sizeof(Entry));
     if (e != hipSuccess) return hip_status(e, "Error in allocating search work lists");
     sc.list_cap = need;
   }
   if (!sc.ctr) {
-    hipError_t e = hipMalloc(&sc.ctr, (2 * kMaxRounds + 4) * sizeof(unsigned long long));
+    hipError_t e = dev_alloc(&sc.ctr, (2 * kMaxRounds + 4) * sizeof(unsigned long long));
     if (e != hipSuccess) return hip_status(e, "Error in allocating search counters");
   }
   if (sc.cursor_cap < std::max<size_t>(nq, 1)) {
-    if (sc.cursor) hipFree(sc.cursor);
-    hipError_t e = hipMalloc(&sc.cursor, std::max<size_t>(nq, 1) * 8);
+    if (sc.cursor) dev_free(sc.cursor);
+    hipError_t e = dev_alloc(&sc.cursor, std::max<size_t>(nq, 1) * 8);
     if (e != hipSuccess) return hip_status(e, "Error in allocating result cursors");
     sc.cursor_cap = std::max<size_t>(nq, 1);
   }
   if (nq > 1 && sc.gcap < nq) {
     // group table (padded to whole groups) and the sort's keys and values
     const size_t cap = ((nq + kGroup - 1) / kGroup) * kGroup;
-    if (sc.groups) hipFree(sc.groups);
-    if (sc.gkeys) hipFree(sc.gkeys);
-    if (sc.gtmp) hipFree(sc.gtmp);
+    if (sc.groups) dev_free(sc.groups);
+    if (sc.gkeys) dev_free(sc.gkeys);
+    if (sc.gtmp) dev_free(sc.gtmp);
     sc.groups = nullptr;
     sc.gkeys = sc.gtmp = nullptr;
     sc.gcap = 0;
     size_t t64 = 0, t32 = 0;
     hipError_t e = radix_sort_u64(nullptr, t64, nullptr, nullptr, nullptr, nullptr, cap, nullptr);
     if (e == hipSuccess) e = radix_sort_u32(nullptr, t32, nullptr, nullptr, nullptr, nullptr, cap, nullptr);
-    if (e == hipSuccess) e = hipMalloc(&sc.groups, cap * 4);
-    if (e == hipSuccess) e = hipMalloc(&sc.gkeys, cap * (2 * 8 + 4 * 4));
+    if (e == hipSuccess) e = dev_alloc(&sc.groups, cap * 4);
+    if (e == hipSuccess) e = dev_alloc(&sc.gkeys, cap * (2 * 8 + 4 * 4));
     sc.gtmp_bytes = std::max<size_t>(std::max(t64, t32), 16);
-    if (e == hipSuccess) e = hipMalloc(&sc.gtmp, sc.gtmp_bytes);
+    if (e == hipSuccess) e = dev_alloc(&sc.gtmp, sc.gtmp_bytes);
     if (e != hipSuccess) return hip_status(e, "Error in allocating query grouping storage");
     sc.gcap = cap;
   }
   return Status{};
 }
 
-void scratch_release(SearchScratch& sc) {
-  if (sc.list[0]) hipFree(sc.list[0]);
-  if (sc.list[1]) hipFree(sc.list[1]);
-  if (sc.ctr) hipFree(sc.ctr);
-  if (sc.cursor) hipFree(sc.cursor);
-  if (sc.groups) hipFree(sc.groups);
-  if (sc.gkeys) hipFree(sc.gkeys);
-  if (sc.gtmp) hipFree(sc.gtmp);
-  if (sc.gstack) hipFree(sc.gstack);
-  if (sc.tasks) hipFree(sc.tasks);
-  if (sc.fseg) hipFree(sc.fseg);
+void scratch_release(SearchScratch& sc, bool idle) {
+  for (void* p : {sc.list[0], sc.list[1], static_cast<void*>(sc.ctr), static_cast<void*>(sc.cursor),
+                  static_cast<void*>(sc.groups), sc.gkeys, sc.gtmp, sc.gstack, sc.tasks, sc.fseg})
+    (void)(idle ? dev_free_idle(p) : dev_free(p));
   sc = SearchScratch{};
 }
 

@@ -46,9 +46,19 @@ constexpr int kLvBlock = 256;
 constexpr int kLvPer = 16;
 constexpr uint32_t kLvTile = kLvBlock * kLvPer;  // points per partition tile
 constexpr uint32_t kTaskCap = 128;               // ranges per query: <= 4 per level, <= 31 levels
-constexpr uint32_t kSearchBit = 0x80000000u;     // range needs a binary search (a REPORT_ABOVE subtree)
-constexpr uint64_t kMinChunk = 32768;            // IDs per copy chunk (at least)
-constexpr uint64_t kChunkCap = 1u << 20;         // chunk table entries
+constexpr uint32_t kFewQueries = 64;             // write plans of up to this many queries probe wider
+// Copy chunks and workgroups. Queries of kLongQuery IDs and more on average
+// copy best in large chunks by three workgroups per CU (2-4 beat 8 on the
+// 2^26 f32 batch of 1.8M IDs per query); shorter ones spend their time
+// moving between queries and ranges, where more workgroups hide each other's
+// waits: 8192 queries of 14,500 IDs 342 -> 272 us with eight per CU and half
+// the chunk. A small batch is cut into about three chunks per CU (one query
+// of 1.5M IDs 33 -> 13 us: chunks of 32768 left 210 of 256 CUs idle).
+constexpr uint64_t kLongQuery = 65536;
+constexpr uint64_t kMinChunk = 1024, kChunkShort = 16384, kChunkLong = 32768;
+constexpr uint64_t kChunkSpread = 768;
+constexpr uint32_t kCopyPerCu = 8, kCopyPerCuLong = 3;
+constexpr uint64_t kChunkCap = 1u << 20;  // chunk table entries
 constexpr int kCopyBlock = 256;
 constexpr int kCopyBytes = 256;  // bytes of loads in flight per lane in the copy
 constexpr uint32_t kFlat = 4096;  // positions per flat pass of the copy (16 per lane)
@@ -251,10 +261,15 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_scatter(const uint32_t* __restr
   }
 }
 
-__host__ __device__ inline uint64_t chunk_len(uint64_t W) {
+// IDs per chunk of a batch of nq queries that writes W IDs.
+__host__ __device__ inline uint64_t chunk_len(uint64_t W, uint64_t nq) {
   uint64_t c = (W + kChunkCap - 1) / kChunkCap;
   c = (c + 255) & ~255ull;
-  return c > kMinChunk ? c : kMinChunk;
+  const uint64_t most = W >= nq * kLongQuery ? kChunkLong : kChunkShort;
+  if (c >= most) return c;
+  uint64_t f = (W / kChunkSpread + 255) & ~255ull;
+  f = f < kMinChunk ? kMinChunk : (f > most ? most : f);
+  return f > c ? f : c;
 }
 
 template <typename T, typename IS>
@@ -283,104 +298,147 @@ struct LvParams {
   uint32_t* chunk_task;      // and its chunk table
 };
 
-// One workgroup (one wave) per query: the open paths, level by level, then
-// the REPORT_ABOVE subtrees' binary searches, one lane per subtree.
-template <typename T, typename IS, bool W>
+// First index of the sorted run kk[0, len) whose key is above qk: a search
+// with PROBES (3 or 7) loads in flight per step, which narrows the run 4 or 8
+// times per memory round trip.
+template <int PROBES, typename K>
+__device__ inline uint32_t run_prefix(const K* __restrict__ kk, uint32_t len, K qk) {
+  static_assert(PROBES == 3 || PROBES == 7, "quarters or eighths");
+  constexpr uint32_t kParts = PROBES + 1;
+  uint32_t lo = 0, hi = len;
+  while (lo < hi) {
+    const uint32_t w = hi - lo;
+    uint32_t p[PROBES];
+    K v[PROBES];
+#pragma unroll
+    for (int k = 0; k < PROBES; k++) {
+      p[k] = lo + (w / kParts) * (k + 1) + ((w % kParts) * (k + 1)) / kParts;  // lo + floor(w (k + 1) / kParts) < hi
+      v[k] = kk[p[k]];
+    }
+    uint32_t nlo = lo, nhi = hi;
+#pragma unroll
+    for (int k = 0; k < PROBES; k++)
+      if (v[k] <= qk) nlo = p[k] + 1;
+#pragma unroll
+    for (int k = PROBES - 1; k >= 0; k--)
+      if (!(v[k] <= qk)) nhi = p[k];
+    lo = nlo;
+    hi = nhi;
+  }
+  return lo;
+}
+
+// One workgroup (one wave) per query: the open paths, then the REPORT_ABOVE
+// subtrees' run searches, one lane per subtree.
+//
+// Bound by the chain of dependent loads, one per tree level and one per
+// search step when taken singly. So the wave loads five levels of the (at
+// most two) path nodes' subtrees at once, 31 nodes each on lanes 0-30 and
+// 31-61, steps the paths down through the lanes' registers (a lane takes its
+// state from its parent's lane), and starts again from the nodes reached;
+// the closed-form starts of the ranges, a loop over the levels each, are left
+// to the end, where every lane has a range of its own; and the searches keep
+// several probes in flight. MI355X, 2^26 f32 points: one query 62 -> 20 us,
+// 1024 queries 99 -> 27 us; 8192 queries on 2^25 i32 points 113 -> 41 us.
+constexpr uint32_t kSpecLevels = 5;                      // levels loaded at once
+constexpr uint32_t kSpecNodes = (1u << kSpecLevels) - 1;  // nodes per path
+template <typename T, typename IS, bool W, int PROBES>
 __global__ __launch_bounds__(kWave) void k_lv_plan(LvParams<T, IS> P) {
   using K = key_of<T>;
-  __shared__ uint64_t s_src[kTaskCap];
-  __shared__ uint32_t s_len[kTaskCap];
+  __shared__ uint64_t s_src[kTaskCap];  // first: level << 33 | searched << 32 | position; then the source
   const uint32_t lane = threadIdx.x;
   const uint32_t q = blockIdx.x;
   const Query<T> Q = P.use_single ? P.single : P.queries[q];
   const Bounds<T> qb{Q.min_dim1, Q.max_dim1, Q.min_dim2};
   const BoundNum bn = bound_num<T, 1>(&qb);
   const uint64_t ns = P.ns;
-  // a path node: slot | l << 32 | h << 33 | valid << 34
-  constexpr uint64_t kValid = 1ull << 34;
-  uint64_t mine = lane == 0 ? (kValid | (static_cast<uint64_t>(lo_open(Q.kind)) << 32) |
-                               (static_cast<uint64_t>(hi_open(Q.kind)) << 33))
-                            : 0ull;
+  // the lane's place in its path's block
+  const uint32_t blk = lane >= kSpecNodes ? 1u : 0u;
+  const uint32_t r = lane - blk * kSpecNodes;
+  const uint32_t rd = 31u - static_cast<uint32_t>(__builtin_clz(r + 1));  // depth in the block
+  const bool in_block = lane < 2 * kSpecNodes;
+  const int parent = static_cast<int>(blk * kSpecNodes + (r ? (r - 1) / 2 : 0));
+  // path states: 4 valid, 2 upper bound open, 1 lower bound open
+  uint32_t root[2] = {0, 0};
+  uint32_t state[2] = {4u | lo_open(Q.kind) | (hi_open(Q.kind) << 1), 0u};
   uint32_t ntask = 0;
-  for (uint32_t t = 0; t < P.H; t++) {
-    if (__ballot((mine & kValid) != 0) == 0) break;
-    uint32_t emit = 0;  // bit 0: own point, bit 1: a REPORT_ABOVE child
-    uint64_t own_src = 0, ra_src = 0;
-    uint32_t ra_size = 0;
-    uint64_t nx0 = 0, nx1 = 0;
-    uint32_t nnx = 0;
-    if (mine & kValid) {
-      const uint32_t slot = static_cast<uint32_t>(mine);
-      const uint32_t l = static_cast<uint32_t>(mine >> 32) & 1u, h = static_cast<uint32_t>(mine >> 33) & 1u;
-      const Node<T, IS> nd = P.nodes[slot];
-      const int32_t m = subtree_size32(P.M, slot);
-      const StepOut o = node_step<T, 1>(nd.dim1, nd.dim2, nd.med, m, &qb, bn, 1u, l, h);
-      const uint32_t j = slot + 1u - (1u << t);
-      if (o.rep) {
-        emit |= 1u;
-        own_src = static_cast<uint64_t>(t) * ns + static_cast<uint64_t>(level_start(P.M, t, j));
-      }
-      auto child = [&](uint32_t a, uint32_t cl, uint32_t ch, uint32_t side) {
-        if (!a) return;
-        const uint32_t cs = 2u * slot + 1u + side;
-        if (!cl && !ch) {
-          emit |= 2u;
-          const uint32_t cjj = 2u * j + side;
-          ra_src = static_cast<uint64_t>(t + 1) * ns + static_cast<uint64_t>(level_start(P.M, t + 1, cjj));
-          ra_size = static_cast<uint32_t>(level_size(P.M, t + 1, cjj));
-        } else {
-          const uint64_t e = kValid | cs | (static_cast<uint64_t>(cl) << 32) | (static_cast<uint64_t>(ch) << 33);
-          if (nnx == 0) nx0 = e;
-          else nx1 = e;
-          nnx++;
+  for (uint32_t t = 0; t < P.H && (state[0] | state[1]); t += kSpecLevels) {
+    const uint32_t rs = blk ? root[1] : root[0], rst = blk ? state[1] : state[0];
+    const uint32_t depth = t + rd;
+    const uint32_t slot = ((rs + 1) << rd) + r - (1u << rd);
+    int32_t m = 0;
+    if (in_block && rst && depth < P.H) m = subtree_size32(P.M, slot);
+    const Node<T, IS> nd = P.nodes[m >= 1 ? slot : 0u];
+    uint32_t st = r == 0 && m >= 1 ? rst : 0u;
+    uint32_t kids = 0;  // open children: left state | right state << 3
+#pragma unroll
+    for (uint32_t d = 0; d < kSpecLevels; d++) {
+      bool rep = false, ra = false;
+      uint32_t side = 0;
+      kids = 0;
+      if (rd == d && st) {
+        const StepOut o = node_step<T, 1>(nd.dim1, nd.dim2, nd.med, m, &qb, bn, 1u, st & 1u, (st >> 1) & 1u);
+        rep = o.rep != 0;
+        const uint32_t ol = o.ll | (o.hl << 1), orr = o.lr | (o.hr << 1);
+        if (o.al) {
+          if (ol) kids |= 4u | ol;
+          else ra = true;
         }
-      };
-      child(o.al, o.ll, o.hl, 0u);
-      child(o.ar, o.lr, o.hr, 1u);
-    }
-    // ranges of this level: lane 0's (own, subtree), then lane 1's
-    const uint32_t c0 = __shfl(__builtin_popcount(emit), 0, kWave);
-    if (lane < 2 && emit) {
-      uint32_t at = ntask + (lane == 0 ? 0u : c0);
-      if (emit & 1u) {
-        s_src[at] = own_src;
-        s_len[at] = 1u;
-        at++;
+        if (o.ar) {
+          if (orr) kids |= (4u | orr) << 3;
+          else {
+            ra = true;
+            side = 1;
+          }
+        }
       }
-      if (emit & 2u) {
-        s_src[at] = ra_src;
-        s_len[at] = ra_size | kSearchBit;
+      // ranges in path order (left to right), a node's own point first
+      const uint64_t b1 = __ballot(rep), b2 = __ballot(ra);
+      uint32_t at = ntask + lanes_below(b1) + lanes_below(b2);
+      const uint32_t j = slot + 1u - (1u << depth);
+      if (rep) s_src[at++] = (static_cast<uint64_t>(depth) << 33) | j;
+      if (ra) s_src[at] = (static_cast<uint64_t>(depth + 1) << 33) | (1ull << 32) | (2u * j + side);
+      ntask += static_cast<uint32_t>(__popcll(b1) + __popcll(b2));
+      if (d + 1 < kSpecLevels) {
+        const uint32_t up = static_cast<uint32_t>(__shfl(static_cast<int>(kids), parent, kWave));
+        if (rd == d + 1) st = m >= 1 ? ((r & 1u) ? up & 7u : up >> 3) : 0u;
       }
     }
-    ntask += c0 + __shfl(__builtin_popcount(emit), 1, kWave);
-    // next level's paths: lane 0's (at most two), then lane 1's (at most one)
-    const uint64_t a0 = __shfl(nx0, 0, kWave), a1 = __shfl(nx1, 0, kWave), b0 = __shfl(nx0, 1, kWave);
-    const uint32_t k0 = __shfl(nnx, 0, kWave);
-    const uint64_t p0 = k0 >= 1 ? a0 : b0;
-    const uint64_t p1 = k0 >= 2 ? a1 : (k0 == 1 ? b0 : 0ull);
-    mine = lane == 0 ? p0 : (lane == 1 ? p1 : 0ull);
+    // the paths' nodes below the block, left to right (at most two)
+    uint64_t bl = __ballot((kids & 7u) != 0), br = __ballot((kids >> 3) != 0);
+    state[0] = state[1] = 0;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const uint64_t any = bl | br;
+      if (any) {
+        const int f = __builtin_ctzll(any);
+        const uint64_t bit = 1ull << f;
+        const bool left = (bl & bit) != 0;
+        const uint32_t ps = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(slot), f));
+        const uint32_t kd = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(kids), f));
+        root[k] = 2 * ps + (left ? 1u : 2u);
+        state[k] = left ? kd & 7u : kd >> 3;
+        if (left) bl &= ~bit;
+        else br &= ~bit;
+      }
+    }
   }
   __syncthreads();
-  // binary searches: points of the subtree's run with key <= ~ord_key(min2)
+  // each range's place in the level arrays and its length: one for a node's
+  // own point, else the points of the subtree's run with key <= ~ord_key(min2)
   const K qk = ~ord_key(qb.min2);
   uint32_t cnt[2] = {0, 0};
 #pragma unroll
-  for (int r = 0; r < 2; r++) {
-    const uint32_t i = lane + r * kWave;
+  for (int h = 0; h < 2; h++) {
+    const uint32_t i = lane + h * kWave;
     if (i < ntask) {
-      const uint32_t len = s_len[i];
-      if (len & kSearchBit) {
-        const K* kk = P.key + s_src[i];
-        uint32_t lo = 0, hi = len & ~kSearchBit;
-        while (lo < hi) {
-          const uint32_t mid = (lo + hi) >> 1;
-          if (kk[mid] <= qk) lo = mid + 1;
-          else hi = mid;
-        }
-        cnt[r] = lo;
-      } else {
-        cnt[r] = len;
-      }
+      const uint64_t e = s_src[i];
+      const uint32_t t = static_cast<uint32_t>(e >> 33), j = static_cast<uint32_t>(e);
+      const uint64_t src = static_cast<uint64_t>(t) * ns + static_cast<uint64_t>(level_start(P.M, t, j));
+      s_src[i] = src;
+      cnt[h] = (e >> 32) & 1u
+                   ? run_prefix<PROBES>(P.key + src, static_cast<uint32_t>(level_size(P.M, t, j)), qk)
+                   : 1u;
     }
   }
   // inclusive prefix over the ranges in order
@@ -437,7 +495,7 @@ __global__ __launch_bounds__(kWave) void k_lv_plan(LvParams<T, IS> P) {
           P.woff[0] = 0;
           P.woff[1] = clip;
         }
-        const uint64_t L = chunk_len(clip);
+        const uint64_t L = chunk_len(clip, 1);
         auto mark = [&](uint32_t at, uint32_t pre, uint32_t c) {
           const uint64_t a = pre, b = pre + c < cw ? pre + c : cw;
           for (uint64_t ch = (a + L - 1) / L; ch * L < b; ch++) P.chunk_task[ch] = at;
@@ -488,7 +546,7 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_mark(const unsigned long long* 
   const uint64_t g = static_cast<uint64_t>(blockIdx.x) * kLvBlock + threadIdx.x;
   const uint32_t q = static_cast<uint32_t>(g / kTaskCap), i = static_cast<uint32_t>(g % kTaskCap);
   if (q >= nq || i >= ntask[q]) return;
-  const uint64_t L = chunk_len(woff[nq]);
+  const uint64_t L = chunk_len(woff[nq], nq);
   const uint64_t base = woff[q];
   const uint64_t qb = static_cast<uint64_t>(q) * kTaskCap;
   const uint64_t a = base + tpre[qb + i], b = base + tpre[qb + i + 1];
@@ -529,10 +587,13 @@ __global__ __launch_bounds__(kCopyBlock) void k_lv_copy(const IS* __restrict__ i
   __shared__ uint32_t s_pre[kTaskCap + 1];
   __shared__ uint64_t s_src[kTaskCap];
   const uint64_t W = woff[nq];
-  const uint64_t L = chunk_len(W);
+  const uint64_t L = chunk_len(W, nq);
   const uint64_t nch = (W + L - 1) / L;
   const uint32_t tid = threadIdx.x;
-  for (uint64_t c = blockIdx.x; c < nch; c += gridDim.x) {
+  // the grid is kCopyPerCu workgroups per CU
+  const uint32_t grid = W >= nq * kLongQuery ? gridDim.x / kCopyPerCu * kCopyPerCuLong : gridDim.x;
+  if (blockIdx.x >= grid) return;
+  for (uint64_t c = blockIdx.x; c < nch; c += grid) {
     const uint32_t e = chunk_task[c];
     uint32_t q = e >> 7, i = e & 127u;
     uint64_t x = c * L;
@@ -784,14 +845,16 @@ Status level_search(const SearchArgs& a, const void* key_d, const void* id_d, Le
       P.chunk_task = sc.chunk_task;
       if (a.mode == 0) {
         P.keep = plan == 1;
-        hipLaunchKernelGGL((k_lv_plan<T, IS, false>), dim3(P.nq), dim3(kWave), 0, s, P);
+        hipLaunchKernelGGL((k_lv_plan<T, IS, false, 3>), dim3(P.nq), dim3(kWave), 0, s, P);
         return hip_status(hipGetLastError(), "Error in launching level search");
       }
       if (plan == 2) {
         hipLaunchKernelGGL(k_lv_clip, dim3((P.nq + kLvBlock - 1) / kLvBlock), dim3(kLvBlock), 0, s, sc.tpre, sc.ntask,
                            sc.wq, a.counts, a.offsets, a.caps, a.cap_all, P.out_total, P.nq);
       } else {
-        hipLaunchKernelGGL((k_lv_plan<T, IS, true>), dim3(P.nq), dim3(kWave), 0, s, P);
+        // few queries leave the memory system idle: more probes per search step
+        if (P.nq <= kFewQueries) hipLaunchKernelGGL((k_lv_plan<T, IS, true, 7>), dim3(P.nq), dim3(kWave), 0, s, P);
+        else hipLaunchKernelGGL((k_lv_plan<T, IS, true, 3>), dim3(P.nq), dim3(kWave), 0, s, P);
       }
       if (!(P.use_single && plan != 2)) {  // a single query's plan wrote these itself
         Status st = exclusive_scan(sc.wq, sc.woff, a.nq, s);
@@ -803,9 +866,7 @@ Status level_search(const SearchArgs& a, const void* key_d, const void* id_d, Le
       int dev = 0, cus = 0;
       hipGetDevice(&dev);
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      // three workgroups per CU: measured on the 2^26 batch, 2-4 beat 8
-      // (fewer waves, each with 256 B of loads in flight)
-      hipLaunchKernelGGL((k_lv_copy<IS>), dim3(static_cast<unsigned>(cus * 3)), dim3(kCopyBlock), 0, s, P.id,
+      hipLaunchKernelGGL((k_lv_copy<IS>), dim3(static_cast<unsigned>(cus * kCopyPerCu)), dim3(kCopyBlock), 0, s, P.id,
                          sc.tsrc, sc.tpre, sc.ntask, sc.woff, a.offsets, sc.chunk_task, P.nq,
                          static_cast<IS*>(a.out));
       return hip_status(hipGetLastError(), "Error in launching level search");

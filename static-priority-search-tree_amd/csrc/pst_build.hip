@@ -6,17 +6,19 @@
 // parallelism, pst/static-pst-gpu-populate-tree.tu:10-158) with rank arrays
 // and level-synchronous passes:
 //
-//   1. key2 ranks: r2[i] = position of point i in the key2-descending order
-//      (key2 = (dim2, id, index), the reference's compareDim2 order).
-//   2. A = r2 listed in key1-ascending order (key1 = (dim1, id, index)).
-//      From here on construction only compares 32-bit ranks.
-//   3. Level t holds 2^t segments of A, one per slot, in slot order; their
-//      sizes and offsets follow from n alone (pst_common.hpp). Per segment,
-//      the node is the minimum rank (max key2); med is the dim1 of the
-//      floor(m/2)-th remaining point; removing the node from A (a coalesced
-//      compaction) yields level t+1, whose left/right segments are the
-//      first floor(m/2) / the remaining points.
-//   4. Once every segment fits in LDS (<= kFinishTile points), one
+//   1. The points are listed in key1 order as values that compare like
+//      key2 (the smaller value is the greater point). Points with 32-bit
+//      dims and 32-bit IDs that rise with the index sort once, by dim1,
+//      carrying (dim2, ID) as a 64-bit value from which the node records are
+//      formed: nothing is gathered (point_sort_*, pst_sort.hip). Others
+//      first sort by key2 = (dim2, id, index), and the value is the 32-bit
+//      key2 rank.
+//   2. The levels above LDS size move no point: a static hierarchy of block
+//      minima (64 values each) gives a segment's node as a range minimum,
+//      taken around the at most `level` nodes already removed from the
+//      segment; the median and the children's ranges follow by counting
+//      those. Their sizes follow from n alone (pst_common.hpp).
+//   3. Once every segment fits in LDS (<= kFinishTile points), one
 //      workgroup finishes its whole subtree in LDS.
 // The node chosen, the median rule and the child split are those of the
 // reference's constructNode (pst/static-pst-gpu.tu:706-806 and
@@ -31,9 +33,6 @@ namespace pst {
 
 namespace {
 
-constexpr int kLevelBlock = 256;
-constexpr int kLevelElems = 32;
-constexpr uint32_t kLevelTile = kLevelBlock * kLevelElems;  // 8192 points
 constexpr int kFinishBlock = 512;      // threads per LDS subtree of the deep tree
 constexpr uint32_t kFinishTile = 2048;  // max points per LDS subtree
 constexpr int kForestBlock = 256;       // threads per forest tree
@@ -131,157 +130,135 @@ __global__ void k_scatter_rank(const uint32_t* __restrict__ perm2, uint32_t n, u
   if (p < n) r2[perm2[p]] = p;
 }
 
-// Segment starts of levels 0..t0, slot-indexed (level t at offset 2^t - 1):
-// the closed form of pst_common.hpp, clamped at 0.
-__global__ void k_level_starts(uint64_t M, uint32_t nstart, uint32_t* __restrict__ starts) {
-  const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= nstart) return;
-  const uint32_t t = depth_of(idx);
-  const uint32_t j = idx + 1u - (1u << t);
-  const int64_t v = level_start(M, t, j);
-  starts[idx] = static_cast<uint32_t>(v > 0 ? v : 0);
-}
-
-// Per level t < t0 and tile b of kLevelTile points: the segment holding the
-// tile's first point, i.e. the last j with starts[j] <= b * kLevelTile.
-__global__ void k_tile_segments(const uint32_t* __restrict__ starts, uint32_t n, uint32_t t0, uint32_t stride,
-                                uint32_t* __restrict__ tileseg) {
-  const uint64_t g = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (g >= static_cast<uint64_t>(t0) * stride) return;
-  const uint32_t t = static_cast<uint32_t>(g / stride), b = static_cast<uint32_t>(g % stride);
-  const uint32_t n_level = n - ((1u << t) - 1u);
-  const uint32_t tiles = (n_level + kLevelTile - 1) / kLevelTile;
-  uint32_t seg = 0;
-  if (b < tiles) {
-    const uint32_t* lv = starts + (1u << t) - 1u;
-    const uint32_t pos = b * kLevelTile;
-    uint32_t lo = 0, hi = 1u << t;  // lv[lo] <= pos (lv[0] = 0); answer in [lo, hi)
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (lv[mid] <= pos) lo = mid;
-      else hi = mid;
-    }
-    seg = lo;
-  }
-  tileseg[g] = seg;
-}
-
-__global__ void k_fill_u64(unsigned long long* p, size_t count, unsigned long long v) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < count) p[i] = v;
-}
-
 // ---------------------------------------------------------------------------
-// Level passes over A (all segments of level t are non-empty here).
+// The levels above LDS size. V: uint32_t ranks or uint64_t values, all
+// different; the smallest of a segment is its node. A segment of level t is
+// the input range [b_j, b_(j+1)) of the key1-ordered array less the nodes of
+// the levels above that lie in it (its holes, a sorted list of at most t
+// positions; one per segment on average, since a node lies in one segment).
 // ---------------------------------------------------------------------------
+constexpr uint32_t kFan = 64;        // values per block minimum, and per step of the hierarchy
+constexpr uint32_t kMaxHoles = 24;   // list entries per segment (levels above LDS size: at most 19)
+constexpr int kTopBlock = 256;
 
-// Segments met by one tile of kLevelTile points: every segment of a level
-// walked by these passes holds at least kFinishTile points.
-constexpr uint32_t kSegSlots = kLevelTile / kFinishTile + 2;
-
-// The tile's elements, each thread's kLevelElems loaded before any is used
-// (position tile + threadIdx.x + e * kLevelBlock).
-__device__ inline void load_tile(const uint32_t* __restrict__ A, uint32_t n_level, uint32_t tile,
-                                 uint32_t (&av)[kLevelElems]) {
-  const uint32_t* p = A + tile + threadIdx.x;
-  if (tile + kLevelTile <= n_level) {
+// mins1[k]: minimum of values [64 k, 64 k + 64); mins2 of 64 such, one
+// workgroup per 4096 values.
+template <typename V>
+__global__ __launch_bounds__(kTopBlock) void k_block_min(const V* __restrict__ a, uint32_t n, V* __restrict__ mins1,
+                                                         V* __restrict__ mins2) {
+  constexpr int kPer = 16 / sizeof(V);            // values per 16-byte load
+  constexpr int kLanes = kFan / kPer;             // lanes per block of 64
+  constexpr int kRounds = 4096 / (kTopBlock * kPer);
+  __shared__ V m1[kFan];
+  const uint64_t base = static_cast<uint64_t>(blockIdx.x) * 4096;
+  V x[kRounds][kPer];
+  if (base + 4096 <= n) {
 #pragma unroll
-    for (int e = 0; e < kLevelElems; e++) av[e] = p[e * kLevelBlock];
+    for (int r = 0; r < kRounds; r++) {
+      const uint4 w = *reinterpret_cast<const uint4*>(a + base + (r * kTopBlock + threadIdx.x) * kPer);
+      __builtin_memcpy(x[r], &w, 16);
+    }
   } else {
 #pragma unroll
-    for (int e = 0; e < kLevelElems; e++)
-      if (tile + threadIdx.x + e * kLevelBlock < n_level) av[e] = p[e * kLevelBlock];
-  }
-}
-
-// The starts of the tile's segments seg0 + k, k <= kSegSlots (n_level past
-// the level's last segment), into LDS. Call before a barrier.
-__device__ inline void load_seg_starts(const uint32_t* __restrict__ starts, uint32_t seg0, uint32_t nseg,
-                                       uint32_t n_level, uint32_t* sst) {
-  if (threadIdx.x <= kSegSlots) {
-    const uint32_t j = seg0 + threadIdx.x;
-    sst[threadIdx.x] = j < nseg ? starts[j] : n_level;
-  }
-}
-
-// Per tile and segment met: min over (rank << 32 | local position), i.e.
-// the max-key2 point and where it sits in the segment, into tmin (per tile
-// kSegSlots entries, combined per segment by k_tile_min_reduce).
-__global__ __launch_bounds__(kLevelBlock) void k_level_argmin(
-    const uint32_t* __restrict__ A, uint32_t n_level, uint32_t nseg,
-    const uint32_t* __restrict__ starts, const uint32_t* __restrict__ tileseg,
-    unsigned long long* __restrict__ tmin) {
-  __shared__ unsigned long long smin[kSegSlots];
-  __shared__ uint32_t sst[kSegSlots + 1];
-  const uint32_t tile = blockIdx.x * kLevelTile;
-  const uint32_t seg0 = tileseg[blockIdx.x];  // the segment holding the tile's first point
-  uint32_t av[kLevelElems];
-  load_tile(A, n_level, tile, av);
-  if (threadIdx.x < kSegSlots) smin[threadIdx.x] = ~0ull;
-  load_seg_starts(starts, seg0, nseg, n_level, sst);
-  __syncthreads();
-  const uint32_t first = tile + threadIdx.x;
-  uint32_t k = 0;
-  uint32_t st = sst[0], next = sst[1];
-  unsigned long long best = ~0ull;
+    for (int r = 0; r < kRounds; r++)
 #pragma unroll
-  for (int e = 0; e < kLevelElems; e++) {
-    const uint32_t P = first + e * kLevelBlock;
-    if (P < n_level) {
-      while (P >= next) {
-        if (best != ~0ull) atomicMin(&smin[k], best);
-        best = ~0ull;
-        k++;
-        st = next;
-        next = sst[k + 1];
+      for (int k = 0; k < kPer; k++) {
+        const uint64_t i = base + (r * kTopBlock + threadIdx.x) * kPer + k;
+        x[r][k] = i < n ? a[i] : static_cast<V>(~V(0));
       }
-      const unsigned long long key = (static_cast<unsigned long long>(av[e]) << 32) | (P - st);
-      best = key < best ? key : best;
-    }
-  }
-  if (best != ~0ull) atomicMin(&smin[k], best);
-  __syncthreads();
-  if (threadIdx.x < kSegSlots) tmin[static_cast<size_t>(blockIdx.x) * kSegSlots + threadIdx.x] = smin[threadIdx.x];
-}
-
-// out[i] for i < gridDim.x (one workgroup each): the minimum of slot
-// i - (tileseg[b] << sh) of the per-tile minima of every tile b that meets
-// segment i >> sh of the level (slots: entries per tile). For the levels
-// with few segments, where the tiles' global atomics would queue on a few
-// addresses.
-__global__ __launch_bounds__(kLevelBlock) void k_tile_min_reduce(
-    const unsigned long long* __restrict__ tmin, uint32_t slots, const uint32_t* __restrict__ tileseg,
-    const uint32_t* __restrict__ starts, uint32_t nseg, uint32_t n_level, uint32_t sh,
-    unsigned long long* __restrict__ out) {
-  __shared__ unsigned long long wbest[kLevelBlock / kWave];
-  const uint32_t i = blockIdx.x;
-  const uint32_t j = i >> sh;
-  const uint32_t lo = starts[j];
-  const uint32_t hi = j + 1 < nseg ? starts[j + 1] : n_level;
-  unsigned long long best = ~0ull;
-  if (hi > lo) {
-    const uint32_t b0 = lo / kLevelTile, b1 = (hi - 1) / kLevelTile;
-    for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kLevelBlock) {
-      const uint32_t slot = i - (tileseg[b] << sh);
-      if (slot < slots) {
-        const unsigned long long v = tmin[static_cast<size_t>(b) * slots + slot];
-        best = v < best ? v : best;
-      }
-    }
   }
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(best, off, kWave);
-    best = o < best ? o : best;
+  for (int r = 0; r < kRounds; r++) {
+    V m = x[r][0];
+#pragma unroll
+    for (int k = 1; k < kPer; k++) m = x[r][k] < m ? x[r][k] : m;
+#pragma unroll
+    for (int o = 1; o < kLanes; o <<= 1) {
+      const V y = __shfl_xor(m, o, kWave);
+      m = y < m ? y : m;
+    }
+    const uint32_t k = (r * kTopBlock + threadIdx.x) / kLanes;
+    if (threadIdx.x % kLanes == 0) {
+      m1[k] = m;
+      if (base + k * kFan < n) mins1[base / kFan + k] = m;
+    }
   }
-  if (lane_id() == 0) wbest[threadIdx.x / kWave] = best;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long m = wbest[0];
-    for (int w = 1; w < kLevelBlock / kWave; w++) m = wbest[w] < m ? wbest[w] : m;
-    out[i] = m;
+  if (threadIdx.x < kFan) {
+    V m = m1[threadIdx.x];
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const V y = __shfl_xor(m, o, kWave);
+      m = y < m ? y : m;
+    }
+    if (threadIdx.x == 0) mins2[blockIdx.x] = m;
   }
 }
+
+// mins3: minima of 64 values of mins2 (a wave each).
+template <typename V>
+__global__ __launch_bounds__(kTopBlock) void k_min_of_mins(const V* __restrict__ mins2, uint32_t n2,
+                                                           V* __restrict__ mins3, uint32_t n3) {
+  const uint32_t k = blockIdx.x * (kTopBlock / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  if (k >= n3) return;
+  const uint32_t i = k * kFan + lane;
+  V m = i < n2 ? mins2[i] : static_cast<V>(~V(0));
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const V y = __shfl_xor(m, o, kWave);
+    m = y < m ? y : m;
+  }
+  if (lane == 0) mins3[k] = m;
+}
+
+// Segments of one level: first positions, hole counts, hole lists.
+struct Segs {
+  uint32_t* b;
+  uint32_t* cnt;
+  uint32_t* holes;  // kMaxHoles per segment
+};
+
+__global__ void k_segs_root(Segs s) {
+  s.b[0] = 0;
+  s.cnt[0] = 0;
+}
+
+// A value of the dim's type from its key (not for -0, which shares +0's key).
+template <typename T>
+__device__ inline T from_key(uint32_t k) {
+  if constexpr (std::is_same<T, float>::value) return __builtin_bit_cast(float, (k & 0x80000000u) ? k ^ 0x80000000u : ~k);
+  else if constexpr (std::is_same<T, int32_t>::value) return static_cast<int32_t>(k ^ 0x80000000u);
+  else return static_cast<T>(k);
+}
+
+// Where the records' fields come from. Ranked: V = uint32_t ranks into the
+// key2 order, records gathered from the points. Direct: V = uint64_t values
+// and the sorted dim1 keys; id_code says how IDs map to keys.
+template <typename T, typename IS>
+struct Ranked {
+  using V = uint32_t;
+  const uint32_t* perm2;
+  const Point<T, IS>* pts;
+  __device__ Point<T, IS> point(V v, uint32_t) const { return pts[perm2[v]]; }
+};
+template <typename T, typename IS>
+struct Direct {
+  using V = uint64_t;
+  const uint32_t* key1;
+  int id_code;
+  __device__ Point<T, IS> make(V v, uint32_t k1) const {
+    Point<T, IS> p;
+    p.dim1_val = from_key<T>(k1);
+    p.dim2_val = from_key<T>(~static_cast<uint32_t>(v >> 32));
+    if constexpr (has_id_v<IS>) {
+      const uint32_t k = ~static_cast<uint32_t>(v);
+      p.id = id_code == F32 ? __builtin_bit_cast(uint32_t, from_key<float>(k))
+                            : (id_code == I32 ? static_cast<uint32_t>(from_key<int32_t>(k)) : k);
+    }
+    return p;
+  }
+  __device__ Point<T, IS> point(V v, uint32_t pos) const { return make(v, key1[pos]); }
+};
 
 template <typename T, typename IS>
 __device__ inline void write_node(Node<T, IS>* nodes, uint64_t slot, const Point<T, IS>& p, T med) {
@@ -293,94 +270,138 @@ __device__ inline void write_node(Node<T, IS>* nodes, uint64_t slot, const Point
   nodes[slot] = r;
 }
 
-// Emits the level's nodes and compacts A into the next level: the point at
-// local position x of segment j (x != q_j) moves to start_j - j + x', with
-// x' = x - [x > q_j]. Unless level t + 1 is built in LDS, the same pass
-// finds the next level's minima: x' < floor(m_j / 2) lands in child 2j at
-// position x', the rest in child 2j + 1 at x' - floor(m_j / 2), and the
-// minimum of (rank << 32 | child position) per child goes to nextmin.
-// The tile's elements are loaded first and its segments' starts, minima and
-// halves staged in LDS, so that the pass streams A at full occupancy.
-template <typename T, typename IS>
-__global__ __launch_bounds__(kLevelBlock) void k_level_emit(
-    const uint32_t* __restrict__ A, uint32_t* __restrict__ Anext, uint32_t n_level, uint32_t t,
-    uint64_t M, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ tileseg,
-    const unsigned long long* __restrict__ segmin, unsigned long long* __restrict__ nextmin,
-    unsigned long long* __restrict__ tmin, const uint32_t* __restrict__ perm2, const Point<T, IS>* __restrict__ pts,
-    Node<T, IS>* __restrict__ nodes) {
-  constexpr uint32_t kChildSlots = 2 * kSegSlots;  // children per tile
+// One level: a wave per segment finds the node, writes its record and hands
+// the two halves of what remains to the next level. The minimum is taken
+// over the stretches between the segment's holes; a stretch reads at most 126
+// values at each end of each step of the hierarchy (and the middle of the
+// top one), all at once, and the winner is traced down a step at a time.
+// Bound by latency (about eight dependent loads). On MI355X the 15 levels of
+// 2^26 points take 0.17 ms after 0.12 ms for the block minima, where moving
+// the points level by level (8 B per point and level) took 1.78 ms.
+template <typename T, typename IS, typename Src>
+__global__ __launch_bounds__(kTopBlock) void k_top_level(Src src, const typename Src::V* __restrict__ a,
+                                                         const typename Src::V* __restrict__ m1,
+                                                         const typename Src::V* __restrict__ m2,
+                                                         const typename Src::V* __restrict__ m3, uint32_t n, uint32_t t,
+                                                         uint64_t M, Segs in, Segs out, Node<T, IS>* __restrict__ nodes) {
+  using V = typename Src::V;
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t j = __builtin_amdgcn_readfirstlane(blockIdx.x * (kTopBlock / kWave) + threadIdx.x / kWave);
   const uint32_t nseg = 1u << t;
-  __shared__ unsigned long long cmin[kChildSlots];
-  __shared__ unsigned long long smn[kSegSlots];
-  __shared__ uint32_t sst[kSegSlots + 1];
-  __shared__ uint32_t shalf[kSegSlots];
-  const uint32_t tile = blockIdx.x * kLevelTile;
-  const uint32_t seg0 = tileseg[blockIdx.x];  // the segment holding the tile's first point
-  uint32_t av[kLevelElems];
-  load_tile(A, n_level, tile, av);
-  if (threadIdx.x < kChildSlots) cmin[threadIdx.x] = ~0ull;
-  load_seg_starts(starts, seg0, nseg, n_level, sst);
-  if (threadIdx.x < kSegSlots) {
-    const uint32_t j = seg0 + threadIdx.x;
-    smn[threadIdx.x] = j < nseg ? segmin[j] : ~0ull;
-    shalf[threadIdx.x] = j < nseg ? static_cast<uint32_t>(level_size(M, t, j)) >> 1 : 0u;
-  }
-  __syncthreads();
-  const uint32_t c0 = 2 * seg0;  // the tile's first child segment
-  const uint32_t first = tile + threadIdx.x;
-  uint32_t k = 0;
-  uint32_t st = sst[0], next = sst[1];
-  uint32_t q = static_cast<uint32_t>(smn[0]);
-  uint32_t half = shalf[0];
-  unsigned long long best = ~0ull;  // running minimum of child bc
-  uint32_t bc = 0;
-#pragma unroll
-  for (int e = 0; e < kLevelElems; e++) {
-    const uint32_t P = first + e * kLevelBlock;
-    if (P < n_level) {
-      while (P >= next) {
-        k++;
-        st = next;
-        next = sst[k + 1];
-        q = static_cast<uint32_t>(smn[k]);
-        half = shalf[k];
-      }
-      const uint32_t x = P - st;
-      const uint32_t a = av[e];
-      const uint32_t j = seg0 + k;
-      if (x == q) {
-        const uint32_t L = half;
-        const Point<T, IS> p = pts[perm2[a]];
-        T med = p.dim1_val;
-        if (L >= 1) {
-          const uint32_t pm = q < L ? L : L - 1;
-          med = pts[perm2[A[st + pm]]].dim1_val;
-        }
-        write_node(nodes, (1ull << t) - 1 + j, p, med);
-      } else {
-        const uint32_t xr = x - (x > q ? 1u : 0u);
-        Anext[st - j + xr] = a;
-        if (nextmin) {
-          const bool right = xr >= half;
-          const uint32_t c = 2 * k + (right ? 1u : 0u);
-          const unsigned long long key = (static_cast<unsigned long long>(a) << 32) | (right ? xr - half : xr);
-          if (c != bc) {
-            if (best != ~0ull) atomicMin(&cmin[bc], best);
-            best = ~0ull;
-            bc = c;
-          }
-          best = key < best ? key : best;
-        }
+  if (j >= nseg) return;
+  const uint32_t b = in.b[j], e = j + 1 < nseg ? in.b[j + 1] : n;
+  const uint32_t cnt = in.cnt[j];
+  uint32_t hole = lane < cnt ? in.holes[static_cast<size_t>(j) * kMaxHoles + lane] : ~0u;
+  const uint32_t n1 = (n + kFan - 1) / kFan, n2 = (n1 + kFan - 1) / kFan;
+  // the lane's best candidate: its value, step of the hierarchy and index
+  V best = static_cast<V>(~V(0));
+  uint32_t step = 0, at = ~0u;
+  auto take = [&](const V* arr, uint32_t i, uint32_t end, uint32_t st) {
+    if (i < end) {
+      const V v = arr[i];
+      if (v < best || at == ~0u) {
+        best = v;
+        step = st;
+        at = i;
       }
     }
+  };
+  for (uint32_t r = 0; r <= cnt; r++) {
+    const uint32_t lo = r == 0 ? b : __builtin_amdgcn_readlane(hole, r - 1) + 1;
+    const uint32_t hi = r == cnt ? e : static_cast<uint32_t>(__builtin_amdgcn_readlane(hole, r));
+    if (lo >= hi) continue;
+    const uint32_t lo1 = (lo + kFan - 1) / kFan, hi1 = hi / kFan;
+    if (lo1 >= hi1) {  // no whole block of 64 inside
+      take(a, lo + lane, hi, 0);
+      take(a, lo + kWave + lane, hi, 0);
+      continue;
+    }
+    take(a, lo + lane, lo1 * kFan, 0);
+    take(a, hi1 * kFan + lane, hi, 0);
+    const uint32_t lo2 = (lo1 + kFan - 1) / kFan, hi2 = hi1 / kFan;
+    if (lo2 >= hi2) {
+      take(m1, lo1 + lane, hi1, 1);
+      take(m1, lo1 + kWave + lane, hi1, 1);
+      continue;
+    }
+    take(m1, lo1 + lane, lo2 * kFan, 1);
+    take(m1, hi2 * kFan + lane, hi1, 1);
+    const uint32_t lo3 = (lo2 + kFan - 1) / kFan, hi3 = hi2 / kFan;
+    if (lo3 >= hi3) {
+      take(m2, lo2 + lane, hi2, 2);
+      take(m2, lo2 + kWave + lane, hi2, 2);
+      continue;
+    }
+    take(m2, lo2 + lane, lo3 * kFan, 2);
+    take(m2, hi3 * kFan + lane, hi2, 2);
+    for (uint32_t i = lo3; i < hi3; i += kWave) take(m3, i + lane, hi3, 3);
   }
-  if (!nextmin) return;
-  if (best != ~0ull) atomicMin(&cmin[bc], best);
-  __syncthreads();
-  if (tmin) {  // per-tile minima, reduced by k_tile_min_reduce
-    if (threadIdx.x < kChildSlots) tmin[static_cast<size_t>(blockIdx.x) * kChildSlots + threadIdx.x] = cmin[threadIdx.x];
-  } else if (threadIdx.x < kChildSlots && cmin[threadIdx.x] != ~0ull) {
-    atomicMin(&nextmin[c0 + threadIdx.x], cmin[threadIdx.x]);
+  V mn = best;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const V y = __shfl_xor(mn, o, kWave);
+    mn = y < mn ? y : mn;
+  }
+  const uint64_t won = __ballot(best == mn && at != ~0u);
+  if (won == 0) return;  // never: the segment holds points
+  const int f = __builtin_ctzll(won);
+  uint32_t q = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(at), f));
+  int st = __builtin_amdgcn_readlane(static_cast<int>(step), f);
+  for (; st > 0; st--) {
+    const V* arr = st == 3 ? m2 : (st == 2 ? m1 : a);
+    const uint32_t len = st == 3 ? n2 : (st == 2 ? n1 : n);
+    const uint32_t i = q * kFan + lane;
+    const uint64_t eq = __ballot(i < len && arr[i < len ? i : 0] == mn);
+    q = q * kFan + static_cast<uint32_t>(eq ? __builtin_ctzll(eq) : 0);
+  }
+  // the node joins the holes (in position order)
+  const uint32_t below = static_cast<uint32_t>(__popcll(__ballot(lane < cnt && hole < q)));
+  const uint32_t prev = static_cast<uint32_t>(__shfl_up(static_cast<int>(hole), 1, kWave));
+  hole = lane < below ? hole : (lane == below ? q : prev);
+  const uint32_t nh = cnt + 1;
+  // position of the last point of the left half: the (L - 1)-th that remains
+  const uint32_t L = static_cast<uint32_t>(level_size(M, t, j)) >> 1;
+  uint32_t last = b + L - 1;
+  for (uint32_t i = 0; i < nh; i++) {
+    const uint32_t h = static_cast<uint32_t>(__builtin_amdgcn_readlane(hole, i));
+    last += h <= last ? 1u : 0u;
+  }
+  const uint32_t c = last + 1;
+  const uint32_t nl = static_cast<uint32_t>(__popcll(__ballot(lane < nh && hole < c)));
+  if (lane < nh) {
+    if (lane < nl) out.holes[static_cast<size_t>(2 * j) * kMaxHoles + lane] = hole;
+    else out.holes[static_cast<size_t>(2 * j + 1) * kMaxHoles + lane - nl] = hole;
+  }
+  if (lane == 0) {
+    out.b[2 * j] = b;
+    out.b[2 * j + 1] = c;
+    out.cnt[2 * j] = nl;
+    out.cnt[2 * j + 1] = nh - nl;
+    write_node(nodes, nseg - 1ull + j, src.point(mn, q), src.point(a[last], last).dim1_val);
+  }
+}
+
+// Subtree minima of dim2 and IDs of the levels above LDS size: levels
+// [s, t0) by one workgroup per subtree of level s, then levels [0, s) by one
+// workgroup (what k_submin_level computes, in two launches).
+template <typename T, typename IS>
+__global__ __launch_bounds__(kTopBlock) void k_top_submin(const Node<T, IS>* __restrict__ nodes, T* submin,
+                                                          IS* __restrict__ ids, uint32_t s, uint32_t t0) {
+  for (uint32_t u = t0; u-- > s;) {
+    const uint32_t per = 1u << (u - s);
+    for (uint32_t k = threadIdx.x; k < per; k += kTopBlock) {
+      const uint32_t slot = (1u << u) - 1 + blockIdx.x * per + k;
+      const Node<T, IS> nd = nodes[slot];
+      if constexpr (has_id_v<IS>) {
+        if (ids) ids[slot] = nd.id;
+      }
+      T v = nd.dim2;
+      const T l = submin[2 * slot + 1], r = submin[2 * slot + 2];  // every such node has both children
+      v = l < v ? l : v;
+      v = r < v ? r : v;
+      submin[slot] = v;
+    }
+    __syncthreads();
   }
 }
 
@@ -484,6 +505,7 @@ __device__ inline void wave_sync() {
 // k >> (u - kWaveLevel), so those levels need no workgroup barrier.
 constexpr uint32_t kFinishLog = 9;
 static_assert((1u << kFinishLog) == kFinishBlock, "block size is a power of two");
+constexpr uint16_t kNoPos = 0xffffu;
 constexpr uint32_t kWaveLevel = kFinishLog - 6;
 static_assert(kWave == 64, "64-lane waves");
 
@@ -496,10 +518,9 @@ static_assert(kWave == 64, "64-lane waves");
 // flight together, so that no level waits on global memory. The levels
 // above kWaveLevel share segments between waves and end in a workgroup
 // barrier; from it on each wave works on its own part of the subtree.
-template <typename T, typename IS>
-__device__ void lds_build_local(uint16_t* bufA, uint16_t* bufB, const uint32_t* rank, uint16_t* slot_of,
-                                uint16_t* med_of, uint16_t* sst, unsigned long long* sres, unsigned long long* wred,
-                                uint32_t m) {
+template <typename V>
+__device__ void lds_build_local(uint16_t* bufA, uint16_t* bufB, const V* rank, uint16_t* slot_of, uint16_t* med_of,
+                                uint16_t* sst, uint16_t* sres, V* wred, uint16_t* wredx, uint32_t m) {
   const uint32_t tid = threadIdx.x;
   constexpr uint32_t nthr = kFinishBlock;  // the launch's block size
   const uint64_t Mp = static_cast<uint64_t>(m) + 1;
@@ -535,31 +556,52 @@ __device__ void lds_build_local(uint16_t* bufA, uint16_t* bufB, const uint32_t* 
       const uint32_t k = tid / G, g = tid % G;
       const int64_t sz = level_size(Mp, u, k);
       const uint32_t st = sz > 0 ? sst[(1u << u) - 1 + k] : 0u;
-      unsigned long long best = ~0ull;
+      // the smallest value, then its position from the one thread that holds it
+      V mine = static_cast<V>(~V(0));
+      uint32_t bx = ~0u;
       for (int64_t x = g; x < sz; x += G) {
-        const unsigned long long key =
-            (static_cast<unsigned long long>(rank[bufA[st + x]]) << 32) | static_cast<unsigned long long>(x);
-        best = key < best ? key : best;
+        const V v = rank[bufA[st + x]];
+        if (v <= mine) {
+          mine = v;
+          bx = static_cast<uint32_t>(x);
+        }
       }
+      V best = mine;
       const uint32_t wg = G < kWave ? G : kWave;
       for (uint32_t off = wg >> 1; off >= 1; off >>= 1) {
-        const unsigned long long o = __shfl_xor(best, off, kWave);
+        const V o = __shfl_xor(best, off, kWave);
         best = o < best ? o : best;
-      }
-      if (G > kWave) {  // uniform across the block
-        if ((tid & (kWave - 1)) == 0) wred[tid / kWave] = best;
-        __syncthreads();
-        if (g == 0) {
-          const uint32_t w0 = tid / kWave, nw = G / kWave;
-          for (uint32_t w = 0; w < nw; w++) best = wred[w0 + w] < best ? wred[w0 + w] : best;
-        }
       }
       // the segment's result sits at its first thread's entry, which no
       // other wave uses at any level
-      if (g == 0) sres[k * G] = best;
+      if (G > kWave) {  // uniform across the block
+        if (bx != ~0u && mine == best) {
+          wred[tid / kWave] = best;
+          wredx[tid / kWave] = static_cast<uint16_t>(bx);
+        }
+        if (__ballot(bx != ~0u) == 0 && (tid & (kWave - 1)) == 0) {  // a wave without points
+          wred[tid / kWave] = static_cast<V>(~V(0));
+          wredx[tid / kWave] = kNoPos;
+        }
+        __syncthreads();
+        if (g == 0) {
+          const uint32_t w0 = tid / kWave, nw = G / kWave;
+          V b2 = wred[w0];
+          uint16_t x2 = wredx[w0];
+          for (uint32_t w = 1; w < nw; w++) {
+            if (wredx[w0 + w] != kNoPos && (x2 == kNoPos || wred[w0 + w] < b2)) {
+              b2 = wred[w0 + w];
+              x2 = wredx[w0 + w];
+            }
+          }
+          sres[k * G] = x2;
+        }
+      } else if (bx != ~0u && mine == best) {
+        sres[k * G] = static_cast<uint16_t>(bx);
+      }
       level_sync(u);
       if (sz > 0) {
-        const uint32_t q = static_cast<uint32_t>(sres[k * G]);
+        const uint32_t q = sres[k * G];
         if (g == 0) note(u, k, st, static_cast<uint32_t>(sz), q);
         const uint32_t dst0 = st;
         for (int64_t x = g; x < sz; x += G) {
@@ -575,13 +617,15 @@ __device__ void lds_build_local(uint16_t* bufA, uint16_t* bufB, const uint32_t* 
         const int64_t sz = level_size(Mp, u, k);
         if (sz <= 0) continue;
         const uint32_t st = sst[(1u << u) - 1 + k];
-        unsigned long long best = ~0ull;
-        for (int64_t x = 0; x < sz; x++) {
-          const unsigned long long key =
-              (static_cast<unsigned long long>(rank[bufA[st + x]]) << 32) | static_cast<unsigned long long>(x);
-          best = key < best ? key : best;
+        V best = rank[bufA[st]];
+        uint32_t q = 0;
+        for (int64_t x = 1; x < sz; x++) {
+          const V v = rank[bufA[st + x]];
+          if (v < best) {
+            best = v;
+            q = static_cast<uint32_t>(x);
+          }
         }
-        const uint32_t q = static_cast<uint32_t>(best);
         note(u, k, st, static_cast<uint32_t>(sz), q);
         if (sz > 1) {
           const uint32_t dst0 = st;
@@ -600,14 +644,18 @@ __device__ void lds_build_local(uint16_t* bufA, uint16_t* bufB, const uint32_t* 
   __syncthreads();
 }
 
+// Direct: 1.36 ms for 2^26 f32/u32 points on MI355X, bound by the LDS passes
+// of the subtree build (12 B read and 24 B written per point are 0.5 ms at a
+// large copy's rate). Ranked, with two 128-byte gathers per point: 2.75 ms.
 // One workgroup per level-t0 segment: its whole subtree in LDS, then every
 // node record; with `submin` also the subtree minima of dim2 and the IDs of
 // the subtree's slots (the bottom levels of what k_submin_level computes).
-template <typename T, typename IS>
+template <typename T, typename IS, typename Src>
 __global__ __launch_bounds__(kFinishBlock) void k_finish(
-    const uint32_t* __restrict__ A, uint32_t t0, uint64_t M, const uint32_t* __restrict__ starts,
-    const uint32_t* __restrict__ perm2, const Point<T, IS>* __restrict__ pts, Node<T, IS>* __restrict__ nodes,
-    T* __restrict__ submin, IS* __restrict__ ids) {
+    Src src, const typename Src::V* __restrict__ A, uint32_t n, uint32_t t0, uint64_t M, Segs segs,
+    Node<T, IS>* __restrict__ nodes, T* __restrict__ submin, IS* __restrict__ ids) {
+  using V = typename Src::V;
+  constexpr bool kDirect = sizeof(V) == 8;  // records from values and dim1 keys, else gathered
   union FinishLds {
     struct {
       uint16_t bufA[kFinishTile];
@@ -618,60 +666,100 @@ __global__ __launch_bounds__(kFinishBlock) void k_finish(
   };
   __shared__ FinishLds U;
   union RankLds {
-    uint32_t rank[kFinishTile];
-    T d1[kFinishTile];  // after the lookups: dim1 of every point, for the meds
+    V rank[kFinishTile];
+    T d1[kFinishTile];  // gathered records, after the lookups: dim1 of every point, for the meds
   };
   __shared__ RankLds R;
-  uint32_t* rank = R.rank;
+  __shared__ uint32_t s_key1[kDirect ? kFinishTile : 1];
+  V* rank = R.rank;
   __shared__ uint16_t slot_of[kFinishTile];  // the subtree slot (heap order) each point fills
   __shared__ uint16_t med_of[kFinishTile];   // and the point whose dim1 is its med
-  __shared__ unsigned long long sres[kFinishBlock];  // a segment's result, at its first thread's entry
-  __shared__ unsigned long long wred[kFinishBlock / kWave];
+  __shared__ uint16_t sres[kFinishBlock];    // a segment's result, at its first thread's entry
+  __shared__ V wred[kFinishBlock / kWave];
+  __shared__ uint16_t wredx[kFinishBlock / kWave];
+  __shared__ uint32_t s_hole[kMaxHoles];
   const uint32_t j = blockIdx.x;
   const int64_t m = level_size(M, t0, j);
   if (m <= 0) return;
-  const uint32_t st = starts[j];
+  const uint32_t st = segs.b[j], len = (j + 1 < gridDim.x ? segs.b[j + 1] : n) - st;
+  const uint32_t nh = segs.cnt[j];
+  if (threadIdx.x < nh) s_hole[threadIdx.x] = segs.holes[static_cast<size_t>(j) * kMaxHoles + threadIdx.x] - st;
   const uint64_t root = (1ull << t0) - 1 + j;
   constexpr int kPer = kFinishTile / kFinishBlock;
+  // the segment's values close up over its holes: point x is the x-th that
+  // is left (a range of at most kFinishTile + kMaxHoles positions)
+  V av[kPer + 1];
+  uint32_t kv[kPer + 1];
 #pragma unroll
-  for (int e = 0; e < kPer; e++) {
-    const uint32_t x = threadIdx.x + e * kFinishBlock;
-    if (x < m) {
-      rank[x] = A[st + x];
-      U.b.bufA[x] = static_cast<uint16_t>(x);
+  for (int e = 0; e < kPer + 1; e++) {
+    const uint32_t p = threadIdx.x + e * kFinishBlock;
+    if (p < len) {
+      av[e] = A[st + p];
+      if constexpr (kDirect) kv[e] = src.key1[st + p];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < kPer + 1; e++) {
+    const uint32_t p = threadIdx.x + e * kFinishBlock;
+    if (p < len) {
+      uint32_t x = p;
+      bool gone = false;
+      for (uint32_t i = 0; i < nh; i++) {
+        const uint32_t h = s_hole[i];
+        x -= h < p ? 1u : 0u;
+        gone |= h == p;
+      }
+      if (!gone && x < m) {
+        rank[x] = av[e];
+        if constexpr (kDirect) s_key1[x] = kv[e];
+        U.b.bufA[x] = static_cast<uint16_t>(x);
+      }
     }
   }
   if (threadIdx.x == 0) U.b.sst[0] = 0;
   __syncthreads();
-  lds_build_local<T, IS>(U.b.bufA, U.b.bufB, rank, slot_of, med_of, U.b.sst, sres, wred, static_cast<uint32_t>(m));
-  // every point's node record (rank -> input index -> record; all loads in
-  // flight together): subtree slot h (level u, position k) is slot
+  lds_build_local<V>(U.b.bufA, U.b.bufB, rank, slot_of, med_of, U.b.sst, sres, wred, wredx, static_cast<uint32_t>(m));
+  // every point's node record: subtree slot h (level u, position k) is slot
   // ((root + 1) << u) - 1 + k of the tree. A med is the dim1 of a point of
-  // the same subtree, exchanged through LDS.
-  uint32_t ix[kPer];
-#pragma unroll
-  for (int e = 0; e < kPer; e++) {
-    const uint32_t x = threadIdx.x + e * kFinishBlock;
-    if (x < m) ix[e] = perm2[rank[x]];
-  }
+  // the same subtree. Gathered records: rank -> input index -> record, all
+  // loads in flight together.
   Point<T, IS> p[kPer];
-#pragma unroll
-  for (int e = 0; e < kPer; e++) {
-    const uint32_t x = threadIdx.x + e * kFinishBlock;
-    if (x < m) p[e] = pts[ix[e]];
-  }
-  __syncthreads();  // the build's LDS arrays and the ranks are free from here
-#pragma unroll
-  for (int e = 0; e < kPer; e++) {
-    const uint32_t x = threadIdx.x + e * kFinishBlock;
-    if (x < m) R.d1[x] = p[e].dim1_val;
-  }
-  __syncthreads();
   T med[kPer];
+  if constexpr (kDirect) {
 #pragma unroll
-  for (int e = 0; e < kPer; e++) {
-    const uint32_t x = threadIdx.x + e * kFinishBlock;
-    if (x < m) med[e] = R.d1[med_of[x]];
+    for (int e = 0; e < kPer; e++) {
+      const uint32_t x = threadIdx.x + e * kFinishBlock;
+      if (x < m) {
+        p[e] = src.make(rank[x], s_key1[x]);
+        med[e] = from_key<T>(s_key1[med_of[x]]);
+      }
+    }
+    __syncthreads();  // the build's LDS arrays are free from here
+  } else {
+    uint32_t ix[kPer];
+#pragma unroll
+    for (int e = 0; e < kPer; e++) {
+      const uint32_t x = threadIdx.x + e * kFinishBlock;
+      if (x < m) ix[e] = src.perm2[rank[x]];
+    }
+#pragma unroll
+    for (int e = 0; e < kPer; e++) {
+      const uint32_t x = threadIdx.x + e * kFinishBlock;
+      if (x < m) p[e] = src.pts[ix[e]];
+    }
+    __syncthreads();  // the build's LDS arrays and the ranks are free from here
+#pragma unroll
+    for (int e = 0; e < kPer; e++) {
+      const uint32_t x = threadIdx.x + e * kFinishBlock;
+      if (x < m) R.d1[x] = p[e].dim1_val;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kPer; e++) {
+      const uint32_t x = threadIdx.x + e * kFinishBlock;
+      if (x < m) med[e] = R.d1[med_of[x]];
+    }
   }
   const uint32_t mdepth = 32u - static_cast<uint32_t>(__builtin_clz(static_cast<uint32_t>(m)));
 #pragma unroll
@@ -991,13 +1079,14 @@ struct DevBuf {
 
 inline unsigned grid_for(size_t n, unsigned block) { return static_cast<unsigned>((n + block - 1) / block); }
 
-// Construction buffers of n points, carved from one allocation: two key
-// arrays, four 32-bit arrays (sort values, the key2 order, the level arrays
-// and the key2 ranks), flags, radix sort storage, level tables.
+// Construction buffers of n points, carved from two blocks. Block A: keys and
+// three 32-bit words per point; block B: keys, two words per point, sort
+// scratch, minima and segment tables. Values that carry (dim2, ID) take two
+// words per point in each block.
 struct BuildLayout {
-  size_t key0, key1, v0, v1, v2, r2, flags, tmp, starts, segmin, tileseg, tmin;
-  size_t total_a, total_b, total;  // part A, part B, both
-  size_t tile_stride;  // tileseg entries per level
+  size_t key0, v0, v2, flags;                       // in A
+  size_t key1, v1, r2, tmp, mins, segs;             // in B
+  size_t total_a, total_b, total;
   size_t tmp_bytes;
   uint32_t t0;
 };
@@ -1017,16 +1106,27 @@ inline uint32_t finish_level(uint64_t M) {
   return t0;
 }
 
+// Block minima of n values: steps 1, 2 and 3 of the hierarchy.
+inline size_t min_words(size_t n) {
+  const size_t n1 = (n + kFan - 1) / kFan, n2 = (n1 + kFan - 1) / kFan;
+  return n1 + n2 + (n2 + kFan - 1) / kFan;
+}
+// One level's segment table, for levels up to t0.
+inline size_t segs_bytes(uint32_t t0) { return (size_t{1} << t0) * (2 + kMaxHoles) * 4; }
+inline Segs segs_at(unsigned char* p, uint32_t t0) {
+  auto* w = reinterpret_cast<uint32_t*>(p);
+  return Segs{w, w + (size_t{1} << t0), w + 2 * (size_t{1} << t0)};
+}
+
 template <typename K>
 BuildLayout build_layout(size_t n) {
   BuildLayout L{};
   size_t tb = 0;
   if constexpr (sizeof(K) == 4) radix_sort_u32(nullptr, tb, nullptr, nullptr, nullptr, nullptr, n, nullptr);
   else radix_sort_u64(nullptr, tb, nullptr, nullptr, nullptr, nullptr, n, nullptr);
+  if (point_sort_tmp_bytes(n) > tb) tb = point_sort_tmp_bytes(n);
   L.tmp_bytes = tb;
   L.t0 = finish_level(static_cast<uint64_t>(n) + 1);
-  const size_t nstart = (1ull << (L.t0 + 1)) - 1;
-  const size_t nmin = L.t0 ? (1ull << L.t0) - 1 : 1;
   size_t o = 0;
   auto take = [&](size_t bytes) {
     const size_t at = o;
@@ -1045,11 +1145,8 @@ BuildLayout build_layout(size_t n) {
   L.v1 = take(n * 4);
   L.r2 = take(n * 4);
   L.tmp = take(tb);
-  L.starts = take(nstart * 4);
-  L.segmin = take(nmin * 8);
-  L.tile_stride = (n + kLevelTile - 1) / kLevelTile;
-  L.tileseg = take(static_cast<size_t>(L.t0) * L.tile_stride * 4);
-  L.tmin = take(L.tile_stride * 2 * kSegSlots * 8);
+  L.mins = take(min_words(n) * 8);
+  L.segs = take(2 * segs_bytes(L.t0));
   L.total_b = o;
   L.total = L.total_a + L.total_b;
   return L;
@@ -1060,8 +1157,46 @@ template <typename T, typename I>
 using BuildKey = typename std::conditional<(sizeof(T) == 8 || (has_id_v<I> && sizeof(I) == 8)), uint64_t,
                                            uint32_t>::type;
 
+// From the key1-ordered array on: the levels above LDS size, the LDS
+// subtrees, and the subtree minima and IDs of the levels above them.
+template <typename T, typename IS, typename Src>
+Status build_levels(Src src, const typename Src::V* A, uint32_t n, uint32_t t0, unsigned char* mins, unsigned char* segs,
+                    const BuildOut& out, hipStream_t s) {
+  using V = typename Src::V;
+  const uint64_t M = static_cast<uint64_t>(n) + 1;
+  auto* nodes = static_cast<Node<T, IS>*>(out.nodes);
+  Segs cur = segs_at(segs, t0), nxt = segs_at(segs + segs_bytes(t0), t0);
+  k_segs_root<<<1, 1, 0, s>>>(cur);
+  if (t0 > 0) {
+    const uint32_t n1 = (n + kFan - 1) / kFan, n2 = (n1 + kFan - 1) / kFan, n3 = (n2 + kFan - 1) / kFan;
+    V* m1 = reinterpret_cast<V*>(mins);
+    V* m2 = m1 + n1;
+    V* m3 = m2 + n2;
+    constexpr unsigned kWaves = kTopBlock / kWave;
+    k_block_min<V><<<n2, kTopBlock, 0, s>>>(A, n, m1, m2);
+    k_min_of_mins<V><<<grid_for(n3, kWaves), kTopBlock, 0, s>>>(m2, n2, m3, n3);
+    for (uint32_t t = 0; t < t0; t++) {
+      k_top_level<T, IS, Src><<<grid_for(size_t{1} << t, kWaves), kTopBlock, 0, s>>>(src, A, m1, m2, m3, n, t, M, cur, nxt,
+                                                                                    nodes);
+      std::swap(cur, nxt);
+    }
+  }
+  k_finish<T, IS, Src><<<1u << t0, kFinishBlock, 0, s>>>(src, A, n, t0, M, cur, nodes, static_cast<T*>(out.submin),
+                                                         static_cast<IS*>(out.ids));
+  if (out.submin && t0 > 0) {
+    const uint32_t split = t0 > 7 ? t0 - 7 : 0;
+    k_top_submin<T, IS><<<1u << split, kTopBlock, 0, s>>>(nodes, static_cast<T*>(out.submin), static_cast<IS*>(out.ids),
+                                                          split, t0);
+    if (split)
+      k_top_submin<T, IS><<<1, kTopBlock, 0, s>>>(nodes, static_cast<T*>(out.submin), static_cast<IS*>(out.ids), 0u,
+                                                  split);
+  }
+  return hip_status(hipGetLastError(), "Error in launching construction kernels");
+}
+
 template <typename T, typename I>
-Status build_typed(const void* pts_v, size_t n64, BuildOut& out, hipStream_t s, BuildTimes* times) {
+Status build_typed(int dtype, int id_dtype, const void* pts_v, size_t n64, BuildOut& out, hipStream_t s,
+                   BuildTimes* times) {
   using IS = typename IdStore<I>::type;
   using K = BuildKey<T, I>;
   Status st;
@@ -1072,12 +1207,10 @@ Status build_typed(const void* pts_v, size_t n64, BuildOut& out, hipStream_t s, 
     return st;
   }
   const uint32_t n = static_cast<uint32_t>(n64);
-  const uint64_t M = n64 + 1;
   const auto* pts = static_cast<const Point<T, I>*>(pts_v);
-  const auto* ptsS = static_cast<const Point<T, IS>*>(pts_v);
   constexpr bool kHasId = has_id_v<I>;
 
-  hipEvent_t ev[5] = {};
+  hipEvent_t ev[3] = {};
   if (times)
     for (auto& e : ev) hipEventCreate(&e);
   auto mark = [&](int k) {
@@ -1091,160 +1224,122 @@ Status build_typed(const void* pts_v, size_t n64, BuildOut& out, hipStream_t s, 
     if (e != hipSuccess) return hip_status(e, what); \
   } while (0)
   const BuildLayout BL = build_layout<K>(n64);
-  // scratch in two parts: what the first key kernel writes, then the rest,
-  // allocated while that kernel runs
   DevBuf arena_a, arena_b;
   PST_TRY(arena_a.alloc(BL.total_a), "Error in allocating construction arrays");
-  unsigned char* base_a = arena_a.as<unsigned char>();
-  K* key0 = reinterpret_cast<K*>(base_a + BL.key0);
-  uint32_t* v0 = reinterpret_cast<uint32_t*>(base_a + BL.v0);
-  uint32_t* v2 = reinterpret_cast<uint32_t*>(base_a + BL.v2);
-  int* flags = reinterpret_cast<int*>(base_a + BL.flags);
-  // flags[0]: NaN seen; flags[1]: IDs not in index order; flags[2]: a sort's wait ran out
-  PST_TRY(hipMemsetAsync(flags, 0, 3 * sizeof(int), s), "Error in clearing construction flags");
-  const unsigned B = 256;
-  const unsigned G = grid_for(n, B);
-  int* nan_flag = flags;
-  mark(0);
-  // ---- key2 descending -> perm2 (v1), r2. One sort by dim2 when the IDs
-  // are in index order (the sort's index tie-break is then the (id, index)
-  // tie-break), else a sort by ID and then a stable one by dim2.
-  // 32-bit keys: the dim1 keys are stored by the same kernel, into v2
-  constexpr bool kKey1First = sizeof(K) == 4;
-  k_keys_single<T, I, K, true, true, false, kHasId>
-      <<<G, B, 0, s>>>(pts, n, key0, v0, nullptr, flags, kKey1First ? v2 : nullptr);
   PST_TRY(arena_b.alloc(BL.total_b), "Error in allocating construction arrays");
+  unsigned char* base_a = arena_a.as<unsigned char>();
   unsigned char* base_b = arena_b.as<unsigned char>();
-  K* key1 = reinterpret_cast<K*>(base_b + BL.key1);
-  uint32_t* v1 = reinterpret_cast<uint32_t*>(base_b + BL.v1);
-  uint32_t* r2 = reinterpret_cast<uint32_t*>(base_b + BL.r2);
+  // flags[0]: NaN seen; flags[1]: IDs not in index order (a point sort: keys
+  // and values do not stand for the points); flags[2]: a sort's wait ran out
+  int* flags = reinterpret_cast<int*>(base_a + BL.flags);
   void* tmp = base_b + BL.tmp;
-  uint32_t* starts_d = reinterpret_cast<uint32_t*>(base_b + BL.starts);
-  uint32_t* tileseg_d = reinterpret_cast<uint32_t*>(base_b + BL.tileseg);
-  // level tables, which depend on n alone: segment starts of levels 0..t0
-  // and, per level t < t0 and tile of kLevelTile points, the segment
-  // holding the tile's first point (so that no workgroup searches the
-  // starts itself)
-  {
-    const uint32_t nstart = (2u << BL.t0) - 1u;
-    k_level_starts<<<grid_for(nstart, 256), 256, 0, s>>>(n64 + 1, nstart, starts_d);
-    if (BL.t0 > 0) {
-      const uint64_t cells = static_cast<uint64_t>(BL.t0) * BL.tile_stride;
-      k_tile_segments<<<grid_for(cells, 256), 256, 0, s>>>(starts_d, static_cast<uint32_t>(n64), BL.t0,
-                                                           static_cast<uint32_t>(BL.tile_stride), tileseg_d);
-    }
-  }
-  // stable radix sort of (key, value) pairs: kin/vin to kout/vout
-  auto sortK = [&](const K* kin, K* kout, const uint32_t* vin, uint32_t* vout) -> hipError_t {
-    size_t tb = BL.tmp_bytes;
-    if constexpr (sizeof(K) == 4) return radix_sort_u32(tmp, tb, kin, kout, vin, vout, n, s, flags + 2);
-    else return radix_sort_u64(tmp, tb, kin, kout, vin, vout, n, s, flags + 2);
+  auto read_flags = [&](int (&h)[3]) -> hipError_t {
+    hipError_t r = hipMemcpyAsync(h, flags, sizeof(h), hipMemcpyDeviceToHost, s);
+    return r == hipSuccess ? hipStreamSynchronize(s) : r;
   };
-  bool ordered = true;
-  if constexpr (kHasId) {
-    int hflags[2] = {0, 0};
-    PST_TRY(hipMemcpyAsync(hflags, flags, sizeof(hflags), hipMemcpyDeviceToHost, s), "Error in reading construction flags");
-    PST_TRY(hipStreamSynchronize(s), "Error in synchronising construction");
-    ordered = hflags[1] == 0;
-  }
-  if (ordered) {
-    PST_TRY(sortK(key0, key1, v0, v1), "Error in sorting by dimension 2");
-  } else {
-    if constexpr (kHasId) {
-      k_keys_id<T, I, K, true><<<G, B, 0, s>>>(pts, n, key0, v0, nan_flag);
-      PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by ID");
-      k_keys_dim_perm<T, I, K, true, true><<<G, B, 0, s>>>(pts, n, v2, key0, v0, nullptr, nan_flag);
-      PST_TRY(sortK(key0, key1, v0, v1), "Error in sorting by dimension 2");
-    }
-  }
-  const uint32_t* perm2 = v1;
-  k_scatter_rank<<<G, B, 0, s>>>(perm2, n, r2);
-  // ---- key1 ascending, carrying r2 -> A (v2; v0 when the dim1 keys came
-  // with the dim2 keys, whose sort reads them from v2 and r2 in place)
-  uint32_t* Acur = v2;
-  uint32_t* Anxt = v0;
-  if (ordered && kKey1First) {
-    PST_TRY(sortK(reinterpret_cast<const K*>(v2), key0, r2, v0), "Error in sorting by dimension 1");
-    std::swap(Acur, Anxt);
-  } else if (ordered) {
-    k_keys_single<T, I, K, false, false, false><<<G, B, 0, s>>>(pts, n, key0, v0, r2, flags);
-    PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by dimension 1");
-  } else {
-    if constexpr (kHasId) {
-      k_keys_id<T, I, K, false><<<G, B, 0, s>>>(pts, n, key0, v0, nan_flag);
-      PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by ID");
-      k_keys_dim_perm<T, I, K, false, false><<<G, B, 0, s>>>(pts, n, v2, key0, v0, r2, nan_flag);
-      PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by dimension 1");
-    }
-  }
-  mark(1);
-  // the output arrays: the caller's hook allocates them while the sorts run
-  if (out.alloc) {
+  int hflag[3] = {0, 0, 0};
+  mark(0);
+  PST_TRY(hipMemsetAsync(flags, 0, 3 * sizeof(int), s), "Error in clearing construction flags");
+  // the output arrays: the caller's hook allocates them while the first pass runs
+  auto out_arrays = [&]() -> Status {
+    if (!out.alloc || out.nodes) return Status{};
     Status sa = out.alloc(out);
-    if (!sa.ok()) {
-      (void)hipStreamSynchronize(s);  // the queued passes still use the scratch
-      return sa;
+    if (!sa.ok()) (void)hipStreamSynchronize(s);  // the queued passes still use the scratch
+    return sa;
+  };
+  bool direct = false;
+  if constexpr (sizeof(T) == 4 && sizeof(K) == 4) {
+    if (point_sort_takes(dtype, id_dtype)) {
+      PST_TRY(point_sort_count(dtype, id_dtype, pts_v, n64, tmp, flags, s), "Error in counting construction keys");
+      st = out_arrays();
+      if (!st.ok()) return st;
+      PST_TRY(read_flags(hflag), "Error in reading construction flags");
+      direct = hflag[1] == 0 && hflag[0] == 0;
+      if (direct) {
+        uint32_t* key_x = reinterpret_cast<uint32_t*>(base_a + BL.key0);
+        uint64_t* val_x = reinterpret_cast<uint64_t*>(base_a + BL.v0);  // v0 and v2
+        uint32_t* key1 = reinterpret_cast<uint32_t*>(base_b + BL.key1);
+        uint64_t* val = reinterpret_cast<uint64_t*>(base_b + BL.v1);    // v1 and r2
+        PST_TRY(point_sort_passes(dtype, id_dtype, pts_v, n64, tmp, key_x, val_x, key1, val, flags + 2, s),
+                "Error in sorting by dimension 1");
+        mark(1);
+        st = build_levels<T, IS>(Direct<T, IS>{key1, id_dtype}, val, n, BL.t0, base_b + BL.mins, base_b + BL.segs, out, s);
+        if (!st.ok()) return st;
+      }
     }
   }
-  auto* nodes = static_cast<Node<T, IS>*>(out.nodes);
-  void* submin_v = out.submin;
-  void* ids_v = out.ids;
-
-  // ---- level schedule (tables computed above)
-  const uint32_t t0 = BL.t0;
-  const size_t nmin = t0 ? (1ull << t0) - 1 : 1;
-  unsigned long long* segmin = reinterpret_cast<unsigned long long*>(base_b + BL.segmin);
-  k_fill_u64<<<grid_for(nmin, B), B, 0, s>>>(segmin, nmin, ~0ull);
-  const uint32_t* starts = starts_d;
-  // level 0's minimum by its own pass; each emit pass then finds the next
-  // level's minima while compacting. Segment sizes within a level differ by
-  // at most one, and some segment of every level t < t0 holds more than
-  // kFinishTile points, so all hold at least kFinishTile: a tile of
-  // kLevelTile points meets at most kLevelTile / kFinishTile + 2 segments,
-  // twice as many children.
-  // Levels with at most kReduceSegs segments combine the tiles' minima by a
-  // reduction instead of global atomics.
-  constexpr uint32_t kReduceSegs = 32;
-  unsigned long long* tmin = reinterpret_cast<unsigned long long*>(base_b + BL.tmin);
-  if (t0 > 0) {
-    k_level_argmin<<<grid_for(n, kLevelTile), kLevelBlock, 0, s>>>(Acur, n, 1u, starts, tileseg_d, tmin);
-    k_tile_min_reduce<<<1, kLevelBlock, 0, s>>>(tmin, kSegSlots, tileseg_d, starts, 1u, n, 0u, segmin);
-  }
-  for (uint32_t t = 0; t < t0; t++) {
-    const uint32_t n_level = n - ((1u << t) - 1);
-    const unsigned tiles = grid_for(n_level, kLevelTile);
-    unsigned long long* nextmin = t + 1 < t0 ? segmin + (2u << t) - 1 : nullptr;
-    const bool reduce = nextmin && (1u << t) <= kReduceSegs;
-    const uint32_t* st_t = starts + (1u << t) - 1;
-    const uint32_t* ts_t = tileseg_d + static_cast<size_t>(t) * BL.tile_stride;
-    k_level_emit<T, IS><<<tiles, kLevelBlock, 0, s>>>(Acur, Anxt, n_level, t, M, st_t, ts_t, segmin + (1u << t) - 1,
-                                                      nextmin, reduce ? tmin : nullptr, perm2, ptsS, nodes);
-    if (reduce)
-      k_tile_min_reduce<<<2u << t, kLevelBlock, 0, s>>>(tmin, 2 * kSegSlots, ts_t, st_t, 1u << t, n_level, 1u,
-                                                        nextmin);
-    std::swap(Acur, Anxt);
+  if (!direct) {
+    PST_TRY(hipMemsetAsync(flags, 0, 3 * sizeof(int), s), "Error in clearing construction flags");
+    K* key0 = reinterpret_cast<K*>(base_a + BL.key0);
+    uint32_t* v0 = reinterpret_cast<uint32_t*>(base_a + BL.v0);
+    uint32_t* v2 = reinterpret_cast<uint32_t*>(base_a + BL.v2);
+    K* key1 = reinterpret_cast<K*>(base_b + BL.key1);
+    uint32_t* v1 = reinterpret_cast<uint32_t*>(base_b + BL.v1);
+    uint32_t* r2 = reinterpret_cast<uint32_t*>(base_b + BL.r2);
+    const unsigned B = 256;
+    const unsigned G = grid_for(n, B);
+    int* nan_flag = flags;
+    // ---- key2 descending -> perm2 (v1), r2. One sort by dim2 when the IDs
+    // are in index order (the sort's index tie-break is then the (id, index)
+    // tie-break), else a sort by ID and then a stable one by dim2.
+    // 32-bit keys: the dim1 keys are stored by the same kernel, into v2
+    constexpr bool kKey1First = sizeof(K) == 4;
+    k_keys_single<T, I, K, true, true, false, kHasId>
+        <<<G, B, 0, s>>>(pts, n, key0, v0, nullptr, flags, kKey1First ? v2 : nullptr);
+    // stable radix sort of (key, value) pairs: kin/vin to kout/vout
+    auto sortK = [&](const K* kin, K* kout, const uint32_t* vin, uint32_t* vout) -> hipError_t {
+      size_t tb = BL.tmp_bytes;
+      if constexpr (sizeof(K) == 4) return radix_sort_u32(tmp, tb, kin, kout, vin, vout, n, s, flags + 2);
+      else return radix_sort_u64(tmp, tb, kin, kout, vin, vout, n, s, flags + 2);
+    };
+    st = out_arrays();
+    if (!st.ok()) return st;
+    bool ordered = true;
+    if constexpr (kHasId) {
+      PST_TRY(read_flags(hflag), "Error in reading construction flags");
+      ordered = hflag[1] == 0;
+    }
+    if (ordered) {
+      PST_TRY(sortK(key0, key1, v0, v1), "Error in sorting by dimension 2");
+    } else {
+      if constexpr (kHasId) {
+        k_keys_id<T, I, K, true><<<G, B, 0, s>>>(pts, n, key0, v0, nan_flag);
+        PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by ID");
+        k_keys_dim_perm<T, I, K, true, true><<<G, B, 0, s>>>(pts, n, v2, key0, v0, nullptr, nan_flag);
+        PST_TRY(sortK(key0, key1, v0, v1), "Error in sorting by dimension 2");
+      }
+    }
+    const uint32_t* perm2 = v1;
+    k_scatter_rank<<<G, B, 0, s>>>(perm2, n, r2);
+    // ---- key1 ascending, carrying r2 -> A (v2; v0 when the dim1 keys came
+    // with the dim2 keys, whose sort reads them from v2 and r2 in place)
+    const uint32_t* A = v2;
+    if (ordered && kKey1First) {
+      PST_TRY(sortK(reinterpret_cast<const K*>(v2), key0, r2, v0), "Error in sorting by dimension 1");
+      A = v0;
+    } else if (ordered) {
+      k_keys_single<T, I, K, false, false, false><<<G, B, 0, s>>>(pts, n, key0, v0, r2, flags);
+      PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by dimension 1");
+    } else {
+      if constexpr (kHasId) {
+        k_keys_id<T, I, K, false><<<G, B, 0, s>>>(pts, n, key0, v0, nan_flag);
+        PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by ID");
+        k_keys_dim_perm<T, I, K, false, false><<<G, B, 0, s>>>(pts, n, v2, key0, v0, r2, nan_flag);
+        PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by dimension 1");
+      }
+    }
+    mark(1);
+    st = build_levels<T, IS>(Ranked<T, IS>{perm2, static_cast<const Point<T, IS>*>(pts_v)}, A, n, BL.t0,
+                             base_b + BL.mins, base_b + BL.segs, out, s);
+    if (!st.ok()) return st;
   }
   mark(2);
-  k_finish<T, IS><<<1u << t0, kFinishBlock, 0, s>>>(Acur, t0, M, starts + (1u << t0) - 1, perm2, ptsS, nodes,
-                                                    static_cast<T*>(submin_v), static_cast<IS*>(ids_v));
-  // subtree minima and IDs of the slots above the LDS subtrees
-  if (submin_v && t0 > 0) {
-    const uint32_t M32 = static_cast<uint32_t>(M);
-    Status st2 = submin_typed<T, IS>(nodes, submin_v, ids_v, t0, 31u, 1u, M32, M32, s);
-    if (!st2.ok()) return st2;
-  }
-  mark(3);
-  PST_TRY(hipGetLastError(), "Error in launching construction kernels");
-  int hflag[3] = {0, 0, 0};
-  PST_TRY(hipMemcpyAsync(hflag, flags, sizeof(hflag), hipMemcpyDeviceToHost, s),
-          "Error in reading construction flag");
-  PST_TRY(hipStreamSynchronize(s), "Error in synchronising after construction");
+  PST_TRY(read_flags(hflag), "Error in synchronising after construction");
   arena_b.release_idle();
   arena_a.release_idle();
   if (times) {
     hipEventElapsedTime(&times->sort_ms, ev[0], ev[1]);
     hipEventElapsedTime(&times->levels_ms, ev[1], ev[2]);
-    hipEventElapsedTime(&times->finish_ms, ev[2], ev[3]);
     for (auto& x : ev) hipEventDestroy(x);
   }
   if (hflag[2]) {
@@ -1356,7 +1451,7 @@ Status with_id(int idt, F&& f) {
 Status build_tree(int dtype, int id_dtype, const void* pts_d, size_t n, BuildOut& out, hipStream_t stream,
                   BuildTimes* times) {
   return with_t(dtype, [&](auto t) {
-    return with_id(id_dtype, [&](auto i) { return build_typed<decltype(t), decltype(i)>(pts_d, n, out, stream, times); });
+    return with_id(id_dtype, [&](auto i) { return build_typed<decltype(t), decltype(i)>(dtype, id_dtype, pts_d, n, out, stream, times); });
   });
 }
 

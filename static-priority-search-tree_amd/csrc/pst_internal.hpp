@@ -35,7 +35,7 @@ size_t dtype_size(int dtype);
 
 // ---- construction (pst_build.hip) ----
 struct BuildTimes {
-  float keys_ms = 0, sort_ms = 0, levels_ms = 0, finish_ms = 0;
+  float sort_ms = 0, levels_ms = 0;  // up to the key1-ordered array; from there on
 };
 // Builds the tree for n AoS points (device pointer) into `nodes`, which
 // holds S = 2^ceil(log2(n+1)) - 1 records. Returns PST_ERR_NAN if a NaN dim
@@ -92,6 +92,20 @@ Status export_forest(int dtype, int id_dtype, size_t n, size_t slots_per_tree, c
 // (slots_per_tree > 0), after construction.
 Status build_submin(int dtype, int id_dtype, size_t n, size_t slots_per_tree, const void* nodes_d, void* submin_d,
                     void* ids_d, hipStream_t stream);
+
+// ---- points sorted by dim1 (pst_sort.hip) ----
+// A stable sort of points with 32-bit dims and 32-bit IDs or none by
+// ord_key(dim1), carrying the value (~ord_key(dim2)) << 32 | ~ord_key(id)
+// (~index without IDs). point_sort_count reads the points once: digit totals
+// into tmp (point_sort_tmp_bytes), flags[0] = 1 on a NaN, flags[1] = 1 when
+// some value is -0 or the IDs do not rise strictly with the index (then keys
+// and values do not stand for the points). point_sort_passes then sorts;
+// key_x and val_x are scratch of the outputs' sizes.
+bool point_sort_takes(int dtype, int id_dtype);
+size_t point_sort_tmp_bytes(size_t n);
+hipError_t point_sort_count(int dtype, int id_dtype, const void* pts_d, size_t n, void* tmp, int* flags, hipStream_t s);
+hipError_t point_sort_passes(int dtype, int id_dtype, const void* pts_d, size_t n, void* tmp, uint32_t* key_x,
+                             uint64_t* val_x, uint32_t* key_out, uint64_t* val_out, int* fail, hipStream_t s);
 
 // ---- device memory (pst_memory.cpp) ----
 // hipMalloc on the current device through the library's bounded cache of

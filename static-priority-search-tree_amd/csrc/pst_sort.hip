@@ -147,11 +147,12 @@ __global__ __launch_bounds__(kDigits) void k_digit_starts(uint32_t* __restrict__
   }
 }
 
-template <typename K>
+template <typename K, typename V>
 struct PassLds {
   union {
     unsigned long long peer[kPassWaves][kDigits];  // while ranking: per-wave lane masks of a round's digits
-    K sbuf[kSortTile];                             // then keys, then values, in (digit, rank) order
+    K sbuf[kSortTile];                             // then keys,
+    V vbuf[kSortTile];                             // then values, in (digit, rank) order
   };
   uint32_t wcnt[kPassWaves][kDigits];   // per-wave digit counters, then their wave prefix
   uint32_t dcnt[kDigits];               // the tile's count of each digit
@@ -161,11 +162,46 @@ struct PassLds {
   uint32_t tile;
 };
 
+// Where a pass reads its pairs: key and value arrays, the value when the
+// keys are ranked (value() is called again then).
+template <typename K, typename V>
+struct ArraySrc {
+  const K* kin;
+  const V* vin;
+  __device__ void at(uint64_t base) {
+    kin += base;
+    vin += base;
+  }
+  __device__ K key(uint32_t i) const { return kin[i]; }
+  __device__ V value(uint32_t i) const { return vin[i]; }
+};
+
+// Or the points themselves (the first pass of a point sort): the key is the
+// dim1 key, the value (~dim2 key, ~ID key), ~index where there is no ID, so
+// that of two values the smaller one belongs to the greater point in
+// (dim2, ID) order.
+template <typename T, typename I>
+struct PointSrc {
+  const Point<T, I>* pts;
+  uint32_t first;
+  __device__ void at(uint64_t base) {
+    pts += base;
+    first = static_cast<uint32_t>(base);
+  }
+  __device__ uint32_t key(uint32_t i) const { return ord_key(pts[i].dim1_val); }
+  __device__ uint64_t value(uint32_t i) const {
+    const Point<T, I> p = pts[i];
+    uint32_t lo = first + i;
+    if constexpr (has_id_v<I>) lo = ord_key(p.id);
+    return (static_cast<uint64_t>(~ord_key(p.dim2_val)) << 32) | static_cast<uint32_t>(~lo);
+  }
+};
+
 // One tile of a digit pass. FULL: the tile holds kSortTile keys, so no
 // element needs a bounds check (and each lane's loads share one address).
-template <typename K, bool FULL>
-__device__ __forceinline__ void sort_tile(PassLds<K>& L, const K* __restrict__ kin, const uint32_t* __restrict__ vin,
-                                          K* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t tile,
+template <typename K, typename V, bool FULL, typename Src>
+__device__ __forceinline__ void sort_tile(PassLds<K, V>& L, Src src,
+                                          K* __restrict__ kout, V* __restrict__ vout, uint32_t tile,
                                           uint32_t valid, uint32_t pass, unsigned long long* __restrict__ status,
                                           const uint32_t* __restrict__ gstart, int* __restrict__ fail) {
   const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
@@ -173,11 +209,11 @@ __device__ __forceinline__ void sort_tile(PassLds<K>& L, const K* __restrict__ k
   const uint64_t base = static_cast<uint64_t>(tile) * kSortTile;
   const uint32_t wbase = wave * kWaveKeys;
   auto in_tile = [&](uint32_t i) { return FULL || i < valid; };
-  const K* kp = kin + base + wbase + lane;
+  src.at(base + wbase);
   K k[kPassPer];
 #pragma unroll
   for (int r = 0; r < kPassPer; r++)
-    if (in_tile(wbase + r * kWave + lane)) k[r] = kp[r * kWave];
+    if (in_tile(wbase + r * kWave + lane)) k[r] = src.key(r * kWave + lane);
   // stable rank within the wave: rounds in element order, lanes in order.
   // The lanes of a round that share a digit find each other through the
   // wave's peer word of that digit: each ORs in its lane bit, all read the
@@ -251,11 +287,10 @@ __device__ __forceinline__ void sort_tile(PassLds<K>& L, const K* __restrict__ k
       rank[r] = p;
     }
   }
-  const uint32_t* vp = vin + base + wbase + lane;
-  uint32_t v[kPassPer];
+  V v[kPassPer];
 #pragma unroll
   for (int r = 0; r < kPassPer; r++)
-    if (in_tile(wbase + r * kWave + lane)) v[r] = vp[r * kWave];
+    if (in_tile(wbase + r * kWave + lane)) v[r] = src.value(r * kWave + lane);
   // look-back: the digit's count over the tiles before this one
   if (tid < kDigits) {
     const uint32_t run = L.dcnt[tid];
@@ -316,30 +351,30 @@ __device__ __forceinline__ void sort_tile(PassLds<K>& L, const K* __restrict__ k
     }
   }
   __syncthreads();
-  uint32_t* sval = reinterpret_cast<uint32_t*>(L.sbuf);
 #pragma unroll
   for (int r = 0; r < kPassPer; r++)
-    if (in_tile(wbase + r * kWave + lane)) sval[rank[r]] = v[r];
+    if (in_tile(wbase + r * kWave + lane)) L.vbuf[rank[r]] = v[r];
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < kPassPer; r++) {
     const uint32_t i = r * kPassBlock + tid;
-    if (in_tile(i)) vout[g[r]] = sval[i];
+    if (in_tile(i)) vout[g[r]] = L.vbuf[i];
   }
 }
 
 // One digit pass: tiles in counter order, look-back over the published
 // per-digit counts of earlier tiles, then a stable scatter.
-// Six waves per SIMD: three workgroups per CU for 32-bit keys (LDS bounds
-// 64-bit keys to two).
-template <typename K>
-__global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_sort_pass(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
-                                                          K* __restrict__ kout, uint32_t* __restrict__ vout,
+// Six waves per SIMD: three workgroups per CU for 32-bit keys and values (LDS
+// bounds 64-bit keys or values to two, four waves per SIMD).
+template <typename K, typename V, typename Src>
+__global__ __launch_bounds__(kPassBlock)
+__attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 ? 4 : 6))) void k_sort_pass(Src src, K* __restrict__ kout,
+                                                          V* __restrict__ vout,
                                                           uint32_t n, uint32_t pass, uint32_t* __restrict__ tile_ctr,
                                                           unsigned long long* __restrict__ status,
                                                           const uint32_t* __restrict__ gstart,
                                                           int* __restrict__ fail) {
-  __shared__ PassLds<K> L;
+  __shared__ PassLds<K, V> L;
   const uint32_t tid = threadIdx.x;
   if (tid == 0) L.tile = atomicAdd(&tile_ctr[pass], 1u);
   for (uint32_t i = tid; i < kPassWaves * kDigits; i += kPassBlock) {
@@ -354,9 +389,9 @@ __global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(6)))
   const uint32_t rem = n - tile * kSortTile;
   const uint32_t valid = rem < kSortTile ? rem : kSortTile;
   if (valid == kSortTile)
-    sort_tile<K, true>(L, kin, vin, kout, vout, tile, valid, pass, status, gstart, fail);
+    sort_tile<K, V, true>(L, src, kout, vout, tile, valid, pass, status, gstart, fail);
   else
-    sort_tile<K, false>(L, kin, vin, kout, vout, tile, valid, pass, status, gstart, fail);
+    sort_tile<K, V, false>(L, src, kout, vout, tile, valid, pass, status, gstart, fail);
 }
 
 inline size_t align256(size_t b) { return (b + 255) & ~size_t{255}; }
@@ -406,15 +441,167 @@ hipError_t radix_sort(void* tmp, size_t& tmp_bytes, const K* kin, K* kout, const
     const bool to_out = ((passes - pass) % 2) == 1;
     K* kdst = to_out ? kout : kt;
     uint32_t* vdst = to_out ? vout : vt;
-    hipLaunchKernelGGL((k_sort_pass<K>), dim3(static_cast<unsigned>(ntiles)), dim3(kPassBlock), 0, s, ksrc, vsrc,
-                       kdst, vdst, n32, pass, ctr, status, hist + pass * kDigits, fail);
+    hipLaunchKernelGGL((k_sort_pass<K, uint32_t, ArraySrc<K, uint32_t>>), dim3(static_cast<unsigned>(ntiles)),
+                       dim3(kPassBlock), 0, s, ArraySrc<K, uint32_t>{ksrc, vsrc}, kdst, vdst, n32, pass, ctr, status,
+                       hist + pass * kDigits, fail);
     ksrc = kdst;
     vsrc = vdst;
   }
   return hipGetLastError();
 }
 
+// ---- points by dim1, with 64-bit values (pst_internal.hpp) ----
+//
+// The first pass reads the points themselves, so no key arrays are written
+// beforehand. 2^26 f32/u32 points on MI355X: 0.20 ms for the digit totals,
+// 0.45 ms for the first pass and 0.43 ms for each later one (24 B moved per
+// point, 3.7 TB/s; LDS holds two workgroups per CU): 1.95 ms where the two
+// sorts of 32-bit values with their key and rank-scatter kernels took 4.2.
+
+constexpr uint32_t kPointPasses = 4;
+
+// Digit totals of the points' dim1 keys, and what the points allow: flags[0]
+// a NaN dim or ID, flags[1] a value that its key does not give back (-0) or
+// IDs that do not rise strictly with the index.
+template <typename T, typename I>
+__global__ __launch_bounds__(kHistBlock) void k_point_hist(const Point<T, I>* __restrict__ pts, uint32_t n,
+                                                           uint32_t* __restrict__ hist, int* __restrict__ flags) {
+  constexpr int P = kPointPasses;
+  __shared__ uint32_t h[kSub][P][kDigits];
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t i = tid; i < kSub * P * kDigits; i += kHistBlock) (&h[0][0][0])[i] = 0u;
+  __syncthreads();
+  uint32_t(*mine)[kDigits] = h[tid % kSub];
+  bool bad = false, plain = true;
+  auto lossless = [](auto v) {
+    if constexpr (std::is_floating_point<decltype(v)>::value) return __builtin_bit_cast(uint32_t, v) != 0x80000000u;
+    else return true;
+  };
+  for (uint64_t b = static_cast<uint64_t>(blockIdx.x) * kHistChunk; b < n;
+       b += static_cast<uint64_t>(gridDim.x) * kHistChunk) {
+#pragma unroll 4
+    for (int e = 0; e < kHistPer; e++) {
+      const uint64_t i = b + static_cast<uint64_t>(e) * kHistBlock + tid;
+      const bool ok = i < n;
+      uint32_t k = 0;
+      if (ok) {
+        const Point<T, I> p = pts[i];
+        bad |= is_nan(p.dim1_val) || is_nan(p.dim2_val);
+        plain &= lossless(p.dim1_val) && lossless(p.dim2_val);
+        if constexpr (has_id_v<I>) {
+          bad |= is_nan(p.id);
+          plain &= lossless(p.id);
+          if (i + 1 < n) plain &= ord_key(p.id) < ord_key(pts[i + 1].id);
+        }
+        k = ord_key(p.dim1_val);
+#pragma unroll
+        for (int q = 0; q < P - 1; q++) atomicAdd(&mine[q][digit_of(k, q * kDigitBits)], 1u);
+      }
+      const uint32_t d = digit_of(k, (P - 1) * kDigitBits);
+      const uint64_t act = __ballot(ok);
+      const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
+      if (act == ~0ull && __ballot(d != d0) == 0ull) {
+        if (tid % kWave == 0) atomicAdd(&h[0][P - 1][d0], static_cast<uint32_t>(kWave));
+      } else if (ok) {
+        atomicAdd(&mine[P - 1][d], 1u);
+      }
+    }
+  }
+  if (bad) flags[0] = 1;
+  if (!plain) flags[1] = 1;
+  __syncthreads();
+  for (uint32_t i = tid; i < P * kDigits; i += kHistBlock) {
+    uint32_t c = 0;
+#pragma unroll
+    for (int u = 0; u < kSub; u++) c += (&h[u][0][0])[i];
+    if (c) atomicAdd(&hist[i], c);
+  }
+}
+
+struct PointSortTmp {
+  unsigned long long* status;
+  uint32_t* ctr;
+  uint32_t* hist;
+  size_t words;  // from status on, cleared once per sort
+};
+PointSortTmp point_sort_tmp(void* tmp, size_t n) {
+  const size_t ntiles = (n + kSortTile - 1) / kSortTile;
+  const size_t status_bytes = std::max<size_t>(ntiles, 1) * kDigits * 8;
+  PointSortTmp t{};
+  auto* p = static_cast<unsigned char*>(tmp);
+  t.status = reinterpret_cast<unsigned long long*>(p);
+  t.ctr = reinterpret_cast<uint32_t*>(p + status_bytes);
+  t.hist = reinterpret_cast<uint32_t*>(p + status_bytes + 256);
+  t.words = (status_bytes + 256 + kPointPasses * kDigits * 4) / 4;
+  return t;
+}
+
+template <typename F>
+hipError_t with_point(int dtype, int id_dtype, F&& f) {
+  auto ids = [&](auto t) {
+    switch (id_dtype) {
+      case NO_ID: return f(t, NoId{});
+      case F32: return f(t, float{});
+      case I32: return f(t, int32_t{});
+      case U32: return f(t, uint32_t{});
+    }
+    return hipErrorInvalidValue;
+  };
+  switch (dtype) {
+    case F32: return ids(float{});
+    case I32: return ids(int32_t{});
+  }
+  return hipErrorInvalidValue;
+}
+
 }  // namespace
+
+bool point_sort_takes(int dtype, int id_dtype) {
+  return (dtype == F32 || dtype == I32) && (id_dtype == NO_ID || id_dtype == F32 || id_dtype == I32 || id_dtype == U32);
+}
+
+size_t point_sort_tmp_bytes(size_t n) { return align256(point_sort_tmp(nullptr, n).words * 4); }
+
+hipError_t point_sort_count(int dtype, int id_dtype, const void* pts_d, size_t n, void* tmp, int* flags,
+                            hipStream_t s) {
+  const PointSortTmp t = point_sort_tmp(tmp, n);
+  hipLaunchKernelGGL(k_fill_zero, dim3(static_cast<unsigned>((t.words + 255) / 256)), dim3(256), 0, s,
+                     reinterpret_cast<uint32_t*>(t.status), t.words);
+  const unsigned blocks = static_cast<unsigned>(std::min<size_t>((n + kHistChunk - 1) / kHistChunk, kHistMaxBlocks));
+  return with_point(dtype, id_dtype, [&](auto tv, auto iv) {
+    using Pt = Point<decltype(tv), decltype(iv)>;
+    hipLaunchKernelGGL((k_point_hist<decltype(tv), decltype(iv)>), dim3(blocks), dim3(kHistBlock), 0, s,
+                       static_cast<const Pt*>(pts_d), static_cast<uint32_t>(n), t.hist, flags);
+    return hipGetLastError();
+  });
+}
+
+hipError_t point_sort_passes(int dtype, int id_dtype, const void* pts_d, size_t n, void* tmp, uint32_t* key_x,
+                             uint64_t* val_x, uint32_t* key_out, uint64_t* val_out, int* fail, hipStream_t s) {
+  const PointSortTmp t = point_sort_tmp(tmp, n);
+  const uint32_t n32 = static_cast<uint32_t>(n);
+  const dim3 grid(static_cast<unsigned>((n + kSortTile - 1) / kSortTile)), block(kPassBlock);
+  hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kDigits), 0, s, t.hist, kPointPasses);
+  hipError_t e = with_point(dtype, id_dtype, [&](auto tv, auto iv) {
+    using Src = PointSrc<decltype(tv), decltype(iv)>;
+    using Pt = Point<decltype(tv), decltype(iv)>;
+    hipLaunchKernelGGL((k_sort_pass<uint32_t, uint64_t, Src>), grid, block, 0, s, Src{static_cast<const Pt*>(pts_d), 0u},
+                       key_x, val_x, n32, 0u, t.ctr, t.status, t.hist, fail);
+    return hipGetLastError();
+  });
+  using Src = ArraySrc<uint32_t, uint64_t>;
+  const uint32_t* ks = key_x;
+  const uint64_t* vs = val_x;
+  for (uint32_t pass = 1; pass < kPointPasses && e == hipSuccess; pass++) {
+    const bool out = pass % 2 == 1;  // the last pass (3) writes the outputs
+    hipLaunchKernelGGL((k_sort_pass<uint32_t, uint64_t, Src>), grid, block, 0, s, Src{ks, vs}, out ? key_out : key_x,
+                       out ? val_out : val_x, n32, pass, t.ctr, t.status, t.hist + pass * kDigits, fail);
+    ks = out ? key_out : key_x;
+    vs = out ? val_out : val_x;
+    e = hipGetLastError();
+  }
+  return e;
+}
 
 hipError_t radix_sort_u32(void* tmp, size_t& tmp_bytes, const uint32_t* kin, uint32_t* kout, const uint32_t* vin,
                           uint32_t* vout, size_t n, hipStream_t s, int* fail) {

@@ -25,7 +25,7 @@ struct pst_tree {
   size_t slots_per_tree = 0;  // forest (StaticPSTGPUArr): slots of a full tree; 0 for one deep tree
   void* tree_bounds = nullptr;  // forest: each tree's dim1 range (stationary batch passes)
   pst::SearchScratch sc;
-  int rounds = 4, budget_small = 0, budget_large = 0, waves_per_cu = 0;
+  int rounds = 0, budget_small = 0, budget_large = 0, waves_per_cu = 0;
   int group = pst::kGroup;  // queries per walk in batched searches
   int copy_min = 256, copy_max = 65535;  // write pass: full subtrees copied in this size range
   size_t copy_tasks = 0;                 // copy task list entries (0: library default)
@@ -35,6 +35,7 @@ struct pst_tree {
   hipStream_t stream = nullptr;
   unsigned long long* debug = nullptr;  // per-round search counters (debug builds)
   int graphs = 0;  // live batch graphs: they hold the scratch and index addresses
+  unsigned long long* host = nullptr;  // pinned words of blocking searches
 };
 
 namespace {
@@ -151,13 +152,37 @@ int single_search(pst_tree* t, int kind, int ret, const void* a, const void* b, 
   args.cap_all = cap;
   args.out = out;
   const bool via_index = t->lv_key && ret != PST_RET_POINT;
-  st = via_index ? pst::level_search(args, t->lv_key, t->lv_id, t->lsc, s) : pst::run_search(args, t->sc, s);
-  if (!st.ok()) return fail(st);
+  if (!t->host) t->host = pst::host_words_take();
+  // a deep tree's walk starts as one workgroup that most searches end in
+  const bool front = !via_index && t->host && !t->slots_per_tree && !t->debug;
   unsigned long long host[2] = {0, 0};
-  hipError_t e = hipMemcpyAsync(&host[0], t->sc.cursor, 8, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess && !via_index)
-    e = hipMemcpyAsync(&host[1], pst::search_error_flag(t->sc), 8, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  hipError_t e = hipSuccess;
+  bool read = true;  // results are copied from the device
+  if (front) {
+    st = pst::search_front(args, t->sc, false, t->host, s);
+    if (!st.ok()) return fail(st);
+    e = hipStreamSynchronize(s);
+    const volatile unsigned long long* h = t->host;
+    host[0] = h[0];
+    host[1] = h[1];
+    read = e == hipSuccess && host[1] == 0 && h[2] != 0;
+    if (read) st = pst::search_front(args, t->sc, true, t->host, s);
+  } else {
+    args.host = t->host;
+    st = via_index ? pst::level_search(args, t->lv_key, t->lv_id, t->lsc, s) : pst::run_search(args, t->sc, s);
+    if (via_index && t->host && st.ok()) {
+      e = hipStreamSynchronize(s);
+      host[0] = *static_cast<const volatile unsigned long long*>(t->host);
+      read = false;
+    }
+  }
+  if (!st.ok()) return fail(st);
+  if (read) {
+    e = hipMemcpyAsync(&host[0], t->sc.cursor, 8, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess && !via_index)
+      e = hipMemcpyAsync(&host[1], pst::search_error_flag(t->sc), 8, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+  }
   if (e != hipSuccess)
     return fail(PST_ERR_HIP, "Error in copying global result array final index from device" +
                                  dev_suffix(t->dev_ind, t->num_devs) + hipGetErrorString(e));
@@ -386,6 +411,7 @@ int pst_gpu_destroy(pst_tree* t) {
   }
   pst::scratch_release(t->sc, idle);
   pst::level_scratch_release(t->lsc, idle);
+  pst::host_words_give(t->host);
   const int di = t->dev_ind, nd = t->num_devs;
   delete t;
   if (e != hipSuccess)
@@ -861,6 +887,9 @@ int pst_gpu_autotune(pst_tree* t, const void* queries_d, size_t nq, int ret, pst
   t->group = best_cfg[4];
   if (chosen6) {
     for (int k = 0; k < 5; k++) chosen6[k] = best_cfg[k];
+    pst::SearchArgs a = base_args(t);
+    a.nq = nq;
+    chosen6[0] = pst::search_rounds(a);  // as set, or the default for this batch
     chosen6[5] = static_cast<int>(best * 500.0f);  // microseconds per batch (two timed repetitions)
   }
   return PST_OK;

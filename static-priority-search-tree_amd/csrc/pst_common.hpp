@@ -179,6 +179,26 @@ __host__ __device__ inline int64_t level_start(uint64_t M, uint32_t t, uint32_t 
   return static_cast<int64_t>(j) * base + extra;
 }
 
+// #{ j' < j : brev_t(j') < r } (positions are t-bit numbers; r may exceed
+// 2^t - 1, counting every position). Positions j' < j are grouped by the
+// highest bit b where they differ from j (bit b set in j, clear in j'):
+// the group's bit reversals are c + k 2^(t-b), k < 2^b.
+__host__ __device__ inline uint64_t brev_below(uint32_t t, uint32_t j, uint64_t r) {
+  uint64_t cnt = 0;
+  for (uint32_t b = 0; b < t; b++) {
+    if ((j >> b) & 1u) {
+      const uint64_t c = brev_bits((j >> b) ^ 1u, t - b);
+      if (r > c) {
+        const uint64_t step = 1ull << (t - b);
+        const uint64_t k = (r - c + step - 1) / step;
+        const uint64_t cap = 1ull << b;
+        cnt += k < cap ? k : cap;
+      }
+    }
+  }
+  return cnt;
+}
+
 // ---------------------------------------------------------------------------
 // Search state of a query at a node, as bits j of three masks for the G
 // queries of a group: `a` the query is walking this subtree, `l` its lower

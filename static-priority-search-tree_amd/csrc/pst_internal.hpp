@@ -124,6 +124,10 @@ hipError_t dev_free(void* p);
 hipError_t dev_free_idle(void* p);
 // Waits for the work of the device that holds the block p.
 hipError_t dev_wait(const void* p);
+// Four words of pinned host memory that kernels of every device can write
+// (null: none left), for results a blocking call returns; and back.
+unsigned long long* host_words_take();
+void host_words_give(unsigned long long* p);
 
 // ---- searches on one deep tree (pst_search.hip) ----
 constexpr int kGroup = 8;  // queries per group walk in batched searches
@@ -142,6 +146,7 @@ struct SearchScratch {
   size_t gstack_bytes = 0;
   void* tasks = nullptr;  // copy tasks of write passes (16-byte entries)
   size_t task_cap = 0;
+  void* front = nullptr;  // copy tasks of one search's first launch
   void* fseg = nullptr;  // forest batches: per (query, segment) hit counts, then offsets
   size_t fseg_bytes = 0;
   // batch graphs of the handle hold these buffers' addresses: while any
@@ -173,7 +178,7 @@ struct SearchArgs {
   const unsigned long long* caps;     // mode 1 (nullable)
   unsigned long long cap_all;
   void* out;
-  int rounds;           // kernel launches enqueued (>= 1)
+  int rounds;           // kernel launches enqueued (0: by the batch's size, search_rounds)
   int budget_small, budget_large;
   int waves_per_cu;
   int group;            // 1: one query per walk; otherwise kGroup
@@ -184,8 +189,11 @@ struct SearchArgs {
   unsigned long long* debug;  // optional per-round counters (8 per round)
   unsigned long long out_total = ~0ull;  // records `out` holds (~0: unlimited; 0: nothing is written)
   const void* tree_bounds = nullptr;     // forest: each tree's dim1 range (T lo, hi)
+  unsigned long long* host = nullptr;    // one search through the level index: its count, in pinned host memory
 };
 Status run_search(const SearchArgs& a, SearchScratch& sc, hipStream_t stream);
+int search_rounds(const SearchArgs& a);
+Status search_front(const SearchArgs& a, SearchScratch& sc, bool rounds, unsigned long long* host, hipStream_t s);
 unsigned long long* search_error_flag(SearchScratch& sc);
 // offsets[q] = sum of in[0..q), offsets[n] = total (one workgroup).
 Status exclusive_scan(const unsigned long long* in, unsigned long long* offsets, size_t n, hipStream_t s);

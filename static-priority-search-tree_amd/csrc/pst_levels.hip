@@ -88,26 +88,6 @@ __device__ inline void load_run(const V* __restrict__ a, uint32_t base, uint32_t
   }
 }
 
-// #{ j' < j : brev_t(j') < r } (positions are t-bit numbers; r may exceed
-// 2^t - 1, counting every position). Positions j' < j are grouped by the
-// highest bit b where they differ from j (bit b set in j, clear in j'):
-// the group's bit reversals are c + k 2^(t-b), k < 2^b.
-__host__ __device__ inline uint64_t brev_below(uint32_t t, uint32_t j, uint64_t r) {
-  uint64_t cnt = 0;
-  for (uint32_t b = 0; b < t; b++) {
-    if ((j >> b) & 1u) {
-      const uint64_t c = brev_bits((j >> b) ^ 1u, t - b);
-      if (r > c) {
-        const uint64_t step = 1ull << (t - b);
-        const uint64_t k = (r - c + step - 1) / step;
-        const uint64_t cap = 1ull << b;
-        cnt += k < cap ? k : cap;
-      }
-    }
-  }
-  return cnt;
-}
-
 // Points of level-(t+1) positions 2j'' + side, j'' < j: the same-way points
 // of the level-t runs before run j.
 __host__ __device__ inline uint64_t side_before(uint64_t M, uint32_t t, uint32_t j, uint32_t side) {
@@ -296,6 +276,7 @@ struct LvParams {
   unsigned long long* wq;  // IDs written per query
   unsigned long long* woff;  // one query (use_single, write mode): its work offsets, written by the plan
   uint32_t* chunk_task;      // and its chunk table
+  unsigned long long* host;  // and its count, in pinned host memory (null: none)
 };
 
 // First index of the sorted run kk[0, len) whose key is above qk: a search
@@ -494,6 +475,8 @@ __global__ __launch_bounds__(kWave) void k_lv_plan(LvParams<T, IS> P) {
         if (lane == 0) {
           P.woff[0] = 0;
           P.woff[1] = clip;
+          if (P.host)
+            __hip_atomic_store(P.host, static_cast<unsigned long long>(total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
         const uint64_t L = chunk_len(clip, 1);
         auto mark = [&](uint32_t at, uint32_t pre, uint32_t c) {
@@ -830,6 +813,7 @@ Status level_search(const SearchArgs& a, const void* key_d, const void* id_d, Le
       if (a.single_query) {
         P.single = *static_cast<const Query<T>*>(a.single_query);
         P.use_single = 1;
+        P.host = a.host;
       }
       P.nq = static_cast<uint32_t>(a.nq);
       P.counts = a.counts;

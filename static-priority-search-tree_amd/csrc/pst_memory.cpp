@@ -95,6 +95,47 @@ std::vector<void*> take_kept(int dev) {
 
 }  // namespace
 
+// One pinned page per process, in slots of four words, taken by handles at
+// their first blocking search. Reading a result from it after the stream's
+// synchronisation replaces a device-to-host copy (13 us each for 8 bytes).
+constexpr int kHostSlots = 128, kHostWords = 4;
+struct HostPage {
+  std::mutex mu;
+  unsigned long long* page = nullptr;
+  bool failed = false;
+  bool used[kHostSlots] = {};
+};
+HostPage& host_page() {
+  static HostPage* h = new HostPage();
+  return *h;
+}
+
+unsigned long long* host_words_take() {
+  HostPage& h = host_page();
+  std::lock_guard<std::mutex> lk(h.mu);
+  if (!h.page && !h.failed) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kHostSlots * kHostWords * 8, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess)
+      h.page = static_cast<unsigned long long*>(p);
+    else
+      h.failed = true;
+  }
+  if (!h.page) return nullptr;
+  for (int k = 0; k < kHostSlots; k++)
+    if (!h.used[k]) {
+      h.used[k] = true;
+      return h.page + k * kHostWords;
+    }
+  return nullptr;
+}
+
+void host_words_give(unsigned long long* p) {
+  if (!p) return;
+  HostPage& h = host_page();
+  std::lock_guard<std::mutex> lk(h.mu);
+  h.used[(p - h.page) / kHostWords] = false;
+}
+
 hipError_t dev_alloc_bytes(void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 1;

@@ -139,6 +139,7 @@ struct Params {
   unsigned long long* task_ctr;
   uint32_t total_waves;
   uint32_t budget_small, budget_large;
+  uint32_t few_items;  // lists shorter than this take the small budget
 };
 
 __device__ inline uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -234,11 +235,11 @@ __device__ __attribute__((always_inline)) inline void copy_subtree(const Params<
     b = at;
   }
   const uint32_t rl = root - tb;
-  const uint32_t levels = 32u - static_cast<uint32_t>(__clz(static_cast<int>(msz)));
-  const uint32_t npos = (1u << levels) - 1u;
-  // a subtree with every position filled (all but those on the tree's
-  // right edge) needs no per-position check
-  const bool complete = msz == npos;
+  const uint32_t klast = 31u - static_cast<uint32_t>(__clz(static_cast<int>(msz)));  // depth of the last level
+  // positions of the levels that are full, of the last one when it is full too
+  const uint32_t above = (1u << klast) - 1u;
+  const uint32_t last = msz - above;  // points of the last level
+  const uint32_t npos = last > above ? msz : above;
   auto local_slot = [&](uint32_t x) {
     const uint32_t k = 31u - static_cast<uint32_t>(__clz(static_cast<int>(x + 1)));
     return ((rl + 1) << k) + x - (1u << k);
@@ -253,53 +254,56 @@ __device__ __attribute__((always_inline)) inline void copy_subtree(const Params<
       r = P.ids[tb + ls];
     }
   };
-  if (complete) {
-    // position x goes to output index x; positions past the subtree load
-    // the root again (discarded), so every load of a pass is issued
-    for (uint32_t x0 = 0; x0 < npos; x0 += kWave * U) {
-      Rec rec[U];
+  // position x goes to output index x; positions past the full levels load
+  // the root again (discarded), so every load of a pass is issued
+  for (uint32_t x0 = 0; x0 < npos; x0 += kWave * U) {
+    Rec rec[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t x = x0 + u * kWave + lane;
+      load_rec(x < npos ? local_slot(x) : rl, rec[u]);
+    }
+    uint32_t qm = qmask;
+    while (qm) {
+      const int j = __builtin_ctz(qm);
+      qm &= qm - 1;
+      Rec* out = static_cast<Rec*>(P.out) + read_lane(b, j);
+      const uint32_t fit_j = read_lane(fit, j);
+      const uint32_t lim = fit_j < npos ? fit_j : npos;
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const uint32_t x = x0 + u * kWave + lane;
-        load_rec(x < npos ? local_slot(x) : rl, rec[u]);
-      }
-      uint32_t qm = qmask;
-      while (qm) {
-        const int j = __builtin_ctz(qm);
-        qm &= qm - 1;
-        Rec* out = static_cast<Rec*>(P.out) + read_lane(b, j);
-        const uint32_t lim = read_lane(fit, j);  // at most msz = npos
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const uint32_t x = x0 + u * kWave + lane;
-          if (x < lim) out[x] = rec[u];
-        }
+        if (x < lim) out[x] = rec[u];
       }
     }
-    return;
   }
-  // subtrees on the tree's right edge: narrower passes (rare)
+  if (npos == msz) return;
+  // A last level that is not full holds its positions of least bit reversal:
+  // brev(0), ..., brev(last - 1). Where they are few they are enumerated so
+  // (a line per load); else the level is read in order and compacted.
   constexpr int UE = U >= 8 ? U / 4 : U;
-  auto exists = [&](uint32_t x) { return x < npos && subtree_size32(Mt, local_slot(x)) >= 1; };
-  uint32_t written = 0;
-  for (uint32_t x0 = 0; x0 < npos; x0 += kWave * UE) {
+  const bool sparse = last < (above + 1) / 8;
+  const uint32_t span = sparse ? last : above + 1;
+  uint32_t written = above;
+  for (uint32_t x0 = 0; x0 < span; x0 += kWave * UE) {
     Rec rec[UE];
+    bool ex[UE];
 #pragma unroll
     for (int u = 0; u < UE; u++) {
-      const uint32_t x = x0 + u * kWave + lane;
-      if (exists(x)) load_rec(local_slot(x), rec[u]);
+      const uint32_t i = x0 + u * kWave + lane;
+      const uint32_t rev = brev_bits(i, klast);
+      ex[u] = i < span && (sparse || rev < last);
+      load_rec(ex[u] ? ((rl + 1) << klast) - 1 + (sparse ? rev : i) : rl, rec[u]);
     }
 #pragma unroll
     for (int u = 0; u < UE; u++) {
-      const uint32_t x = x0 + u * kWave + lane;
-      const bool ex = exists(x);
-      const uint64_t em = __ballot(ex);
+      const uint64_t em = __ballot(ex[u]);
       const uint32_t idx = written + lanes_below(em);
 #pragma unroll
       for (int j = 0; j < G; j++) {
         if (!((qmask >> j) & 1u)) continue;
         Rec* out = static_cast<Rec*>(P.out) + read_lane(b, j);
-        if (ex && idx < read_lane(fit, j)) out[idx] = rec[u];
+        if (ex[u] && idx < read_lane(fit, j)) out[idx] = rec[u];
       }
       written += __popcll(em);
     }
@@ -375,7 +379,7 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
   unsigned long long chunk = count_in / P.total_waves;
   chunk = chunk < 1 ? 1 : (chunk > kWave ? kWave : chunk);
   const uint32_t budget =
-      last ? 0xffffffffu : (count_in < P.total_waves ? P.budget_small : P.budget_large);
+      last ? 0xffffffffu : (count_in < P.few_items ? P.budget_small : P.budget_large);
 
   // The first chunk of each wave is fixed by its index; later chunks are
   // grabbed from a shared counter, which is read first so that waves with
@@ -780,6 +784,220 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
 }
 
 // ---------------------------------------------------------------------------
+// One search on a deep tree, first launch: a workgroup of 1024 threads walks
+// from the root with a stack in LDS, up to 1024 items per step. Small
+// searches end here; a search whose stack outgrows LDS, or that is still
+// walking after kFrontSteps steps, hands its stack to the round kernels. Full
+// subtrees become copy tasks with their output position, which k_front_copy
+// writes in parts of kFrontPart positions.
+//
+// Bound by latency: a step is a node load, and the tree's depth in steps is
+// the least a search takes. The four rounds of 7168 one-wave workgroups that
+// every search took cost 31 us of launches that mostly found nothing to do,
+// and the two 8-byte copies of its results 13 us each; both kernels' results
+// now lie in pinned host memory when the stream is done. On 131,075 f32 points
+// (MI355X, call to result) a search of 2,639 results took 86 us, now 37; one of
+// 65,742, whose subtrees one wave each copied with a check per position, 306,
+// now 42.
+// ---------------------------------------------------------------------------
+constexpr int kFrontBlock = 1024;
+constexpr uint32_t kFrontStack = 7168;  // 56 KB of LDS
+constexpr uint32_t kFrontSteps = 40;
+constexpr uint32_t kFrontTasks = 16384;
+constexpr uint32_t kFrontPart = 4096;   // positions per part of a copy
+constexpr uint32_t kFrontParts = 16;    // parts that take turns on a task
+constexpr uint32_t kFrontCopyWaves = 1024;
+
+struct FrontTask {
+  uint32_t root, size;     // slot and points of the subtree
+  unsigned long long at;   // output index of its first record
+};
+
+template <typename T, typename IS, bool RET_POINT>
+__global__ __launch_bounds__(kFrontBlock) void k_front(Params<T, IS> P, FrontTask* __restrict__ tasks,
+                                                       uint32_t task_cap, unsigned long long* __restrict__ task_count,
+                                                       uint32_t nctr, unsigned long long* __restrict__ host) {
+  using Rec = typename OutRec<T, IS, RET_POINT>::type;
+  using It = Items;
+  __shared__ uint64_t stack[kFrontStack];
+  __shared__ uint32_t s_push[2], s_found, s_tasks, s_bad;
+  const uint32_t tid = threadIdx.x, lane = tid % kWave;
+  const Bounds<T> qb{P.single.min_dim1, P.single.max_dim1, P.single.min_dim2};
+  const BoundNum bn = bound_num<T, 1>(&qb);
+  const unsigned long long off = P.offsets ? P.offsets[0] : 0ull;
+  const unsigned long long room = off < P.out_total ? P.out_total - off : 0ull;
+  const unsigned long long fit = P.cap_all < room ? P.cap_all : room;
+  Rec* out = static_cast<Rec*>(P.out) + off;
+  if (tid == 0) {
+    const uint32_t kind = P.single.kind;
+    stack[0] = It::make(0, 1u, lo_open(kind), hi_open(kind), 0u);
+    s_push[0] = s_push[1] = s_found = s_tasks = s_bad = 0;
+  }
+  uint32_t sp = 1;
+  __syncthreads();
+  for (uint32_t step = 0; sp > 0 && sp <= kFrontStack - kFrontBlock && step < kFrontSteps; step++) {
+    const uint32_t n = sp < kFrontBlock ? sp : kFrontBlock;
+    const uint32_t base = sp - n;
+    const bool act = tid < n;
+    const uint64_t item = act ? stack[base + tid] : 0ull;
+    uint32_t* push = &s_push[step & 1];
+    __syncthreads();  // the items are read before children take their places
+    if (__ballot(act)) {
+      const uint32_t slot = It::slot(item);
+      const int32_t m = act && slot < P.S ? subtree_size32(P.last_M, slot) : 0;
+      const bool ok = m >= 1;
+      if (act && !ok) s_bad = 1;
+      const uint32_t il = It::l(item), ih = It::h(item);
+      uint32_t full = It::f(item);
+      const bool cand = ok && m >= P.check_min && !il && !ih && !full;
+      const T sm = P.submin[cand ? slot : 0u];
+      const Node<T, IS> nd = P.nodes[ok ? slot : 0u];
+      if (cand && qb.min2 <= sm) full = 1;
+      // a subtree reported whole: a copy task when it is small enough for
+      // one and the list has room, else walked on
+      bool bulk = ok && full && m <= P.copy_max && !il && !ih;
+      if (bulk) {
+        const uint32_t k = atomicAdd(&s_tasks, 1u);
+        if (k < task_cap) {
+          const uint32_t at = atomicAdd(&s_found, static_cast<uint32_t>(m));
+          tasks[k] = FrontTask{slot, static_cast<uint32_t>(m), at};
+        } else {
+          bulk = false;
+        }
+      }
+      StepOut so{};
+      if (ok && !bulk) so = node_step<T, 1>(nd.dim1, nd.dim2, nd.med, m, &qb, bn, 1u, il, ih);
+      const uint64_t rep = __ballot(so.rep != 0);
+      if (rep) {
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&s_found, static_cast<uint32_t>(__popcll(rep)));
+        at = __builtin_amdgcn_readfirstlane(at) + lanes_below(rep);
+        if (so.rep && at < fit) {
+          Rec rec;
+          if constexpr (RET_POINT) {
+            rec.dim1_val = nd.dim1;
+            rec.dim2_val = nd.dim2;
+            if constexpr (has_id_v<IS>) rec.id = nd.id;
+          } else {
+            rec = nd.id;
+          }
+          out[at] = rec;
+        }
+      }
+      const uint64_t lm = __ballot(so.al != 0), rm = __ballot(so.ar != 0);
+      if (lm | rm) {
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(push, static_cast<uint32_t>(__popcll(lm) + __popcll(rm)));
+        at = base + __builtin_amdgcn_readfirstlane(at) + lanes_below(lm) + lanes_below(rm);
+        if (so.al) stack[at] = It::make(2 * slot + 1, 1u, so.ll, so.hl, full);
+        if (so.ar) stack[at + (so.al ? 1u : 0u)] = It::make(2 * slot + 2, 1u, so.lr, so.hr, full);
+      }
+    }
+    if (tid == 0) s_push[(step + 1) & 1] = 0;
+    __syncthreads();
+    sp = base + *push;
+  }
+  // what is left goes to the first round's list
+  for (uint32_t i = tid; i < sp; i += kFrontBlock) P.list[0][i] = Entry{stack[i], 0};
+  if (tid < nctr) P.ctr[tid] = tid == 0 ? sp : 0;
+  if (tid == 0) {
+    const uint32_t nt = s_tasks < task_cap ? s_tasks : task_cap;
+    P.counts[0] = s_found;
+    P.err[0] = s_bad ? 2ull : 0ull;
+    P.err[1] = 0;
+    *task_count = nt;
+    __hip_atomic_store(&host[0], static_cast<unsigned long long>(s_found), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&host[1], s_bad ? 2ull : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&host[2], static_cast<unsigned long long>(sp), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// Writes the tasks' subtrees in breadth-first order: wave w of the grid takes
+// part w % kFrontParts of every (gridDim.x / kFrontParts)-th task.
+template <typename T, typename IS, bool RET_POINT>
+__global__ __launch_bounds__(kWave) void k_front_copy(Params<T, IS> P, const FrontTask* __restrict__ tasks,
+                                                      const unsigned long long* __restrict__ task_count) {
+  using Rec = typename OutRec<T, IS, RET_POINT>::type;
+  constexpr int U = sizeof(Rec) <= 4 ? 32 : (sizeof(Rec) <= 8 ? 16 : 8);
+  const uint32_t lane = threadIdx.x;
+  const uint32_t nt = static_cast<uint32_t>(__hip_atomic_load(task_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  const uint32_t part = blockIdx.x % kFrontParts;
+  const unsigned long long off = P.offsets ? P.offsets[0] : 0ull;
+  const unsigned long long room = off < P.out_total ? P.out_total - off : 0ull;
+  const unsigned long long fit = P.cap_all < room ? P.cap_all : room;
+  for (uint32_t t = blockIdx.x / kFrontParts; t < nt; t += gridDim.x / kFrontParts) {
+    const uint32_t root = __hip_atomic_load(&tasks[t].root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t msz = __hip_atomic_load(&tasks[t].size, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long at = __hip_atomic_load(&tasks[t].at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (msz == 0 || at >= fit) continue;
+    const uint32_t lim = fit - at < msz ? static_cast<uint32_t>(fit - at) : msz;
+    Rec* out = static_cast<Rec*>(P.out) + off + at;
+    // the levels that are full, and the last one where it is full too, as one
+    // breadth-first range; else the last level by itself (see copy_subtree)
+    const uint32_t klast = 31u - static_cast<uint32_t>(__clz(static_cast<int>(msz)));
+    const uint32_t above = (1u << klast) - 1u;
+    const uint32_t last = msz - above;
+    const uint32_t npos = last > above ? msz : above;
+    auto load_rec = [&](uint32_t s, Rec& r) {
+      if constexpr (RET_POINT) {
+        const Node<T, IS> nd = P.nodes[s];
+        r.dim1_val = nd.dim1;
+        r.dim2_val = nd.dim2;
+        if constexpr (has_id_v<IS>) r.id = nd.id;
+      } else {
+        r = P.ids[s];
+      }
+    };
+    auto slot_of = [&](uint32_t x) {
+      const uint32_t k = 31u - static_cast<uint32_t>(__clz(static_cast<int>(x + 1)));
+      return ((root + 1) << k) + x - (1u << k);
+    };
+    for (uint32_t p0 = part * kFrontPart; p0 < npos; p0 += kFrontParts * kFrontPart) {
+      const uint32_t p1 = p0 + kFrontPart < npos ? p0 + kFrontPart : npos;
+      for (uint32_t x0 = p0; x0 < p1; x0 += kWave * U) {
+        Rec rec[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint32_t x = x0 + u * kWave + lane;
+          load_rec(x < p1 ? slot_of(x) : root, rec[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint32_t x = x0 + u * kWave + lane;
+          if (x < p1 && x < lim) out[x] = rec[u];
+        }
+      }
+    }
+    if (npos == msz) continue;
+    constexpr int UE = U >= 16 ? U / 4 : U / 2;
+    const bool sparse = last < (above + 1) / 8;
+    const uint32_t span = sparse ? last : above + 1;
+    for (uint32_t p0 = part * kFrontPart; p0 < span; p0 += kFrontParts * kFrontPart) {
+      const uint32_t p1 = p0 + kFrontPart < span ? p0 + kFrontPart : span;
+      uint32_t written = above + (sparse ? p0 : static_cast<uint32_t>(brev_below(klast, p0, last)));
+      for (uint32_t x0 = p0; x0 < p1; x0 += kWave * UE) {
+        Rec rec[UE];
+        bool ex[UE];
+#pragma unroll
+        for (int u = 0; u < UE; u++) {
+          const uint32_t i = x0 + u * kWave + lane;
+          const uint32_t rev = brev_bits(i, klast);
+          ex[u] = i < p1 && (sparse || rev < last);
+          load_rec(ex[u] ? ((root + 1) << klast) - 1 + (sparse ? rev : i) : root, rec[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < UE; u++) {
+          const uint64_t em = __ballot(ex[u]);
+          const uint32_t idx = written + lanes_below(em);
+          if (ex[u] && idx < lim) out[idx] = rec[u];
+          written += static_cast<uint32_t>(__popcll(em));
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Grouping: queries are ordered by kind, then by their leading dim1 bound
 // (max_dim1 for left searches, min_dim1 otherwise), with two stable radix
 // sorts; group k holds sorted positions [kG, kG + G).
@@ -933,9 +1151,24 @@ TreeShape tree_shape(const SearchArgs& a) {
   return t;
 }
 
+}  // namespace
+
+// Launches of a pass: a.rounds, or by default 4 for walks of single queries
+// and 3 for group walks, 2 where the batch is small (a launch more costs what
+// its balance gains: 32 queries on 2^20 points 196 with 3, 62 us with 2; 256
+// on 2^23 184 with 3, 268 with 2).
+constexpr uint64_t kSmallWalk = 1ull << 25;  // groups x points
+int search_rounds(const SearchArgs& a) {
+  if (a.rounds > 0) return std::min(a.rounds, kMaxRounds);
+  if (group_size(a) == 1) return 4;
+  return (a.nq + kGroup - 1) / kGroup * static_cast<uint64_t>(a.n) <= kSmallWalk ? 2 : 3;
+}
+
+namespace {
+
+// The walk's kernel parameters, but for its overflow stacks and task list.
 template <typename T, typename IS, bool RP, bool W, int G>
-Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
-  Params<T, IS> P{};
+Status make_params(const SearchArgs& a, SearchScratch& sc, Params<T, IS>& P, TreeShape& sh) {
   P.nodes = static_cast<const Node<T, IS>*>(a.nodes);
   P.submin = static_cast<const T*>(a.submin);
   P.ids = static_cast<const IS*>(a.ids);
@@ -965,7 +1198,7 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
   P.out = a.out;
   P.err = sc.ctr + 2 * kMaxRounds + 2;
   P.dbg = a.debug;
-  const TreeShape sh = tree_shape(a);
+  sh = tree_shape(a);
   P.S = static_cast<uint32_t>(sh.S);
   P.tree_shift = sh.shift;
   P.ntrees = static_cast<uint32_t>(sh.ntrees);
@@ -973,14 +1206,33 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
   P.last_M = static_cast<uint32_t>(sh.last_M);
   P.nq = static_cast<uint32_t>(a.nq);
   P.ngroups = static_cast<uint32_t>((a.nq + G - 1) / G);
+  return Status{};
+}
+
+template <typename T, typename IS, bool RP, bool W, int G>
+Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
+  Params<T, IS> P{};
+  TreeShape sh{};
+  Status sp = make_params<T, IS, RP, W, G>(a, sc, P, sh);
+  if (!sp.ok()) return sp;
   const uint32_t H = sh.levels;
   // deepest stack: 128 items (a step's two batches) per level below the
   // first popped batch, plus a step's growth, in whole move blocks
   const uint32_t bound = 2 * kWave * (H + 2) + 4 * kWave;
   P.gcap = ((bound + kMoveBlock - 1) / kMoveBlock) * kMoveBlock;
-  P.budget_small = a.budget_small > 0 ? a.budget_small : 6;
-  // a write step costs more than a count step (staging, flushes, copy
-  // tasks), so the write pass hands work on after fewer steps
+  const int R = search_rounds(a);
+  // Step budgets. Group walks spread their work in rounds of 8 steps per
+  // batch (9 when there is one such round), and run every stack to empty in
+  // the last: a batch of one item needs seven steps to fill a wave's lanes, so
+  // with 6 a list of 10^4 items still held whole subtrees, and the 384 steps
+  // that followed at 8192 items and more ran on a few waves only. MI355X, count
+  // / write passes, 4 rounds of 6 and 384 -> these: 256 queries on 700,001
+  // points 450/464 -> 75/96 us, 700 on 5,000,011 271/768 -> 230/700, 2048 on
+  // 2^26 4.23/8.12 -> 3.48/7.98 ms; budgets of 7, 10 and more lose on most
+  // sizes. One query's walk (no group) keeps its own. A write step costs more
+  // than a count step (staging, flushes, copy tasks), so long lists hand work
+  // on after fewer steps there.
+  P.budget_small = a.budget_small > 0 ? a.budget_small : (G == 1 ? 6 : (R <= 2 ? 9 : 8));
   P.budget_large = a.budget_large > 0 ? a.budget_large : (W ? 192 : 384);
   auto kern = k_search_round<T, IS, RP, W, G>;
   int dev = 0;
@@ -995,6 +1247,7 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
   hipError_t e = hipSuccess;
   const uint32_t grid = static_cast<uint32_t>(cus * occ);
   P.total_waves = grid;
+  P.few_items = G == 1 ? grid : 4 * grid;
   const size_t gbytes = static_cast<size_t>(grid) * P.gcap * sizeof(Items::type);
   if (sc.gstack_bytes < gbytes) {
     if (sc.pinned) return Status{1, kPinnedScratchMsg};
@@ -1021,7 +1274,6 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
     P.task_cap = want;
     P.task_ctr = sc.ctr + 2 * kMaxRounds + 3;
   }
-  const int R = std::max(1, std::min(a.rounds, kMaxRounds));
   for (int r = 0; r < R; r++) {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kWave), 0, s, P, static_cast<uint32_t>(r),
                        static_cast<uint32_t>(r == R - 1));
@@ -1159,7 +1411,8 @@ Status scratch_reserve(SearchScratch& sc, size_t nq, size_t roots, hipStream_t) 
 
 void scratch_release(SearchScratch& sc, bool idle) {
   for (void* p : {sc.list[0], sc.list[1], static_cast<void*>(sc.ctr), static_cast<void*>(sc.cursor),
-                  static_cast<void*>(sc.groups), sc.gkeys, sc.gtmp, sc.gstack, sc.tasks, sc.fseg})
+                  static_cast<void*>(sc.groups), sc.gkeys, sc.gtmp, sc.gstack, sc.tasks, sc.fseg,
+                  sc.front})
     (void)(idle ? dev_free_idle(p) : dev_free(p));
   sc = SearchScratch{};
 }
@@ -1214,6 +1467,42 @@ Status run_search(const SearchArgs& a_in, SearchScratch& sc, hipStream_t s) {
       };
       if (G == 1) return go(std::integral_constant<int, 1>{});
       return go(std::integral_constant<int, kGroup>{});
+    });
+  });
+}
+
+template <typename T, typename IS, bool RP>
+Status front_typed(const SearchArgs& a, SearchScratch& sc, bool rounds, unsigned long long* host, hipStream_t s) {
+  if (rounds) return launch_rounds<T, IS, RP, true, 1>(a, sc, s);
+  Params<T, IS> P{};
+  TreeShape sh{};
+  Status st = make_params<T, IS, RP, true, 1>(a, sc, P, sh);
+  if (!st.ok()) return st;
+  const uint32_t cap = a.copy_tasks > 0 ? static_cast<uint32_t>(std::min<size_t>(a.copy_tasks, kFrontTasks)) : kFrontTasks;
+  auto* tasks = static_cast<FrontTask*>(sc.front);
+  auto* count = reinterpret_cast<unsigned long long*>(tasks + kFrontTasks);
+  k_front<T, IS, RP><<<1, kFrontBlock, 0, s>>>(P, tasks, cap, count, 2 * kMaxRounds + 2, host);
+  if (P.copy_max > 0) k_front_copy<T, IS, RP><<<kFrontCopyWaves, kWave, 0, s>>>(P, tasks, count);
+  return hip_status(hipGetLastError(), "Error in launching search kernel");
+}
+
+// One search of a deep tree (a.single_query): its first launches, whose
+// results, error bits and leftover walk items lie in host[0..2] once the
+// stream is done, or (rounds) the walk of the leftover items.
+Status search_front(const SearchArgs& a, SearchScratch& sc, bool rounds, unsigned long long* host, hipStream_t s) {
+  Status st = scratch_reserve(sc, 1, 0, s);
+  if (!st.ok()) return st;
+  if (!sc.front) {
+    st = hip_status(dev_alloc(&sc.front, (kFrontTasks + 1) * sizeof(FrontTask)), "Error in allocating search buffers");
+    if (!st.ok()) return st;
+  }
+  return with_t(a.dtype, [&](auto t) -> Status {
+    using T = decltype(t);
+    return with_is(a.id_dtype, [&](auto i) -> Status {
+      using IS = decltype(i);
+      if (a.ret_point) return front_typed<T, IS, true>(a, sc, rounds, host, s);
+      if constexpr (has_id_v<IS>) return front_typed<T, IS, false>(a, sc, rounds, host, s);
+      return Status{1, "Error: IDs requested from a tree built without IDs"};
     });
   });
 }

@@ -95,21 +95,20 @@ __global__ void k_keys_single(const Point<T, I>* __restrict__ pts, uint32_t n, K
   vals[j] = r2 ? r2[i] : i;
 }
 
-// Two-pass keys (when dim or id is 8 bytes): pass A orders by id.
-template <typename T, typename I, typename K, bool DESC>
+// Keys of points whose IDs are not in index order: by ID first, then by dim
+// over the points in that order (`perm`; backwards for a descending order, so
+// that equal dims come by descending (id, index)).
+template <typename T, typename I, typename K>
 __global__ void k_keys_id(const Point<T, I>* __restrict__ pts, uint32_t n, K* __restrict__ keys,
                           uint32_t* __restrict__ vals, int* __restrict__ nan_flag) {
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  const uint32_t i = DESC ? n - 1 - j : j;
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
   const I id = pts[i].id;
   if (is_nan(id)) *nan_flag = 1;
-  const K k = static_cast<K>(ord_key(id));
-  keys[j] = DESC ? static_cast<K>(~k) : k;
-  vals[j] = i;
+  keys[i] = static_cast<K>(ord_key(id));
+  vals[i] = i;
 }
 
-// Pass B: orders by dim, visiting points in pass-A order.
 template <typename T, typename I, typename K, bool DIM2, bool DESC>
 __global__ void k_keys_dim_perm(const Point<T, I>* __restrict__ pts, uint32_t n,
                                 const uint32_t* __restrict__ perm, K* __restrict__ keys,
@@ -117,7 +116,7 @@ __global__ void k_keys_dim_perm(const Point<T, I>* __restrict__ pts, uint32_t n,
                                 int* __restrict__ nan_flag) {
   const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
-  const uint32_t i = perm[j];
+  const uint32_t i = perm[DESC ? n - 1 - j : j];
   const T d = DIM2 ? pts[i].dim2_val : pts[i].dim1_val;
   if (is_nan(d)) *nan_flag = 1;
   const K k = static_cast<K>(ord_key(d));
@@ -1303,7 +1302,8 @@ Status build_typed(int dtype, int id_dtype, const void* pts_v, size_t n64, Build
       PST_TRY(sortK(key0, key1, v0, v1), "Error in sorting by dimension 2");
     } else {
       if constexpr (kHasId) {
-        k_keys_id<T, I, K, true><<<G, B, 0, s>>>(pts, n, key0, v0, nan_flag);
+        // v2: the points in (id, index) order, read backwards for key2
+        k_keys_id<T, I, K><<<G, B, 0, s>>>(pts, n, key0, v0, nan_flag);
         PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by ID");
         k_keys_dim_perm<T, I, K, true, true><<<G, B, 0, s>>>(pts, n, v2, key0, v0, nullptr, nan_flag);
         PST_TRY(sortK(key0, key1, v0, v1), "Error in sorting by dimension 2");
@@ -1322,8 +1322,6 @@ Status build_typed(int dtype, int id_dtype, const void* pts_v, size_t n64, Build
       PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by dimension 1");
     } else {
       if constexpr (kHasId) {
-        k_keys_id<T, I, K, false><<<G, B, 0, s>>>(pts, n, key0, v0, nan_flag);
-        PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by ID");
         k_keys_dim_perm<T, I, K, false, false><<<G, B, 0, s>>>(pts, n, v2, key0, v0, r2, nan_flag);
         PST_TRY(sortK(key0, key1, v0, v2), "Error in sorting by dimension 1");
       }

@@ -32,7 +32,8 @@
 // counts before it waits: every wait ends. The wait is still bounded; a
 // tile that exceeds the bound sets the caller's failure word and goes on.
 // Passes alternate between the output and a scratch buffer, ending in the
-// output; the inputs are not modified.
+// output; the inputs are not modified. A pass in which all keys share the
+// digit is left out (64-bit IDs and integers use few of their bytes).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -48,15 +49,26 @@ constexpr int kDigitBits = 8;
 constexpr int kDigits = 1 << kDigitBits;
 constexpr int kPassBlock = 512;
 constexpr int kPassWaves = kPassBlock / kWave;            // 8
-constexpr int kPassPer = 16;                              // keys per lane
-constexpr uint32_t kWaveKeys = kWave * kPassPer;          // 1024
-constexpr uint32_t kSortTile = kPassBlock * kPassPer;     // 8192
+// Keys per lane: tiles of 8192 keys, of 4096 where those are few (a pass then
+// waits for its tile's rounds, and half the rounds run on twice the CUs).
+// Building trees whose sorts take 8 and 4 instead of 16 keys per lane, MI355X:
+// 20,000 f64 points 474, 442, 415 us; 300,007 615, 601, 625; 10^6 820, 828, 943.
+constexpr int kPassPerFull = 16, kPassPerFew = 8;
+constexpr uint32_t kFewKeys = 1u << 19;
+constexpr uint32_t tile_keys(int per) { return kPassBlock * static_cast<uint32_t>(per); }
+inline uint32_t tiles_of(size_t n) {
+  const uint32_t t = tile_keys(n <= kFewKeys ? kPassPerFew : kPassPerFull);
+  return static_cast<uint32_t>((n + t - 1) / t);
+}
 constexpr int kHistBlock = 512;
 constexpr int kHistPer = 16;
 constexpr uint32_t kHistChunk = kHistBlock * kHistPer;
 constexpr unsigned kHistMaxBlocks = 1024;
 constexpr uint32_t kLookbackSpins = 1u << 24;             // about a second
-constexpr uint32_t kLookAhead = 4;                        // look-back words read at once
+// Look-back words read at once. Where all tiles run at once none finds a
+// prefix before the first tiles have finished, and each adds up every tile
+// before it: such a sort reads more words per step.
+constexpr uint32_t kLookAhead = 4, kLookAheadFew = 16;
 
 template <typename K>
 __device__ inline uint32_t digit_of(K k, uint32_t shift) {
@@ -129,26 +141,52 @@ __global__ __launch_bounds__(kHistBlock) void k_sort_hist(const K* __restrict__ 
   }
 }
 
-// Exclusive scan of each of `passes` rows of 256 digit totals, in place (one block).
-__global__ __launch_bounds__(kDigits) void k_digit_starts(uint32_t* __restrict__ hist, uint32_t passes) {
-  __shared__ uint32_t s[kDigits];
-  for (uint32_t p = 0; p < passes; p++) {
-    const uint32_t v = hist[p * kDigits + threadIdx.x];
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (uint32_t off = 1; off < kDigits; off <<= 1) {
-      const uint32_t o = threadIdx.x >= off ? s[threadIdx.x - off] : 0u;
-      __syncthreads();
-      s[threadIdx.x] += o;
-      __syncthreads();
+// Exclusive scan of each of `passes` rows of 256 digit totals, in place (one
+// workgroup, four rows at a time), and the passes' order: a pass whose keys
+// all share one digit would only copy and is left out. order[p]: passes that
+// run before p, or kNoPass; order[kMaxPasses]: passes that run. With
+// `keep_first` pass 0 always runs; some pass always does.
+constexpr uint32_t kMaxPasses = 8;
+constexpr uint32_t kNoPass = ~0u;
+constexpr int kStartsBlock = 4 * kDigits;
+__global__ __launch_bounds__(kStartsBlock) void k_digit_starts(uint32_t* __restrict__ hist, uint32_t passes, uint32_t n,
+                                                               uint32_t keep_first, uint32_t* __restrict__ order) {
+  __shared__ uint32_t wsum[kStartsBlock / kWave];
+  __shared__ uint32_t one[kMaxPasses];
+  const uint32_t d = threadIdx.x % kDigits, lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  if (threadIdx.x < kMaxPasses) one[threadIdx.x] = 0;
+  __syncthreads();
+  for (uint32_t p0 = 0; p0 < passes; p0 += kStartsBlock / kDigits) {
+    const uint32_t p = p0 + threadIdx.x / kDigits;
+    const uint32_t v = p < passes ? hist[p * kDigits + d] : 0u;
+    uint32_t inc = v;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint32_t o = __shfl_up(inc, off, kWave);
+      if (static_cast<int>(lane) >= off) inc += o;
     }
-    hist[p * kDigits + threadIdx.x] = s[threadIdx.x] - v;
+    if (lane == kWave - 1) wsum[wave] = inc;
+    if (p < passes && v == n) one[p] = 1;
     __syncthreads();
+    uint32_t before = 0;
+    for (uint32_t w = wave & ~3u; w < wave; w++) before += wsum[w];
+    if (p < passes) hist[p * kDigits + d] = before + inc - v;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    uint32_t run = 0;
+    for (uint32_t p = 0; p < passes; p++) {
+      const bool skip = one[p] && !(keep_first && p == 0) && !(p + 1 == passes && run == 0);
+      order[p] = skip ? kNoPass : run;
+      run += skip ? 0u : 1u;
+    }
+    order[kMaxPasses] = run;
   }
 }
 
-template <typename K, typename V>
+template <typename K, typename V, int PER>
 struct PassLds {
+  static constexpr uint32_t kSortTile = tile_keys(PER);
   union {
     unsigned long long peer[kPassWaves][kDigits];  // while ranking: per-wave lane masks of a round's digits
     K sbuf[kSortTile];                             // then keys,
@@ -199,11 +237,12 @@ struct PointSrc {
 
 // One tile of a digit pass. FULL: the tile holds kSortTile keys, so no
 // element needs a bounds check (and each lane's loads share one address).
-template <typename K, typename V, bool FULL, typename Src>
-__device__ __forceinline__ void sort_tile(PassLds<K, V>& L, Src src,
+template <typename K, typename V, bool FULL, uint32_t LOOK, int kPassPer, typename Src>
+__device__ __forceinline__ void sort_tile(PassLds<K, V, kPassPer>& L, Src src,
                                           K* __restrict__ kout, V* __restrict__ vout, uint32_t tile,
                                           uint32_t valid, uint32_t pass, unsigned long long* __restrict__ status,
                                           const uint32_t* __restrict__ gstart, int* __restrict__ fail) {
+  constexpr uint32_t kSortTile = tile_keys(kPassPer), kWaveKeys = kWave * kPassPer;
   const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   const uint32_t shift = pass * kDigitBits;
   const uint64_t base = static_cast<uint64_t>(tile) * kSortTile;
@@ -301,18 +340,18 @@ __device__ __forceinline__ void sort_tile(PassLds<K, V>& L, Src src,
       uint32_t spins = 0;
       bool done = false;
       while (!done) {
-        // kLookAhead words at a time (independent loads), then taken in
+        // LOOK words at a time (independent loads), then taken in
         // order: a prefix ends the walk, a count is added, a word not yet
         // published stops this step
-        unsigned long long w[kLookAhead];
+        unsigned long long w[LOOK];
 #pragma unroll
-        for (uint32_t i = 0; i < kLookAhead; i++)
+        for (uint32_t i = 0; i < LOOK; i++)
           w[i] = i <= j ? __hip_atomic_load(&status[static_cast<size_t>(j - i) * kDigits + tid], __ATOMIC_RELAXED,
                                             __HIP_MEMORY_SCOPE_AGENT)
                         : 0ull;
         bool stalled = false;
 #pragma unroll
-        for (uint32_t i = 0; i < kLookAhead; i++) {
+        for (uint32_t i = 0; i < LOOK; i++) {
           if (done || stalled) continue;
           const uint32_t tag = static_cast<uint32_t>(w[i] >> 32);
           if (tag == tp) {
@@ -366,15 +405,28 @@ __device__ __forceinline__ void sort_tile(PassLds<K, V>& L, Src src,
 // per-digit counts of earlier tiles, then a stable scatter.
 // Six waves per SIMD: three workgroups per CU for 32-bit keys and values (LDS
 // bounds 64-bit keys or values to two, four waves per SIMD).
-template <typename K, typename V, typename Src>
+// The first pass that runs reads `first`; the passes alternate between the
+// scratch and the output so that the last one writes the output.
+template <typename K, typename V, uint32_t LOOK, int PER, typename Src>
 __global__ __launch_bounds__(kPassBlock)
-__attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 ? 4 : 6))) void k_sort_pass(Src src, K* __restrict__ kout,
-                                                          V* __restrict__ vout,
-                                                          uint32_t n, uint32_t pass, uint32_t* __restrict__ tile_ctr,
-                                                          unsigned long long* __restrict__ status,
-                                                          const uint32_t* __restrict__ gstart,
-                                                          int* __restrict__ fail) {
-  __shared__ PassLds<K, V> L;
+__attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 ? 4 : 6))) void k_sort_pass(
+    Src first, K* __restrict__ kout, V* __restrict__ vout, K* __restrict__ kx, V* __restrict__ vx, uint32_t n,
+    uint32_t pass, const uint32_t* __restrict__ order, uint32_t* __restrict__ tile_ctr,
+    unsigned long long* __restrict__ status, const uint32_t* __restrict__ gstart, int* __restrict__ fail) {
+  const uint32_t c = __builtin_amdgcn_readfirstlane(
+      __hip_atomic_load(&order[pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  if (c == kNoPass) return;
+  const uint32_t runs = __builtin_amdgcn_readfirstlane(
+      __hip_atomic_load(&order[kMaxPasses], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  const bool to_out = ((runs - c) & 1u) != 0;
+  K* kdst = to_out ? kout : kx;
+  V* vdst = to_out ? vout : vx;
+  Src src = first;
+  if constexpr (std::is_same<Src, ArraySrc<K, V>>::value) {
+    if (c > 0) src = Src{to_out ? kx : kout, to_out ? vx : vout};
+  }
+  constexpr uint32_t kSortTile = tile_keys(PER);
+  __shared__ PassLds<K, V, PER> L;
   const uint32_t tid = threadIdx.x;
   if (tid == 0) L.tile = atomicAdd(&tile_ctr[pass], 1u);
   for (uint32_t i = tid; i < kPassWaves * kDigits; i += kPassBlock) {
@@ -389,10 +441,25 @@ __attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 ? 4 : 6))) void k_sort_pass(Sr
   const uint32_t rem = n - tile * kSortTile;
   const uint32_t valid = rem < kSortTile ? rem : kSortTile;
   if (valid == kSortTile)
-    sort_tile<K, V, true>(L, src, kout, vout, tile, valid, pass, status, gstart, fail);
+    sort_tile<K, V, true, LOOK, PER>(L, src, kdst, vdst, tile, valid, pass, status, gstart, fail);
   else
-    sort_tile<K, V, false>(L, src, kout, vout, tile, valid, pass, status, gstart, fail);
+    sort_tile<K, V, false, LOOK, PER>(L, src, kdst, vdst, tile, valid, pass, status, gstart, fail);
 }
+
+// One pass over n pairs.
+template <typename K, typename V, typename Src>
+void launch_pass(Src first, K* kout, V* vout, K* kx, V* vx, uint32_t n, uint32_t pass, const uint32_t* order,
+                 uint32_t* ctr, unsigned long long* status, const uint32_t* hist, int* fail, hipStream_t s) {
+  const dim3 grid(tiles_of(n)), block(kPassBlock);
+  if (n <= kFewKeys)
+    hipLaunchKernelGGL((k_sort_pass<K, V, kLookAheadFew, kPassPerFew, Src>), grid, block, 0, s, first, kout, vout, kx, vx,
+                       n, pass, order, ctr, status, hist + pass * kDigits, fail);
+  else
+    hipLaunchKernelGGL((k_sort_pass<K, V, kLookAhead, kPassPerFull, Src>), grid, block, 0, s, first, kout, vout, kx, vx,
+                       n, pass, order, ctr, status, hist + pass * kDigits, fail);
+}
+
+constexpr uint32_t kOrderWord = 32;  // of the 64 counter words: tile counters, a failure word, then the order
 
 inline size_t align256(size_t b) { return (b + 255) & ~size_t{255}; }
 
@@ -400,7 +467,7 @@ template <typename K>
 hipError_t radix_sort(void* tmp, size_t& tmp_bytes, const K* kin, K* kout, const uint32_t* vin, uint32_t* vout,
                       size_t n, hipStream_t s, int* fail) {
   constexpr uint32_t passes = sizeof(K) * 8 / kDigitBits;
-  const size_t ntiles = (n + kSortTile - 1) / kSortTile;
+  const size_t ntiles = tiles_of(n);
   const size_t need_keys = align256(n * sizeof(K));
   const size_t need_vals = align256(n * 4);
   // cleared once per sort: the status words, the tile counters and the
@@ -432,21 +499,10 @@ hipError_t radix_sort(void* tmp, size_t& tmp_bytes, const K* kin, K* kout, const
   const unsigned hblocks =
       static_cast<unsigned>(std::min<size_t>((n + kHistChunk - 1) / kHistChunk, kHistMaxBlocks));
   hipLaunchKernelGGL((k_sort_hist<K>), dim3(hblocks), dim3(kHistBlock), 0, s, kin, n32, hist);
-  hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kDigits), 0, s, hist, passes);
-  // passes alternate so that the last one writes kout: an even number of
-  // passes starts into the scratch, an odd number into kout
-  const K* ksrc = kin;
-  const uint32_t* vsrc = vin;
-  for (uint32_t pass = 0; pass < passes; pass++) {
-    const bool to_out = ((passes - pass) % 2) == 1;
-    K* kdst = to_out ? kout : kt;
-    uint32_t* vdst = to_out ? vout : vt;
-    hipLaunchKernelGGL((k_sort_pass<K, uint32_t, ArraySrc<K, uint32_t>>), dim3(static_cast<unsigned>(ntiles)),
-                       dim3(kPassBlock), 0, s, ArraySrc<K, uint32_t>{ksrc, vsrc}, kdst, vdst, n32, pass, ctr, status,
-                       hist + pass * kDigits, fail);
-    ksrc = kdst;
-    vsrc = vdst;
-  }
+  uint32_t* order = ctr + kOrderWord;
+  hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kStartsBlock), 0, s, hist, passes, n32, 0u, order);
+  for (uint32_t pass = 0; pass < passes; pass++)
+    launch_pass(ArraySrc<K, uint32_t>{kin, vin}, kout, vout, kt, vt, n32, pass, order, ctr, status, hist, fail, s);
   return hipGetLastError();
 }
 
@@ -525,7 +581,7 @@ struct PointSortTmp {
   size_t words;  // from status on, cleared once per sort
 };
 PointSortTmp point_sort_tmp(void* tmp, size_t n) {
-  const size_t ntiles = (n + kSortTile - 1) / kSortTile;
+  const size_t ntiles = tiles_of(n);
   const size_t status_bytes = std::max<size_t>(ntiles, 1) * kDigits * 8;
   PointSortTmp t{};
   auto* p = static_cast<unsigned char*>(tmp);
@@ -580,26 +636,19 @@ hipError_t point_sort_passes(int dtype, int id_dtype, const void* pts_d, size_t 
                              uint64_t* val_x, uint32_t* key_out, uint64_t* val_out, int* fail, hipStream_t s) {
   const PointSortTmp t = point_sort_tmp(tmp, n);
   const uint32_t n32 = static_cast<uint32_t>(n);
-  const dim3 grid(static_cast<unsigned>((n + kSortTile - 1) / kSortTile)), block(kPassBlock);
-  hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kDigits), 0, s, t.hist, kPointPasses);
-  hipError_t e = with_point(dtype, id_dtype, [&](auto tv, auto iv) {
+  uint32_t* order = t.ctr + kOrderWord;
+  hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kStartsBlock), 0, s, t.hist, kPointPasses, n32, 1u, order);
+  const hipError_t e = with_point(dtype, id_dtype, [&](auto tv, auto iv) {
     using Src = PointSrc<decltype(tv), decltype(iv)>;
     using Pt = Point<decltype(tv), decltype(iv)>;
-    hipLaunchKernelGGL((k_sort_pass<uint32_t, uint64_t, Src>), grid, block, 0, s, Src{static_cast<const Pt*>(pts_d), 0u},
-                       key_x, val_x, n32, 0u, t.ctr, t.status, t.hist, fail);
+    launch_pass(Src{static_cast<const Pt*>(pts_d), 0u}, key_out, val_out, key_x, val_x, n32, 0u, order, t.ctr, t.status,
+                t.hist, fail, s);
     return hipGetLastError();
   });
-  using Src = ArraySrc<uint32_t, uint64_t>;
-  const uint32_t* ks = key_x;
-  const uint64_t* vs = val_x;
-  for (uint32_t pass = 1; pass < kPointPasses && e == hipSuccess; pass++) {
-    const bool out = pass % 2 == 1;  // the last pass (3) writes the outputs
-    hipLaunchKernelGGL((k_sort_pass<uint32_t, uint64_t, Src>), grid, block, 0, s, Src{ks, vs}, out ? key_out : key_x,
-                       out ? val_out : val_x, n32, pass, t.ctr, t.status, t.hist + pass * kDigits, fail);
-    ks = out ? key_out : key_x;
-    vs = out ? val_out : val_x;
-    e = hipGetLastError();
-  }
+  for (uint32_t pass = 1; pass < kPointPasses && e == hipSuccess; pass++)
+    launch_pass(ArraySrc<uint32_t, uint64_t>{nullptr, nullptr}, key_out, val_out, key_x, val_x, n32, pass, order, t.ctr,
+                t.status, t.hist, fail, s);
+  if (e == hipSuccess) return hipGetLastError();
   return e;
 }
 

@@ -195,8 +195,10 @@ Status run_search(const SearchArgs& a, SearchScratch& sc, hipStream_t stream);
 int search_rounds(const SearchArgs& a);
 Status search_front(const SearchArgs& a, SearchScratch& sc, bool rounds, unsigned long long* host, hipStream_t s);
 unsigned long long* search_error_flag(SearchScratch& sc);
-// offsets[q] = sum of in[0..q), offsets[n] = total (one workgroup).
-Status exclusive_scan(const unsigned long long* in, unsigned long long* offsets, size_t n, hipStream_t s);
+// offsets[q] = sum of in[0..q), offsets[n] = total (one workgroup); for
+// `rows` arrays `stride` (more than n) apart.
+Status exclusive_scan(const unsigned long long* in, unsigned long long* offsets, size_t n, hipStream_t s,
+                      unsigned rows = 1, size_t stride = 0);
 
 // ---- forest batches with the trees held stationary (pst_forest.hip) ----
 // Batches of at most this many queries on a forest of trees of at most 511

@@ -241,6 +241,217 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_scatter(const uint32_t* __restr
   }
 }
 
+// ---------------------------------------------------------------------------
+// Two levels at a time: level t's points go to level t + 1 (a child's run) and
+// to level t + 2 (a grandchild's) from one read of their keys, IDs and slots;
+// level t + 1 needs no slots of its own. A point's class is its two turns
+// below level t (first turn high). In a run, the first point is the root, and
+// among the points of one side the child's root comes first, so with the
+// counts of the four classes before the point and before its run
+//   level t + 2: run start + classes before its own + rank in its class,
+//   level t + 1: run start + 1 + ranks in its side's two classes (0 for the
+//                child's root itself).
+// The runs before run j have dropped j roots by level t + 1 and 3j by level
+// t + 2, so the starts there follow from the run's start at level t; that, and
+// the class counts before it, are carried along the tile from root to root
+// (closed form for the run that reaches into the tile from the left). For
+// levels whose grandchild runs all exist or are empty: M >> (t + 2) >= 1.
+//
+// Bound by HBM: 36 B per point and two levels (56 with a pass per level). The
+// moves hold keys and IDs in registers between the two levels, so that one
+// LDS buffer of destinations serves both (with two, 12 waves per CU: 0.61
+// ms). MI355X, 2^26 f32/u32 points: 0.52 ms per pair of levels after 0.08 ms of
+// counts (4.2 TB/s), where single steps took 0.65 and 0.15.
+// ---------------------------------------------------------------------------
+__device__ inline uint32_t lv_class(uint32_t s, uint32_t t) {  // 4: the root or a child's root
+  const uint32_t d = depth_of(s);
+  return d < t + 2 ? 4u : ((s + 1u) >> (d - t - 2u)) & 3u;
+}
+// Class counts: classes 0 and 1 in the low and high half of a, 2 and 3 of b.
+struct Counts4 {
+  unsigned long long a, b;
+  __device__ void add(uint32_t c) {
+    const unsigned long long one = 1ull << (32 * (c & 1u));
+    a += c < 2 ? one : 0ull;
+    b += (c >> 1) == 1 ? one : 0ull;
+  }
+  __device__ uint32_t get(uint32_t c) const {
+    const unsigned long long w = c < 2 ? a : b;
+    return static_cast<uint32_t>((c & 1u) ? w >> 32 : w);
+  }
+};
+
+// agg[tile], agg[stride + tile]: the tile's class counts.
+__global__ __launch_bounds__(kLvBlock) void k_lv_tile_counts2(const uint32_t* __restrict__ slots, uint32_t nt,
+                                                              uint32_t t, unsigned long long* __restrict__ agg,
+                                                              uint32_t stride) {
+  __shared__ Counts4 wsum[kLvBlock / kWave];
+  const uint32_t base = blockIdx.x * kLvTile + threadIdx.x * kLvPer;
+  uint32_t sl[kLvPer];
+  load_run(slots, base, nt, sl);
+  Counts4 c{0, 0};
+#pragma unroll
+  for (int u = 0; u < kLvPer; u++)
+    if (base + u < nt) c.add(lv_class(sl[u], t));
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    c.a += __shfl_xor(c.a, o, kWave);
+    c.b += __shfl_xor(c.b, o, kWave);
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) wsum[threadIdx.x / kWave] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    Counts4 s{0, 0};
+    for (int w = 0; w < kLvBlock / kWave; w++) s.a += wsum[w].a, s.b += wsum[w].b;
+    agg[blockIdx.x] = s.a;
+    agg[stride + blockIdx.x] = s.b;
+  }
+}
+
+template <typename K, typename IS>
+__global__ __launch_bounds__(kLvBlock) void k_lv_scatter2(const uint32_t* __restrict__ slots_in,
+                                                          uint32_t* __restrict__ slots_out,
+                                                          const K* __restrict__ key_in, K* __restrict__ key1,
+                                                          K* __restrict__ key2, const IS* __restrict__ id_in,
+                                                          IS* __restrict__ id1, IS* __restrict__ id2,
+                                                          const unsigned long long* __restrict__ tile_pre,
+                                                          uint32_t stride, uint32_t nt, uint32_t t, uint64_t M) {
+  constexpr int kWaves = kLvBlock / kWave;
+  __shared__ Counts4 wsum[kWaves];
+  __shared__ uint64_t wroots[kWaves];          // per wave: threads whose points hold a root
+  __shared__ Counts4 s_at[kLvBlock + 1];       // the thread's last root: class counts before it,
+  __shared__ uint32_t s_pos[kLvBlock + 1];     // its position (entry kLvBlock: the run that enters the tile)
+  __shared__ uint32_t s_dst[kLvBlock * kDstPad];  // level t + 1, then t + 2
+  const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const uint32_t tile = blockIdx.x * kLvTile;
+  const uint32_t base = tile + tid * kLvPer;
+  uint32_t s[kLvPer];
+  load_run(slots_in, base, nt, s);
+  Counts4 loc{0, 0};
+#pragma unroll
+  for (int u = 0; u < kLvPer; u++)
+    if (base + u < nt) loc.add(lv_class(s[u], t));
+  Counts4 inc = loc;
+  for (int o = 1; o < kWave; o <<= 1) {
+    const unsigned long long ya = __shfl_up(inc.a, o, kWave), yb = __shfl_up(inc.b, o, kWave);
+    if (static_cast<int>(lane) >= o) inc.a += ya, inc.b += yb;
+  }
+  if (lane == kWave - 1) wsum[wave] = inc;
+  if (tid == 0) {  // the run that holds the tile's first point
+    const uint32_t d = depth_of(s[0]);
+    const uint32_t j = ((s[0] + 1u) >> (d - t)) - (1u << t);
+    s_pos[kLvBlock] = static_cast<uint32_t>(level_start(M, t, j));
+    const uint64_t size = (M >> (t + 2)) - 1;
+    const uint64_t r2 = M & ((4ull << t) - 1ull);
+    uint32_t c[4];
+    for (uint32_t k = 0; k < 4; k++) {
+      // points of level-(t+2) positions 4j' + k, j' < j
+      const uint64_t off = static_cast<uint64_t>(brev_bits(k, 2)) << t;
+      c[k] = static_cast<uint32_t>(j * size + brev_below(t, j, r2 > off ? r2 - off : 0));
+    }
+    s_at[kLvBlock] = Counts4{c[0] | (static_cast<unsigned long long>(c[1]) << 32),
+                             c[2] | (static_cast<unsigned long long>(c[3]) << 32)};
+  }
+  __syncthreads();
+  Counts4 run{tile_pre[blockIdx.x] + inc.a - loc.a, tile_pre[stride + blockIdx.x] + inc.b - loc.b};
+  for (uint32_t w = 0; w < wave; w++) run.a += wsum[w].a, run.b += wsum[w].b;
+  // the thread's last root
+  {
+    Counts4 c = run;
+    bool has = false;
+#pragma unroll
+    for (int u = 0; u < kLvPer; u++) {
+      if (base + u < nt) {
+        if (depth_of(s[u]) == t) {
+          has = true;
+          s_at[tid] = c;
+          s_pos[tid] = base + u;
+        }
+        c.add(lv_class(s[u], t));
+      }
+    }
+    const uint64_t b = __ballot(has);
+    if (lane == 0) wroots[wave] = b;
+  }
+  __syncthreads();
+  // the run the thread's first point lies in: the last root before it
+  uint32_t from = kLvBlock;
+  {
+    uint64_t b = wroots[wave] & ((1ull << lane) - 1ull);
+    uint32_t w = wave;
+    while (!b && w > 0) b = wroots[--w];
+    if (b) from = w * kWave + 63u - static_cast<uint32_t>(__clzll(static_cast<long long>(b)));
+  }
+  Counts4 at = s_at[from];
+  uint32_t pos = s_pos[from];
+  uint32_t cj = ~0u, s1 = 0, s2 = 0, left1 = 0, g[3] = {0, 0, 0};
+  uint32_t dst2[kLvPer];
+#pragma unroll
+  for (int u = 0; u < kLvPer; u++) {
+    uint32_t d1 = ~0u, d2 = ~0u;
+    if (base + u < nt) {
+      const uint32_t d = depth_of(s[u]);
+      const uint32_t j = ((s[u] + 1u) >> (d - t)) - (1u << t);
+      if (d == t) {
+        at = run;
+        pos = base + u;
+      }
+      if (j != cj) {
+        cj = j;
+        s1 = pos - j;
+        s2 = pos - 3 * j;
+        left1 = static_cast<uint32_t>(level_size(M, t + 1, 2 * j));
+        for (uint32_t k = 0; k < 3; k++) g[k] = static_cast<uint32_t>(level_size(M, t + 2, 4 * j + k));
+      }
+      if (d == t + 1) {
+        d1 = s1 + (((s[u] + 1u) & 1u) ? left1 : 0u);
+      } else if (d > t + 1) {
+        const uint32_t c = ((s[u] + 1u) >> (d - t - 2u)) & 3u, side = c >> 1;
+        const uint32_t r0 = run.get(2 * side) - at.get(2 * side), r1 = run.get(2 * side + 1) - at.get(2 * side + 1);
+        d1 = s1 + (side ? left1 : 0u) + 1u + r0 + r1;
+        d2 = s2 + (c > 0 ? g[0] : 0u) + (c > 1 ? g[1] : 0u) + (c > 2 ? g[2] : 0u) + ((c & 1u) ? r1 : r0);
+        run.add(c);
+      }
+    }
+    s_dst[tid * kDstPad + u] = d1;
+    dst2[u] = d2;
+  }
+  // the moves, a thread per point, 256 consecutive points per pass
+  K k[kLvPer];
+  IS id[kLvPer];
+#pragma unroll
+  for (int u = 0; u < kLvPer; u++) {
+    const uint32_t p = tile + u * kLvBlock + tid;
+    if (p < nt) {
+      k[u] = key_in[p];
+      id[u] = id_in[p];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kLvPer; u++) {
+    const uint32_t r = u * kLvBlock + tid;
+    const uint32_t d = s_dst[(r / kLvPer) * kDstPad + r % kLvPer];
+    if (tile + r < nt && d != ~0u) {
+      key1[d] = k[u];
+      id1[d] = id[u];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kLvPer; u++) s_dst[tid * kDstPad + u] = dst2[u];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kLvPer; u++) {
+    const uint32_t r = u * kLvBlock + tid;
+    const uint32_t d = s_dst[(r / kLvPer) * kDstPad + r % kLvPer];
+    if (tile + r < nt && d != ~0u) {
+      key2[d] = k[u];
+      id2[d] = id[u];
+      slots_out[d] = slots_in[tile + r];
+    }
+  }
+}
+
 // IDs per chunk of a batch of nq queries that writes W IDs.
 __host__ __device__ inline uint64_t chunk_len(uint64_t W, uint64_t nq) {
   uint64_t c = (W + kChunkCap - 1) / kChunkCap;
@@ -525,15 +736,33 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_mark(const unsigned long long* 
                                                       const uint32_t* __restrict__ tpre,
                                                       const uint32_t* __restrict__ ntask, uint32_t nq,
                                                       uint32_t* __restrict__ chunk_task) {
-  // one thread per (query, range)
-  const uint64_t g = static_cast<uint64_t>(blockIdx.x) * kLvBlock + threadIdx.x;
-  const uint32_t q = static_cast<uint32_t>(g / kTaskCap), i = static_cast<uint32_t>(g % kTaskCap);
-  if (q >= nq || i >= ntask[q]) return;
+  // one wave per query: a lane per range, but all lanes on a range that
+  // starts many chunks (one thread per range took 33 us for 56,000 chunks of
+  // 1024 queries on MI355X, this 8)
+  const uint32_t q = blockIdx.x * (kLvBlock / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  if (q >= nq) return;
+  const uint32_t nt = ntask[q];
   const uint64_t L = chunk_len(woff[nq], nq);
   const uint64_t base = woff[q];
   const uint64_t qb = static_cast<uint64_t>(q) * kTaskCap;
-  const uint64_t a = base + tpre[qb + i], b = base + tpre[qb + i + 1];
-  for (uint64_t c = (a + L - 1) / L; c * L < b; c++) chunk_task[c] = (q << 7) | i;
+  for (uint32_t i0 = 0; i0 < nt; i0 += kWave) {
+    const uint32_t i = i0 + lane;
+    uint32_t c0 = 0, c1 = 0;  // chunks that start in the lane's range (at most kChunkCap in all)
+    if (i < nt) {
+      c0 = static_cast<uint32_t>((base + tpre[qb + i] + L - 1) / L);
+      c1 = static_cast<uint32_t>((base + tpre[qb + i + 1] + L - 1) / L);
+    }
+    const bool many = c1 > c0 + 4;
+    if (!many)
+      for (uint32_t c = c0; c < c1; c++) chunk_task[c] = (q << 7) | i;
+    uint64_t m = __ballot(many);
+    while (m) {
+      const int f = __builtin_ctzll(m);
+      m &= m - 1;
+      const uint32_t e = __shfl(c1, f, kWave);
+      for (uint32_t c = __shfl(c0, f, kWave) + lane; c < e; c += kWave) chunk_task[c] = (q << 7) | (i0 + f);
+    }
+  }
 }
 
 // All lanes of the workgroup copy len IDs, a multiple of the pass size,
@@ -710,8 +939,8 @@ Status build_level_index(int dtype, int id_dtype, size_t n, const void* nodes_d,
       uint32_t* slot_block = nullptr;
       void* sort_block = nullptr;
       if (e == hipSuccess) e = dev_alloc(&slot_block, std::max(slots, n * 8));
-      if (e == hipSuccess) e = dev_alloc(&agg, (ntiles + 1) * 8ull);
-      if (e == hipSuccess) e = dev_alloc(&pre, (ntiles + 1) * 8ull);
+      if (e == hipSuccess) e = dev_alloc(&agg, 2 * (ntiles + 1) * 8ull);
+      if (e == hipSuccess) e = dev_alloc(&pre, 2 * (ntiles + 2) * 8ull);
       const size_t kin_bytes = (n * sizeof(K) + 255) & ~size_t{255};
       if (e == hipSuccess && !inside) e = dev_alloc(&sort_block, kin_bytes + std::max<size_t>(tmp_bytes, 16));
       sa = slot_block;
@@ -737,6 +966,19 @@ Status build_level_index(int dtype, int id_dtype, size_t n, const void* nodes_d,
         for (uint32_t t = 0; t + 1 < H && st.ok(); t++) {
           const uint32_t nt = n32 - ((1u << t) - 1u);
           const uint32_t tiles = (nt + kLvTile - 1) / kLvTile;
+          if ((M >> (t + 2)) >= 1 && t + 2 < H) {
+            hipLaunchKernelGGL(k_lv_tile_counts2, dim3(tiles), dim3(kLvBlock), 0, s, sa, nt, t, agg, ntiles + 1);
+            st = exclusive_scan(agg, pre, tiles, s, 2, ntiles + 1);
+            if (!st.ok()) break;
+            hipLaunchKernelGGL((k_lv_scatter2<K, IS>), dim3(tiles), dim3(kLvBlock), 0, s, sa, sb,
+                               key + static_cast<size_t>(t) * ns, key + static_cast<size_t>(t + 1) * ns,
+                               key + static_cast<size_t>(t + 2) * ns, id + static_cast<size_t>(t) * ns,
+                               id + static_cast<size_t>(t + 1) * ns, id + static_cast<size_t>(t + 2) * ns, pre,
+                               ntiles + 1, nt, t, M);
+            std::swap(sa, sb);
+            t++;
+            continue;
+          }
           hipLaunchKernelGGL(k_lv_tile_counts, dim3(tiles), dim3(kLvBlock), 0, s, sa, nt, t, agg);
           st = exclusive_scan(agg, pre, tiles, s);
           if (!st.ok()) break;
@@ -843,9 +1085,8 @@ Status level_search(const SearchArgs& a, const void* key_d, const void* id_d, Le
       if (!(P.use_single && plan != 2)) {  // a single query's plan wrote these itself
         Status st = exclusive_scan(sc.wq, sc.woff, a.nq, s);
         if (!st.ok()) return st;
-        const uint64_t mark_threads = static_cast<uint64_t>(P.nq) * kTaskCap;
-        hipLaunchKernelGGL(k_lv_mark, dim3(static_cast<unsigned>((mark_threads + kLvBlock - 1) / kLvBlock)),
-                           dim3(kLvBlock), 0, s, sc.woff, sc.tpre, sc.ntask, P.nq, sc.chunk_task);
+        constexpr uint32_t kWaves = kLvBlock / kWave;
+        hipLaunchKernelGGL(k_lv_mark, dim3((P.nq + kWaves - 1) / kWaves), dim3(kLvBlock), 0, s, sc.woff, sc.tpre, sc.ntask, P.nq, sc.chunk_task);
       }
       int dev = 0, cus = 0;
       hipGetDevice(&dev);

@@ -47,20 +47,27 @@ constexpr int kLvPer = 16;
 constexpr uint32_t kLvTile = kLvBlock * kLvPer;  // points per partition tile
 constexpr uint32_t kTaskCap = 128;               // ranges per query: <= 4 per level, <= 31 levels
 constexpr uint32_t kFewQueries = 64;             // write plans of up to this many queries probe wider
-// Copy chunks and workgroups. Queries of kLongQuery IDs and more on average
-// copy best in large chunks by three workgroups per CU (2-4 beat 8 on the
-// 2^26 f32 batch of 1.8M IDs per query); shorter ones spend their time
-// moving between queries and ranges, where more workgroups hide each other's
-// waits: 8192 queries of 14,500 IDs 342 -> 272 us with eight per CU and half
-// the chunk. A small batch is cut into about three chunks per CU (one query
-// of 1.5M IDs 33 -> 13 us: chunks of 32768 left 210 of 256 CUs idle).
-constexpr uint64_t kLongQuery = 65536;
-constexpr uint64_t kMinChunk = 1024, kChunkShort = 16384, kChunkLong = 32768;
-constexpr uint64_t kChunkSpread = 768;
-constexpr uint32_t kCopyPerCu = 8, kCopyPerCuLong = 3;
+// Copy chunks and workgroups. Queries of kLongQuery IDs and more on average,
+// in a large batch, copy best in large chunks by three workgroups per CU (4, 6,
+// 8 are 1 to 3% slower on 1.84G IDs of 1024 queries). Other batches spend
+// their time moving between queries and ranges, where the hardware's own
+// balancing of one chunk per workgroup hides each other's waits: 8192 queries
+// of 14,500 IDs take 342 us with three per CU and chunks of 32768, 273 with
+// eight and 16384, 234 with sixteen, 209 with 64 and 8192 (4.6 TB/s, a large
+// copy's rate). Small batches are cut into about eight chunks per CU, at least
+// 1024 IDs each (one query of 1.5M IDs 33 us in chunks of 32768, which leave
+// most CUs idle, now 11). 64 bytes of loads in flight per lane: with 256 the
+// registers held the CU to half the waves (2785 instead of 2681 us on the
+// large batch).
+constexpr uint64_t kLongQuery = 65536, kLongBatch = 1ull << 26;
+constexpr uint64_t kMinChunk = 1024, kChunkShort = 8192, kChunkLong = 32768;
+constexpr uint64_t kChunkSpread = 2048;
 constexpr uint64_t kChunkCap = 1u << 20;  // chunk table entries
+constexpr uint32_t kCopyPerCu = 64, kCopyPerCuLong = 3, kCopyPerCuFew = 8;
+constexpr uint32_t kFewCopies = 16;  // queries that rarely fill more than kCopyPerCuFew workgroups per CU
+__host__ __device__ inline bool long_copies(uint64_t W, uint64_t nq) { return W >= kLongBatch && W >= nq * kLongQuery; }
 constexpr int kCopyBlock = 256;
-constexpr int kCopyBytes = 256;  // bytes of loads in flight per lane in the copy
+constexpr int kCopyBytes = 64;  // bytes of loads in flight per lane in the copy
 constexpr uint32_t kFlat = 4096;  // positions per flat pass of the copy (16 per lane)
 
 template <typename T>
@@ -456,7 +463,7 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_scatter2(const uint32_t* __rest
 __host__ __device__ inline uint64_t chunk_len(uint64_t W, uint64_t nq) {
   uint64_t c = (W + kChunkCap - 1) / kChunkCap;
   c = (c + 255) & ~255ull;
-  const uint64_t most = W >= nq * kLongQuery ? kChunkLong : kChunkShort;
+  const uint64_t most = long_copies(W, nq) ? kChunkLong : kChunkShort;
   if (c >= most) return c;
   uint64_t f = (W / kChunkSpread + 255) & ~255ull;
   f = f < kMinChunk ? kMinChunk : (f > most ? most : f);
@@ -518,6 +525,23 @@ __device__ inline uint32_t run_prefix(const K* __restrict__ kk, uint32_t len, K 
     hi = nhi;
   }
   return lo;
+}
+
+// Chunks c0..c1-1 start in the lane's range: their table entries. All lanes
+// take part in a range that starts many (one lane per range took 33 us for
+// 56,000 chunks of 1024 queries on MI355X, this 3; in one query's plan 14).
+__device__ inline void mark_chunks(uint32_t* __restrict__ chunk_task, uint32_t entry, uint32_t c0, uint32_t c1,
+                                   uint32_t lane) {
+  const bool many = c1 > c0 + 4;
+  if (!many)
+    for (uint32_t c = c0; c < c1; c++) chunk_task[c] = entry;
+  uint64_t m = __ballot(many);
+  while (m) {
+    const int f = __builtin_ctzll(m);
+    m &= m - 1;
+    const uint32_t v = __shfl(entry, f, kWave), e = __shfl(c1, f, kWave);
+    for (uint32_t c = __shfl(c0, f, kWave) + lane; c < e; c += kWave) chunk_task[c] = v;
+  }
 }
 
 // One workgroup (one wave) per query: the open paths, then the REPORT_ABOVE
@@ -689,13 +713,13 @@ __global__ __launch_bounds__(kWave) void k_lv_plan(LvParams<T, IS> P) {
           if (P.host)
             __hip_atomic_store(P.host, static_cast<unsigned long long>(total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
-        const uint64_t L = chunk_len(clip, 1);
-        auto mark = [&](uint32_t at, uint32_t pre, uint32_t c) {
-          const uint64_t a = pre, b = pre + c < cw ? pre + c : cw;
-          for (uint64_t ch = (a + L - 1) / L; ch * L < b; ch++) P.chunk_task[ch] = at;
+        const uint32_t L = static_cast<uint32_t>(chunk_len(clip, 1));
+        auto mark = [&](bool keep, uint32_t at, uint32_t pre, uint32_t c) {
+          const uint32_t end = keep ? (pre + c < cw ? pre + c : cw) : 0u;
+          mark_chunks(P.chunk_task, at, keep ? (pre + L - 1) / L : 0u, (end + L - 1) / L, lane);
         };
-        if (k0) mark(at0, pre0, cnt[0]);
-        if (k1) mark(at1, pre1, cnt[1]);
+        mark(k0, at0, pre0, cnt[0]);
+        mark(k1, at1, pre1, cnt[1]);
       }
     }
   }
@@ -736,9 +760,7 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_mark(const unsigned long long* 
                                                       const uint32_t* __restrict__ tpre,
                                                       const uint32_t* __restrict__ ntask, uint32_t nq,
                                                       uint32_t* __restrict__ chunk_task) {
-  // one wave per query: a lane per range, but all lanes on a range that
-  // starts many chunks (one thread per range took 33 us for 56,000 chunks of
-  // 1024 queries on MI355X, this 8)
+  // one wave per query, a lane per range
   const uint32_t q = blockIdx.x * (kLvBlock / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
   if (q >= nq) return;
   const uint32_t nt = ntask[q];
@@ -752,16 +774,7 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_mark(const unsigned long long* 
       c0 = static_cast<uint32_t>((base + tpre[qb + i] + L - 1) / L);
       c1 = static_cast<uint32_t>((base + tpre[qb + i + 1] + L - 1) / L);
     }
-    const bool many = c1 > c0 + 4;
-    if (!many)
-      for (uint32_t c = c0; c < c1; c++) chunk_task[c] = (q << 7) | i;
-    uint64_t m = __ballot(many);
-    while (m) {
-      const int f = __builtin_ctzll(m);
-      m &= m - 1;
-      const uint32_t e = __shfl(c1, f, kWave);
-      for (uint32_t c = __shfl(c0, f, kWave) + lane; c < e; c += kWave) chunk_task[c] = (q << 7) | (i0 + f);
-    }
+    mark_chunks(chunk_task, (q << 7) | i, c0, c1, lane);
   }
 }
 
@@ -795,15 +808,14 @@ __global__ __launch_bounds__(kCopyBlock) void k_lv_copy(const IS* __restrict__ i
                                                         const unsigned long long* __restrict__ woff,
                                                         const unsigned long long* __restrict__ offsets,
                                                         const uint32_t* __restrict__ chunk_task, uint32_t nq,
-                                                        IS* __restrict__ out) {
+                                                        uint32_t long_grid, IS* __restrict__ out) {
   __shared__ uint32_t s_pre[kTaskCap + 1];
   __shared__ uint64_t s_src[kTaskCap];
   const uint64_t W = woff[nq];
   const uint64_t L = chunk_len(W, nq);
   const uint64_t nch = (W + L - 1) / L;
   const uint32_t tid = threadIdx.x;
-  // the grid is kCopyPerCu workgroups per CU
-  const uint32_t grid = W >= nq * kLongQuery ? gridDim.x / kCopyPerCu * kCopyPerCuLong : gridDim.x;
+  const uint32_t grid = long_copies(W, nq) ? long_grid : gridDim.x;
   if (blockIdx.x >= grid) return;
   for (uint64_t c = blockIdx.x; c < nch; c += grid) {
     const uint32_t e = chunk_task[c];
@@ -1091,9 +1103,10 @@ Status level_search(const SearchArgs& a, const void* key_d, const void* id_d, Le
       int dev = 0, cus = 0;
       hipGetDevice(&dev);
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      hipLaunchKernelGGL((k_lv_copy<IS>), dim3(static_cast<unsigned>(cus * kCopyPerCu)), dim3(kCopyBlock), 0, s, P.id,
-                         sc.tsrc, sc.tpre, sc.ntask, sc.woff, a.offsets, sc.chunk_task, P.nq,
-                         static_cast<IS*>(a.out));
+      const uint32_t per = P.nq <= kFewCopies ? kCopyPerCuFew : kCopyPerCu;
+      hipLaunchKernelGGL((k_lv_copy<IS>), dim3(static_cast<unsigned>(cus) * per), dim3(kCopyBlock), 0, s, P.id, sc.tsrc,
+                         sc.tpre, sc.ntask, sc.woff, a.offsets, sc.chunk_task, P.nq,
+                         static_cast<uint32_t>(cus) * kCopyPerCuLong, static_cast<IS*>(a.out));
       return hip_status(hipGetLastError(), "Error in launching level search");
     });
   });

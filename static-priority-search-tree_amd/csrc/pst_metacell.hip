@@ -16,8 +16,9 @@
 // of reading it again; at the end of each metacell row it reduces every
 // metacell's mx + 1 columns from LDS. The volume is read about 1 + 1/mz
 // times (the shared boundary planes of neighbouring slabs); the bound is HBM
-// bandwidth. Metacells of 256 or more voxels along x use k_metacells, one
-// workgroup per metacell row with an LDS column tile.
+// bandwidth. Metacells of 4 x 4 x 4 voxels with 4-byte values use
+// k_metacells4, a metacell per lane; those of 256 or more voxels along x use
+// k_metacells, one workgroup per metacell row with an LDS column tile.
 #include <cfloat>
 #include <climits>
 
@@ -30,15 +31,15 @@ namespace {
 constexpr int kMcBlock = 256;
 constexpr uint32_t kMcCols = 4096;  // vertex columns per LDS tile
 
+// The first of two equal values, and of two that do not compare: one
+// comparison and one select.
 template <typename T>
 __device__ inline T vmin(T a, T b) {
-  if constexpr (std::is_floating_point<T>::value) return a < b ? a : (b < a ? b : a);
-  else return a < b ? a : b;
+  return b < a ? b : a;
 }
 template <typename T>
 __device__ inline T vmax(T a, T b) {
-  if constexpr (std::is_floating_point<T>::value) return a > b ? a : (b > a ? b : a);
-  else return a > b ? a : b;
+  return b > a ? b : a;
 }
 
 template <typename T, typename I>
@@ -182,6 +183,128 @@ __global__ __launch_bounds__(kSweepBlock) void k_metacells_sweep(const T* __rest
 }
 
 // ---------------------------------------------------------------------------
+// Metacells of 4 x 4 x 4 voxels with 4-byte values: a wave owns 64 metacells
+// of a row, a lane one metacell's first four vertex columns, which it reads as
+// 16 bytes per vertex row. A metacell's fifth column is the next lane's first,
+// by one shuffle; the wave's last lane gets its from lanes 0 to 4, which load
+// one row each. No LDS and no barrier; the fifth rows and planes are read by
+// two waves, mostly out of the caches.
+//
+// Bound by HBM and the caches behind it: 1024^3 f32 takes 0.81 ms, 5.6 TB/s of
+// the volume and the records (a plain read of the volume runs at 6.4 TB/s;
+// k_metacells_sweep took 1.15 ms, fetching 6.1 GB for the 4.3, and 1.10 with
+// one select per minimum). What was tried at that size: a wave sweeping 2, 4,
+// 8 or 16 layers with the shared plane carried reads 5.1 GB but takes 0.88,
+// 0.90, 0.93, 0.92 ms, and two or three metacell rows per wave 0.93, 0.90
+// (fewer bytes, but the waves at work are spread over more planes); sharing
+// rows and columns of a workgroup through LDS 1.3-2.0; x before y in the block
+// order 0.86; a range of blocks per XCD 0.85-0.90; 1, 2, 4, 8, 16 waves per
+// workgroup 0.89, 0.84, 0.82, 0.81, 0.84; 1, 2, 4 planes folded together all
+// 0.82; non-temporal loads 1.19 against 0.96 (the rows shared by waves leave
+// the L2).
+//
+// Minima of equal values (-0 and +0) keep the first, and NaN stays if first,
+// as in k_metacells_sweep: each column of each row is folded over z, then the
+// rows in y order, then the columns in x order.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kWaves4 = 8;     // metacell rows per workgroup
+constexpr uint32_t kTogether4 = 2;  // planes folded together
+
+template <typename T, typename I>
+__global__ __launch_bounds__(64 * kWaves4) void k_metacells4(const T* __restrict__ vol, uint32_t px, uint32_t py,
+                                                             uint32_t pz, uint32_t gx, uint32_t gy, uint32_t bx,
+                                                             uint32_t by, Point<T, I>* __restrict__ out) {
+  typedef T __attribute__((ext_vector_type(4), aligned(sizeof(T)))) V4;
+  const uint32_t lane = threadIdx.x % 64;
+  uint32_t blk = blockIdx.x;  // y, then x, then z
+  const uint32_t b = blk % by * kWaves4 + threadIdx.x / 64;
+  blk /= by;
+  const uint32_t a0 = blk % bx * 64, a = a0 + lane;
+  const uint32_t c = blk / bx;
+  if (b >= gy) return;
+  const size_t plane = static_cast<size_t>(px) * py;
+  const uint32_t last = px - 1;
+  const uint32_t base = min(4 * a, last - 3), shift = min(4 * a - base, 3u);
+  const bool edge = lane < 5 && 4 * (a0 + 64) <= last;
+  const T* const mine = vol + base;
+  const T* const col = vol + static_cast<size_t>(min(4 * b + lane, py - 1)) * px + 4 * (a0 + 64);
+  struct Plane {
+    V4 v[5];
+    T e;
+  };
+  auto load = [&](uint32_t z, Plane& p) {
+    const size_t at = static_cast<size_t>(z) * plane;
+#pragma unroll
+    for (uint32_t r = 0; r < 5; r++)  // rows past the grid repeat the last one
+      p.v[r] = *reinterpret_cast<const V4*>(mine + at + static_cast<size_t>(min(4 * b + r, py - 1)) * px);
+    p.e = T{};
+    if (edge) p.e = col[at];
+  };
+  Plane lo, hi, p[kTogether4];
+  load(4 * c, lo);
+#pragma unroll
+  for (uint32_t z = 1; z <= 4; z += kTogether4) {
+#pragma unroll
+    for (uint32_t i = 0; i < kTogether4; i++) load(min(4 * c + z + i, pz - 1), p[i]);
+    if (z == 1) hi = lo;
+#pragma unroll
+    for (uint32_t i = 0; i < kTogether4; i++) {
+#pragma unroll
+      for (uint32_t r = 0; r < 5; r++)
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+          lo.v[r][k] = vmin<T>(lo.v[r][k], p[i].v[r][k]);
+          hi.v[r][k] = vmax<T>(hi.v[r][k], p[i].v[r][k]);
+        }
+      lo.e = vmin(lo.e, p[i].e);
+      hi.e = vmax(hi.e, p[i].e);
+    }
+  }
+  V4 l = lo.v[0], h = hi.v[0];
+#pragma unroll
+  for (uint32_t r = 1; r < 5; r++)
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+      l[k] = vmin<T>(l[k], lo.v[r][k]);
+      h[k] = vmax<T>(h[k], hi.v[r][k]);
+    }
+  // where the grid ends within the lane's four columns the last four were
+  // loaded: its own to the front, the last one repeated
+#pragma unroll
+  for (uint32_t s = 1; s < 4; s *= 2)
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+      l[k] = shift & s ? l[min(k + s, 3u)] : l[k];
+      h[k] = shift & s ? h[min(k + s, 3u)] : h[k];
+    }
+  T el = __shfl(lo.e, 0), eh = __shfl(hi.e, 0);
+#pragma unroll
+  for (uint32_t r = 1; r < 5; r++) {
+    el = vmin(el, __shfl(lo.e, r));
+    eh = vmax(eh, __shfl(hi.e, r));
+  }
+  const T nl = __shfl_down(static_cast<T>(l[0]), 1), nh = __shfl_down(static_cast<T>(h[0]), 1);
+  T mn = l[0], mx = h[0];
+#pragma unroll
+  for (uint32_t k = 1; k < 4; k++) {
+    mn = vmin<T>(mn, l[k]);
+    mx = vmax<T>(mx, h[k]);
+  }
+  if (4 * a + 4 <= last) {
+    mn = vmin(mn, lane == 63 ? el : nl);
+    mx = vmax(mx, lane == 63 ? eh : nh);
+  }
+  if (a < gx) {
+    const uint64_t id = a + (static_cast<uint64_t>(b) + static_cast<uint64_t>(c) * gy) * gx;
+    Point<T, I> q;
+    q.dim1_val = mn;
+    q.dim2_val = mx;
+    if constexpr (has_id_v<I>) q.id = static_cast<I>(id);
+    out[id] = q;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Synthetic volume: value(i, j, k) = sum_g amp_g exp(-|p - c_g|^2 / (2 s_g^2))
 // + noise_std * N(0, 1), p = (i, j, k) / (dims - 1). The normal draw is a
 // Box-Muller transform of two uniforms from SplitMix64 over (seed, vertex
@@ -271,13 +394,29 @@ Status form_metacells(int dtype, int id_dtype, const void* vertices_d, const uin
     return with_id(id_dtype, [&](auto i) {
       using T = decltype(t);
       using I = decltype(i);
-      if (mc_dims[0] < static_cast<uint32_t>(kSweepBlock)) {
+      // Metacells of 4 x 4 x 4 with 4-byte values: 40^3 5.1 us against 15.8 of
+      // the sweep, 256^3 14 / 32, 12 x 301 x 1639 37 / 63, 1023 x 511 x 300
+      // 119 / 155, 1024^3 0.81 / 1.10 ms. 8-byte values stay with the sweep: a
+      // lane's 32 bytes take two loads that each use half of every line, and
+      // rows off the lines lose (1030 x 300 x 300 f64 202 us against 186;
+      // 512^3 251 / 278). The grid's limit is 2^31 lanes.
+      bool fours = false;
+      if constexpr (sizeof(T) == 4) {
+        const uint64_t bx = (g[0] + 63) / 64, by = (g[1] + kWaves4 - 1) / kWaves4, blocks = bx * by * g[2];
+        fours = mc_dims[0] == 4 && mc_dims[1] == 4 && mc_dims[2] == 4 && pt_dims[0] >= 4 &&
+                blocks <= (1ull << 31) / (64 * kWaves4);
+        if (fours)
+          k_metacells4<T, I><<<static_cast<uint32_t>(blocks), 64 * kWaves4, 0, stream>>>(
+              static_cast<const T*>(vertices_d), pt_dims[0], pt_dims[1], pt_dims[2], g[0], g[1],
+              static_cast<uint32_t>(bx), static_cast<uint32_t>(by), static_cast<Point<T, I>*>(out_pts_d));
+      }
+      if (!fours && mc_dims[0] < static_cast<uint32_t>(kSweepBlock)) {
         const uint32_t cpb = (kSweepBlock - 1) / mc_dims[0];
         const dim3 grid((g[0] + cpb - 1) / cpb, g[2], (g[1] + kSweepRows - 1) / kSweepRows);
         k_metacells_sweep<T, I><<<grid, kSweepBlock, 0, stream>>>(
             static_cast<const T*>(vertices_d), pt_dims[0], pt_dims[1], pt_dims[2], mc_dims[0], mc_dims[1],
             mc_dims[2], g[0], g[1], static_cast<Point<T, I>*>(out_pts_d));
-      } else {
+      } else if (!fours) {
         k_metacells<T, I><<<dim3(g[1], g[2]), kMcBlock, 0, stream>>>(
             static_cast<const T*>(vertices_d), pt_dims[0], pt_dims[1], pt_dims[2], mc_dims[0], mc_dims[1],
             mc_dims[2], g[0], g[1], static_cast<Point<T, I>*>(out_pts_d));

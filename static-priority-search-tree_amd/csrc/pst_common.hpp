@@ -323,4 +323,39 @@ __device__ inline V shfl(V v, int src) {
   return __shfl(v, src, kWave);
 }
 
+// Loads and stores of data that is used once, marked as streaming, for values
+// of 4, 8, 12 or 16 bytes (others: ordinary). The hint keeps them from taking
+// the place of data in the caches that is used again; the users name what it
+// gave.
+template <typename V>
+constexpr bool kStreams = sizeof(V) % 4 == 0 && sizeof(V) <= 16 && alignof(V) >= 4;
+
+template <typename V>
+__device__ inline V stream_load(const V* p) {
+  if constexpr (kStreams<V>) {
+    typedef uint32_t __attribute__((may_alias)) Word;
+    Word w[sizeof(V) / 4];  // the compiler joins the words' accesses
+#pragma unroll
+    for (size_t k = 0; k < sizeof(V) / 4; k++) w[k] = __builtin_nontemporal_load(reinterpret_cast<const Word*>(p) + k);
+    V v;
+    __builtin_memcpy(&v, w, sizeof(V));
+    return v;
+  } else {
+    return *p;
+  }
+}
+
+template <typename V>
+__device__ inline void stream_store(V* p, const V& v) {
+  if constexpr (kStreams<V>) {
+    typedef uint32_t __attribute__((may_alias)) Word;
+    Word w[sizeof(V) / 4];
+    __builtin_memcpy(w, &v, sizeof(V));
+#pragma unroll
+    for (size_t k = 0; k < sizeof(V) / 4; k++) __builtin_nontemporal_store(w[k], reinterpret_cast<Word*>(p) + k);
+  } else {
+    *p = v;
+  }
+}
+
 }  // namespace pst

@@ -439,8 +439,9 @@ __global__ __launch_bounds__(kIsoWave) void k_mc_write(const T* __restrict__ vol
 //
 // Measured on 670,647 active metacells of a 1024^3 volume (49.1M triangles,
 // 1.77 GB) on MI355X, against the general kernels above: count 0.309 -> 0.207
-// ms (4.3 TB/s of 128-byte row requests), write 1.68 -> 0.75 ms (1.23 GB read
-// and 1.79 GB written, 4.0 TB/s; a large copy reaches 4.8).
+// ms (4.3 TB/s of 128-byte row requests), write 1.68 -> 0.63 ms (1.23 GB read
+// and 1.79 GB written, 4.8 TB/s; 0.75 before the triangles were stored as
+// streaming, which leaves the L2 to the vertices that metacells share).
 // ---------------------------------------------------------------------------
 constexpr int kMc4Waves = 4;               // waves per workgroup (one LDS case table)
 constexpr int kMc4BlocksPerCu = 20;
@@ -687,7 +688,7 @@ __global__ __launch_bounds__(kMc4Waves * kIsoWave) void k_mc_write4(const T* __r
           p.x = fx + static_cast<float>(pl.x & 0xff) + t * static_cast<float>(pl.y & 0xff);
           p.y = fy + static_cast<float>((pl.x >> 8) & 0xff) + t * static_cast<float>((pl.y >> 8) & 0xff);
           p.z = fz + static_cast<float>((pl.x >> 16) & 0xff) + t * static_cast<float>((pl.y >> 16) & 0xff);
-          *reinterpret_cast<float3*>(o + 3 * j) = p;
+          stream_store(reinterpret_cast<float3*>(o + 3 * j), p);
         }
         iso_wave_sync();
       }
@@ -707,7 +708,7 @@ __global__ __launch_bounds__(kMc4Waves * kIsoWave) void k_mc_write4(const T* __r
 // take the output's vertices.
 //
 // Measured on the same 670,647 metacells on MI355X against the general
-// kernels above: count 0.316 -> 0.229 ms, write 4.14 -> 1.74 ms (bound by
+// kernels above: count 0.316 -> 0.229 ms, write 4.14 -> 1.56 ms (bound by
 // instruction issue: seven divisions per vertex pair and two passes over the
 // triangles).
 // ---------------------------------------------------------------------------
@@ -947,7 +948,7 @@ __global__ __launch_bounds__(kMc4Waves * kIsoWave) void k_iso_write4(const T* __
         }
         iso_wave_sync();
         float* o = out + 9 * base;
-        for (uint32_t j = lane; j < 3 * nt; j += kIsoWave) *reinterpret_cast<float3*>(o + 3 * j) = point(list[j]);
+        for (uint32_t j = lane; j < 3 * nt; j += kIsoWave) stream_store(reinterpret_cast<float3*>(o + 3 * j), point(list[j]));
         iso_wave_sync();
       }
       c = cn;

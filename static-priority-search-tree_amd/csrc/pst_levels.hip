@@ -53,12 +53,13 @@ constexpr uint32_t kFewQueries = 64;             // write plans of up to this ma
 // their time moving between queries and ranges, where the hardware's own
 // balancing of one chunk per workgroup hides each other's waits: 8192 queries
 // of 14,500 IDs take 342 us with three per CU and chunks of 32768, 273 with
-// eight and 16384, 234 with sixteen, 209 with 64 and 8192 (4.6 TB/s, a large
-// copy's rate). Small batches are cut into about eight chunks per CU, at least
+// eight and 16384, 234 with sixteen, 209 with 64 and 8192 (4.6 TB/s). Small batches are cut into about eight chunks per CU, at least
 // 1024 IDs each (one query of 1.5M IDs 33 us in chunks of 32768, which leave
 // most CUs idle, now 11). 64 bytes of loads in flight per lane: with 256 the
 // registers held the CU to half the waves (2785 instead of 2681 us on the
-// large batch).
+// large batch). The IDs are stored as streaming: 2687 -> 2480 us on the large
+// batch and 209 -> 193 (5.0 TB/s) on the short one; loads stay ordinary, since
+// queries share ranges (3154 us with both, the short one 222).
 constexpr uint64_t kLongQuery = 65536, kLongBatch = 1ull << 26;
 constexpr uint64_t kMinChunk = 1024, kChunkShort = 8192, kChunkLong = 32768;
 constexpr uint64_t kChunkSpread = 2048;
@@ -790,7 +791,7 @@ __device__ inline void copy_passes(const IS* __restrict__ src, IS* __restrict__ 
 #pragma unroll
     for (int u = 0; u < U; u++) v[u] = src[k0 + u * kCopyBlock + tid];
 #pragma unroll
-    for (int u = 0; u < U; u++) dst[k0 + u * kCopyBlock + tid] = v[u];
+    for (int u = 0; u < U; u++) stream_store(&dst[k0 + u * kCopyBlock + tid], v[u]);
   }
 }
 
@@ -881,7 +882,7 @@ __global__ __launch_bounds__(kCopyBlock) void k_lv_copy(const IS* __restrict__ i
         }
 #pragma unroll
         for (int u = 0; u < V; u++)
-          if (x + u * kCopyBlock + tid < fend) out[obase + loc[u]] = v[u];
+          if (x + u * kCopyBlock + tid < fend) stream_store(&out[obase + loc[u]], v[u]);
       }
       x = fend;
       while (i < nt && wbase + s_pre[i + 1] <= x) i++;

@@ -15,7 +15,11 @@
 //    per-wave stage in LDS at their ballot/mbcnt prefix;
 //  - a full stage is flushed with one atomic on the per-call counter
 //    followed by coalesced stores; a chunk with many hits (dense queries)
-//    reserves its own range and is written directly.
+//    reserves its own range and is written directly;
+//  - what is left at the end is written with one atomic per workgroup: the
+//    4096 waves' own atomics on the one counter came all at once and took up
+//    to 45 us (f32, 10^6 points 17 -> 9 us, 4 * 10^6 54 -> 20, 16 * 10^6
+//    71 -> 36, 67 * 10^6 150 -> 136; there the bound is HBM, 5.9 TB/s).
 // So the counter sees about one atomic per 512 results (sparse) or per
 // chunk (dense), not one per tile.
 #include <algorithm>
@@ -30,9 +34,13 @@ constexpr int kIpsBlock = 256;              // four independent waves per workgr
 constexpr int kIpsElems = 16;               // records per lane per chunk
 constexpr uint32_t kIpsChunk = kWave * kIpsElems;  // 1024 records per wave chunk
 constexpr uint32_t kIpsStage = 512;         // staged results per wave
+// Arrays beyond the last-level cache are loaded as streaming: 805 MB that are
+// not cached 172 -> 143 us; smaller ones may still be there from the last call
+// (10^5 points 8.4 us, as streaming 9.0).
+constexpr uint64_t kIpsStreamBytes = 256ull << 20;
 constexpr uint32_t kIpsDirect = 256;        // a chunk with at least this many hits is written directly
 
-template <typename T, typename IS, bool RET_POINT>
+template <typename T, typename IS, bool RET_POINT, bool STREAM>
 __global__ __launch_bounds__(kIpsBlock) void k_ips(const Point<T, IS>* __restrict__ pts, uint64_t n, T q,
                                                    void* __restrict__ out, unsigned long long cap,
                                                    unsigned long long* __restrict__ counter) {
@@ -68,7 +76,10 @@ __global__ __launch_bounds__(kIpsBlock) void k_ips(const Point<T, IS>* __restric
     if (first + kIpsChunk <= n) {
       // full chunk: every load issued before any test
 #pragma unroll
-      for (int e = 0; e < kIpsElems; e++) p[e] = pts[first + static_cast<uint64_t>(e) * kWave + lane];
+      for (int e = 0; e < kIpsElems; e++) {
+        const Point<T, IS>* at = &pts[first + static_cast<uint64_t>(e) * kWave + lane];
+        p[e] = STREAM ? stream_load(at) : *at;
+      }
 #pragma unroll
       for (int e = 0; e < kIpsElems; e++) hb[e] = __ballot(p[e].dim1_val <= q && q <= p[e].dim2_val);
     } else {
@@ -112,7 +123,23 @@ __global__ __launch_bounds__(kIpsBlock) void k_ips(const Point<T, IS>* __restric
     }
     staged = run;
   }
-  if (staged) flush();
+  // the waves' last results, with one atomic for the workgroup
+  __shared__ uint32_t left[kIpsBlock / kWave];
+  __shared__ unsigned long long left_at;
+  if (lane == 0) left[wave] = staged;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < kIpsBlock / kWave; w++) {
+    before += w < wave ? left[w] : 0u;
+    all += left[w];
+  }
+  if (all == 0) return;
+  if (threadIdx.x == 0) left_at = atomicAdd(counter, static_cast<unsigned long long>(all));
+  __syncthreads();
+  const unsigned long long base = left_at + before;
+  for (uint32_t i = lane; i < staged; i += kWave)
+    if (base + i < cap) o[base + i] = stage[i];
 }
 
 template <typename F>
@@ -159,13 +186,16 @@ Status ips_search(int dtype, int id_dtype, const void* pts_d, size_t n, int ret_
         const uint64_t blocks = (chunks + kIpsBlock / kWave - 1) / (kIpsBlock / kWave);
         grid = static_cast<unsigned>(std::max<uint64_t>(1, std::min<uint64_t>(blocks, static_cast<uint64_t>(cus) * 4)));
       }
+      const bool streams = n > kIpsStreamBytes / sizeof(Point<T, IS>);
       const auto* p = static_cast<const Point<T, IS>*>(pts_d);
       if (ret_point) {
-        k_ips<T, IS, true><<<grid, kIpsBlock, 0, stream>>>(p, n, q, out_d, cap, counter_d);
+        if (streams) k_ips<T, IS, true, true><<<grid, kIpsBlock, 0, stream>>>(p, n, q, out_d, cap, counter_d);
+        else k_ips<T, IS, true, false><<<grid, kIpsBlock, 0, stream>>>(p, n, q, out_d, cap, counter_d);
       } else {
-        if constexpr (has_id_v<IS>)
-          k_ips<T, IS, false><<<grid, kIpsBlock, 0, stream>>>(p, n, q, out_d, cap, counter_d);
-        else
+        if constexpr (has_id_v<IS>) {
+          if (streams) k_ips<T, IS, false, true><<<grid, kIpsBlock, 0, stream>>>(p, n, q, out_d, cap, counter_d);
+          else k_ips<T, IS, false, false><<<grid, kIpsBlock, 0, stream>>>(p, n, q, out_d, cap, counter_d);
+        } else
           return Status{1, "Error: IDs requested from points without IDs"};
       }
       return hip_status(hipGetLastError(), "Error in launching interval parallel search");

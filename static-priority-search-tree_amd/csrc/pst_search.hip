@@ -1160,18 +1160,48 @@ TreeShape tree_shape(const SearchArgs& a) {
 
 }  // namespace
 
-// Launches of a pass: a.rounds, or by default 4 for walks of single queries
-// and 3 for group walks, 2 where the batch is small (a launch more costs what
-// its balance gains: 32 queries on 2^20 points 196 with 3, 62 us with 2; 256
-// on 2^23 184 with 3, 268 with 2).
-constexpr uint64_t kSmallWalk = 1ull << 25;  // groups x points
+// The schedule of a pass: a.rounds launches, or by default 4 for walks of
+// single queries and 2 or 3 for group walks, whose first rounds stop after a
+// few steps per batch (search_budget) and whose last one runs every stack to
+// empty. A batch of one item needs seven steps to fill a wave's lanes, and each
+// step after that doubles what a round hands on: many groups on few points
+// have enough items after one round, and a second would only move them through
+// memory; few groups on many points need it for balance. By points per group,
+// count / write passes in us on MI355X, at 2 rounds (9 steps), 3 (7), 3 (8):
+//   1396 queries on 4,183,215 (24k)  350/ 965   276/ 846   475/1063
+//   2500 on 4,183,215         (13k)  403/1227   443/1210  1115/1898
+//   2500 on 2,000,003          (6k)  232/ 817   331/ 887   887/1468
+//   1000 on 2,000,003         (16k)  129/ 595   199/ 586   219/ 630
+//   256 on 2^20               (33k)   66/ 181   189/ 284   143/ 213
+//   2000 on 2^23              (34k)  793/1605   577/1477  1096/1828
+//   3000 on 2^25              (89k)      3368       2728       3159
+//   4096 on 2^26             (131k)      9016       6562       5391
+//   2048 on 2^26             (262k)      4788       4368       3462
+//   256 on 2^23              (262k)  247/ 675   167/ 447   165/ 445
+//   32 on 2^20               (262k)   74/ 175   244/ 237   136/ 193
+// 4 rounds of 6 and 384 steps take 309/1540, 466/1884, 327/1555, 216/1263,
+// 256/345, 637/1659, 3432, 6387, 4135, 435/718 and 228/318.
+constexpr uint64_t kSmallWalk = 1ull << 25;    // groups x points
+constexpr uint64_t kSmallTree = 1ull << 21;    // points
+constexpr uint64_t kGroupPoints = 1ull << 14;  // points per group below which groups alone fill the rounds
+constexpr uint64_t kWidePoints = 1ull << 17;   // and from which a round hands on one more doubling
+
 int search_rounds(const SearchArgs& a) {
   if (a.rounds > 0) return std::min(a.rounds, kMaxRounds);
   if (group_size(a) == 1) return 4;
-  return (a.nq + kGroup - 1) / kGroup * static_cast<uint64_t>(a.n) <= kSmallWalk ? 2 : 3;
+  const uint64_t n = a.n, groups = (a.nq + kGroup - 1) / kGroup;
+  return n <= kSmallTree || groups * n <= kSmallWalk || n < groups * kGroupPoints ? 2 : 3;
 }
 
 namespace {
+
+// Steps per batch in the rounds before the last, while lists are short.
+int search_budget(const SearchArgs& a, int group, int rounds) {
+  if (group == 1) return 6;
+  if (rounds <= 2) return 9;
+  return a.n >= (a.nq + kGroup - 1) / kGroup * kWidePoints ? 8 : 7;
+}
+
 
 // The walk's kernel parameters, but for its overflow stacks and task list.
 template <typename T, typename IS, bool RP, bool W, int G>
@@ -1228,18 +1258,10 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
   const uint32_t bound = 2 * kWave * (H + 2) + 4 * kWave;
   P.gcap = ((bound + kMoveBlock - 1) / kMoveBlock) * kMoveBlock;
   const int R = search_rounds(a);
-  // Step budgets. Group walks spread their work in rounds of 8 steps per
-  // batch (9 when there is one such round), and run every stack to empty in
-  // the last: a batch of one item needs seven steps to fill a wave's lanes, so
-  // with 6 a list of 10^4 items still held whole subtrees, and the 384 steps
-  // that followed at 8192 items and more ran on a few waves only. MI355X, count
-  // / write passes, 4 rounds of 6 and 384 -> these: 256 queries on 700,001
-  // points 450/464 -> 75/96 us, 700 on 5,000,011 271/768 -> 230/700, 2048 on
-  // 2^26 4.23/8.12 -> 3.48/7.98 ms; budgets of 7, 10 and more lose on most
-  // sizes. One query's walk (no group) keeps its own. A write step costs more
-  // than a count step (staging, flushes, copy tasks), so long lists hand work
-  // on after fewer steps there.
-  P.budget_small = a.budget_small > 0 ? a.budget_small : (G == 1 ? 6 : (R <= 2 ? 9 : 8));
+  // Step budgets of lists shorter and longer than few_items. A write step
+  // costs more than a count step (staging, flushes, copy tasks), so long lists
+  // hand work on after fewer steps there.
+  P.budget_small = a.budget_small > 0 ? a.budget_small : search_budget(a, G, R);
   P.budget_large = a.budget_large > 0 ? a.budget_large : (W ? 192 : 384);
   auto kern = k_search_round<T, IS, RP, W, G>;
   int dev = 0;
@@ -1353,8 +1375,9 @@ size_t search_scratch_bytes(size_t n, int dtype, int cus) {
   const size_t lists = 2 * (size_t{1} << 22) * sizeof(Entry);
   const size_t tasks = kCopyTaskCap * sizeof(CopyTask);
   const size_t ctr = (2 * kMaxRounds + 4) * 8 + 8;
+  const size_t front = (kFrontTasks + 1) * sizeof(FrontTask);  // single queries
   (void)dtype;
-  return lists + tasks + waves * gcap * sizeof(Items::type) + ctr;
+  return lists + tasks + waves * gcap * sizeof(Items::type) + ctr + front;
 }
 
 const char* const kPinnedScratchMsg =

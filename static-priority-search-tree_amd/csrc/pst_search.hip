@@ -1195,11 +1195,19 @@ int search_rounds(const SearchArgs& a) {
 
 namespace {
 
-// Steps per batch in the rounds before the last, while lists are short.
+// Steps per batch in the rounds before the last, while lists are short. Of two
+// rounds, 9 steps lose to 8 on small trees between 128 and 384 groups, where
+// the longer list of the second round is dealt to the waves less evenly: count
+// passes in us, 9 / 8 steps (4 rounds of 6: last)
+//   2000 queries on 65536 122 / 65 (131), on 200,000 217 / 74 (227), on
+//   1,000,003 326 / 127 (199); 3000 on 100,000 357 / 101 (253);
+//   beyond: 4096 on 65536 140 / 213 (334), 1000 on 2,000,003 127 / 165 (216),
+//   640 on 2^20 79 / 96 (165), 3400 on 2^20 265 / 318 (356).
 int search_budget(const SearchArgs& a, int group, int rounds) {
   if (group == 1) return 6;
-  if (rounds <= 2) return 9;
-  return a.n >= (a.nq + kGroup - 1) / kGroup * kWidePoints ? 8 : 7;
+  const uint64_t groups = (a.nq + kGroup - 1) / kGroup;
+  if (rounds <= 2) return groups >= 128 && groups < 384 && a.n <= kSmallTree / 2 ? 8 : 9;
+  return a.n >= groups * kWidePoints ? 8 : 7;
 }
 
 

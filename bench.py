@@ -36,8 +36,8 @@ sys.path.insert(0, PKG)
 
 HBM_PEAK_GBPS = 8000.0
 BYTES_PER_ID = 21  # 3 x f32 (dim1, dim2, med) + u32 id + 1 B bitcode read, u32 written
-# kernel launches of one write pass of the walk: four walk rounds and the subtree copy kernel
-WRITE_LAUNCHES = 5
+# kernel launches of one write pass of the walk: three walk rounds and the subtree copy kernel
+WRITE_LAUNCHES = 4
 # level index write pass: each reported u32 ID is read once from a sorted run and written once
 COPY_BYTES_PER_ID = 8
 
@@ -1052,7 +1052,7 @@ def main():
                      "unit": "GB/s", "frac": round(frac, 4), "traffic": traffic,
                      "traffic_frac": traffic_frac,
                      "alg_bytes_per_id": BYTES_PER_ID,
-                     "kernel": "write pass: k_search_round<float, unsigned int, false, true, 8> x 4 "
+                     "kernel": "write pass: k_search_round<float, unsigned int, false, true, 8> x 3 "
                                "+ k_copy_tasks<float, unsigned int, false, 8> x 1",
                      "launches_per_pass": WRITE_LAUNCHES,
                      "avg_launch_ms": round(t_write / WRITE_LAUNCHES, 3),

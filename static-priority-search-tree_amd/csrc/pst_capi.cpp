@@ -213,13 +213,13 @@ int blocking_search(pst_tree* t, int kind, int ret, size_t* num, void** res, con
   hipSetDevice(t->device);
   const size_t rec = ret == PST_RET_POINT ? pst_point_size(t->dtype, t->id_dtype) : id_size(t->id_dtype);
   void* out = nullptr;
-  hipError_t e = pst::dev_alloc(&out, t->n * rec);
+  hipError_t e = pst::result_alloc(&out, t->n * rec);
   if (e != hipSuccess)
     return fail(PST_ERR_HIP, "Error in allocating array to store PointStruct search result" +
                                  dev_suffix(t->dev_ind, t->num_devs) + hipGetErrorString(e));
   int rc = single_search(t, kind, ret, a, b, c, out, t->n, num, t->stream);
   if (rc != PST_OK) {
-    pst::dev_free(out);
+    pst::result_free(out);
     *res = nullptr;
     return rc;
   }
@@ -350,7 +350,7 @@ size_t pst_point_size(int dtype, int id_dtype) {
 
 int pst_free(void* p) {
   if (!p) return PST_OK;
-  hipError_t e = pst::dev_free(p);
+  hipError_t e = pst::result_free(p);
   if (e != hipSuccess) return fail(pst::hip_status(e, "Error in freeing search result array"));
   return PST_OK;
 }
@@ -1189,18 +1189,19 @@ int surface_blocking(IsoCountFn cfn, IsoWriteFn wfn, const void* vertex_arr_d, i
                          "Error in reading the triangle count");
   if (st.ok()) st = pst::hip_status(hipMemcpy(&bad, err, 8, hipMemcpyDeviceToHost), "Error in reading the error flag");
   if (st.ok() && bad) st = Status{PST_ERR_INVALID, "Error: a metacell ID lies past the metacell grid"};
-  float* tri = nullptr;
+  void* tri = nullptr;
   if (st.ok() && total)
-    st = pst::hip_status(pst::dev_alloc(&tri, total * 9 * sizeof(float)), "Error in allocating the triangle array");
+    st = pst::hip_status(pst::result_alloc(&tri, total * 9 * sizeof(float)), "Error in allocating the triangle array");
   if (st.ok() && total)
-    st = wfn(dtype, id_dtype, vertex_arr_d, p32, m32, metacell_ids_d, num_ids, isovalue, offsets, total, tri, nullptr);
+    st = wfn(dtype, id_dtype, vertex_arr_d, p32, m32, metacell_ids_d, num_ids, isovalue, offsets, total,
+             static_cast<float*>(tri), nullptr);
   if (st.ok()) st = pst::hip_status(hipStreamSynchronize(nullptr), "Error in synchronising after isosurface extraction");
   pst::dev_free(counts);
   if (!st.ok()) {
-    if (tri) pst::dev_free(tri);
+    if (tri) pst::result_free(tri);
     return fail(st);
   }
-  *triangles_d = tri;
+  *triangles_d = static_cast<float*>(tri);
   *num_triangles = total;
   return PST_OK;
 }
@@ -1258,7 +1259,7 @@ int pst_form_metacell_tags(const void* vertex_arr_d, int dtype, int id_dtype, co
   const size_t nm = pst_calc_num_metacells(pt_grid_dims, metacell_dims, nullptr);
   if (nm == 0) return fail(PST_ERR_INVALID, "Error: empty metacell grid");
   void* out = nullptr;
-  hipError_t e = pst::dev_alloc(&out, nm * pst::point_size(dtype, id_dtype));
+  hipError_t e = pst::result_alloc(&out, nm * pst::point_size(dtype, id_dtype));
   if (e != hipSuccess)
     return fail(PST_ERR_HIP, "Error in allocating metacell tag storage array" + dev_suffix(dev_ind, num_devs) +
                                  hipGetErrorString(e));
@@ -1266,7 +1267,7 @@ int pst_form_metacell_tags(const void* vertex_arr_d, int dtype, int id_dtype, co
   if (rc == PST_OK && hipStreamSynchronize(nullptr) != hipSuccess)
     rc = fail(PST_ERR_HIP, "Error in synchronising after metacell formation");
   if (rc != PST_OK) {
-    pst::dev_free(out);
+    pst::result_free(out);
     return rc;
   }
   *metacell_arr_d = out;
@@ -1298,7 +1299,7 @@ int pst_interval_parallel_search(const void* pt_arr_d, size_t n, int dtype, int 
     return fail(PST_ERR_INVALID, "Error: IDs requested from points without IDs");
   const size_t rec = ret == PST_RET_POINT ? pst::point_size(dtype, id_dtype) : id_size(id_dtype);
   void* out = nullptr;
-  hipError_t e = pst::dev_alloc(&out, (n ? n : 1) * rec);
+  hipError_t e = pst::result_alloc(&out, (n ? n : 1) * rec);
   if (e != hipSuccess)
     return fail(PST_ERR_HIP, "Error in allocating array to store PointStruct search result" +
                                  dev_suffix(dev_ind, num_devs) + hipGetErrorString(e));
@@ -1306,12 +1307,12 @@ int pst_interval_parallel_search(const void* pt_arr_d, size_t n, int dtype, int 
   hipGetDevice(&dev);
   unsigned long long* ctr = device_counter(dev);
   if (!ctr) {
-    pst::dev_free(out);
+    pst::result_free(out);
     return fail(PST_ERR_HIP, "Error in allocating global result array index" + dev_suffix(dev_ind, num_devs));
   }
   e = hipMemsetAsync(ctr, 0, 8, nullptr);
   if (e != hipSuccess) {
-    pst::dev_free(out);
+    pst::result_free(out);
     return fail(PST_ERR_HIP, "Error in initialising global result array index to 0" +
                                  dev_suffix(dev_ind, num_devs) + hipGetErrorString(e));
   }
@@ -1320,7 +1321,7 @@ int pst_interval_parallel_search(const void* pt_arr_d, size_t n, int dtype, int 
   if (st.ok()) st = pst::hip_status(hipMemcpy(&h, ctr, 8, hipMemcpyDeviceToHost),
                                     "Error in copying global result array final index from device");
   if (!st.ok()) {
-    pst::dev_free(out);
+    pst::result_free(out);
     return fail(st);
   }
   *num = h;

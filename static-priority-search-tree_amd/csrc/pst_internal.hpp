@@ -122,6 +122,10 @@ hipError_t dev_alloc(U** p, size_t bytes) {
 hipError_t dev_free(void* p);
 // The same without waiting: the caller has waited for every use of p.
 hipError_t dev_free_idle(void* p);
+// Memory of results that go to the caller, who may free it by hipFree: never
+// from or into the cache.
+hipError_t result_alloc(void** p, size_t bytes);
+hipError_t result_free(void* p);
 // Waits for the work of the device that holds the block p.
 hipError_t dev_wait(const void* p);
 // Four words of pinned host memory that kernels of every device can write

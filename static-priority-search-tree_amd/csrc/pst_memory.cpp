@@ -19,6 +19,10 @@
 //     kept. When less than 1/8 of the device is free nothing large is kept.
 //   - Given back: every kept block of a device is freed when an allocation
 //     on it fails, before that allocation is tried once more.
+//   - Only the library's own blocks: results go to callers, who free them by
+//     pst_free or hipFree, so they come from hipMalloc and go by hipFree. (A
+//     kept block that a caller could free behind the cache's back would be
+//     handed out unmapped.) Up to 2 MB that pair takes 1.4 us, 64 MB 24 us.
 //   - Safe over streams: a block enters the cache only when nothing on the
 //     device can use it any more: dev_free waits for the device, as hipFree
 //     does, and dev_free_idle is for callers that have waited themselves.
@@ -136,6 +140,37 @@ void host_words_give(unsigned long long* p) {
   h.used[(p - h.page) / kHostWords] = false;
 }
 
+namespace {
+// hipMalloc on device `dev`, the current one, once more without the kept
+// blocks where it finds too little.
+hipError_t malloc_on(int dev, void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    const std::vector<void*> back = take_kept(dev);
+    if (!back.empty()) {
+      free_all(back);
+      (void)hipGetLastError();  // the failed attempt's
+      e = hipMalloc(p, bytes);
+    }
+  }
+  if (e != hipSuccess) *p = nullptr;
+  return e;
+}
+}  // namespace
+
+hipError_t result_alloc(void** p, size_t bytes) {
+  *p = nullptr;
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  return e == hipSuccess ? malloc_on(dev, p, bytes ? bytes : 1) : e;
+}
+
+hipError_t result_free(void* p) {
+  const hipError_t e = hipFree(p);
+  if (e != hipSuccess) (void)hipGetLastError();  // the caller's mistake, not the next launch's
+  return e;
+}
+
 hipError_t dev_alloc_bytes(void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 1;
@@ -155,19 +190,8 @@ hipError_t dev_alloc_bytes(void** p, size_t bytes) {
       return hipSuccess;
     }
   }
-  e = hipMalloc(p, bytes);
-  if (e == hipErrorOutOfMemory) {
-    const std::vector<void*> back = take_kept(dev);
-    if (!back.empty()) {
-      free_all(back);
-      (void)hipGetLastError();  // the failed attempt's
-      e = hipMalloc(p, bytes);
-    }
-  }
-  if (e != hipSuccess) {
-    *p = nullptr;
-    return e;
-  }
+  e = malloc_on(dev, p, bytes);
+  if (e != hipSuccess) return e;
   std::lock_guard<std::mutex> lk(c.mu);
   c.live[*p] = Block{*p, bytes, dev};
   return hipSuccess;

@@ -1,0 +1,142 @@
+// Host check of the device memory tables (csrc/pst_memory.cpp) over a stub of
+// the HIP runtime's memory calls: what is kept, handed out again and given
+// back; results that callers free themselves; waits beside a stream capture.
+// The stub refuses to free an address that is not allocated and gives freed
+// addresses out again, as the runtime does.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include <mutex>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "pst_internal.hpp"
+
+namespace {
+struct Dev {
+  size_t total = size_t{1} << 30, used = 0;
+};
+Dev g_dev[2];
+int g_cur = 0;
+std::map<char*, std::pair<size_t, int>> g_mem;  // allocations: bytes, device
+std::map<size_t, std::vector<char*>> g_free[2];  // freed addresses by size, reused last first
+char* g_next = reinterpret_cast<char*>(size_t{1} << 40);
+int g_waits = 0;          // hipFree calls that worked: each waits for the device
+bool g_capturing = false;  // some stream is being captured (relaxed)
+bool g_capture_broken = false;
+int g_fail_host = 0;       // hipHostMalloc calls that fail
+hipError_t g_last = hipSuccess;
+std::mutex g_mu;
+hipError_t set_last(hipError_t e) {
+  if (e != hipSuccess) g_last = e;
+  return e;
+}
+bool allocated(void* p) { return g_mem.count(static_cast<char*>(p)) != 0; }
+}  // namespace
+
+extern "C" {
+hipError_t hipGetDevice(int* d) { return *d = g_cur, hipSuccess; }
+hipError_t hipSetDevice(int d) { return g_cur = d, hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  Dev& d = g_dev[g_cur];
+  if (n > d.total - d.used) return set_last(hipErrorOutOfMemory);
+  auto& f = g_free[g_cur][n];
+  char* a = g_next;
+  if (!f.empty()) a = f.back(), f.pop_back();
+  else g_next += n + 4096;
+  g_mem[a] = {n, g_cur};
+  d.used += n;
+  *p = a;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  if (!p) return hipSuccess;
+  auto it = g_mem.find(static_cast<char*>(p));
+  if (it == g_mem.end()) return set_last(hipErrorInvalidValue);
+  g_dev[it->second.second].used -= it->second.first;
+  g_free[it->second.second][it->second.first].push_back(it->first);
+  g_mem.erase(it);
+  g_waits++;
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() {
+  if (g_capturing) return g_capture_broken = true, hipErrorStreamCaptureUnsupported;
+  return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t* f, size_t* t) {
+  *f = g_dev[g_cur].total - g_dev[g_cur].used;
+  *t = g_dev[g_cur].total;
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (g_fail_host > 0) return g_fail_host--, set_last(hipErrorOutOfMemory);
+  *p = std::calloc(1, n);
+  return hipSuccess;
+}
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
+}
+
+namespace {
+int g_bad = 0;
+void check(bool ok, const char* what, int line) {
+  if (ok) return;
+  g_bad++;
+  std::printf("FAILED line %d: %s\n", line, what);
+}
+#define CHECK(x) check((x), #x, __LINE__)
+
+void* take(size_t n) {
+  void* p = nullptr;
+  CHECK(pst::dev_alloc(&p, n) == hipSuccess);
+  CHECK(allocated(p));
+  return p;
+}
+
+// A result freed twice, or by hipFree and then pst_free, is refused as hipFree
+// refuses it, and the memory handed out afterwards is allocated.
+void results() {
+  constexpr size_t n = 1 << 20;
+  for (int how = 0; how < 4; how++) {
+    void* r = nullptr;
+    CHECK(pst::result_alloc(&r, n) == hipSuccess);
+    const hipError_t first = how & 1 ? hipFree(r) : pst::result_free(r);
+    const hipError_t second = how & 2 ? hipFree(r) : pst::result_free(r);
+    CHECK(first == hipSuccess);
+    CHECK(second != hipSuccess);
+    CHECK((how & 2) || hipGetLastError() == hipSuccess);
+    void* a = take(n);
+    void* b = take(n);
+    CHECK(a != b);
+    CHECK(pst::dev_free(a) == hipSuccess && pst::dev_free(b) == hipSuccess);
+    (void)hipGetLastError();
+  }
+  // another owner's block of another size at a freed result's address
+  void* r = nullptr;
+  CHECK(pst::result_alloc(&r, 2 * n) == hipSuccess);
+  CHECK(hipFree(r) == hipSuccess);
+  g_free[0][n / 2].push_back(static_cast<char*>(r));
+  void* other = nullptr;
+  CHECK(hipMalloc(&other, n / 2) == hipSuccess && other == r);
+  CHECK(pst::result_free(other) == hipSuccess);
+  CHECK(!allocated(other));
+  void* big = take(2 * n);
+  CHECK(g_mem[static_cast<char*>(big)].first == 2 * n);
+  CHECK(pst::dev_free(big) == hipSuccess);
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::string only = argc > 1 ? argv[1] : "";
+  if (only.empty() || only == "results") results();
+  std::printf(g_bad ? "%d checks failed\n" : "MEMORY OK\n", g_bad);
+  return g_bad != 0;
+}

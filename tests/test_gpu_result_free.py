@@ -1,0 +1,32 @@
+"""Results of blocking searches belong to the caller, who frees them once, by
+pst_free: a second free is an error, as the runtime's is, and what the library
+allocates and searches afterwards is unharmed by it."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle as O
+from test_gpu_forest import P, torch  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def test_second_free_is_refused(torch, P):  # noqa: F811
+    import pst_data as D
+    pts = D.interval_points(300_000, seed=9)
+    d = P.to_device(pts)
+    q = np.array([0.5], np.float32)
+    want = np.sort(pts["id"][O.brute_force(pts, O.LEFT, 0, q[0], q[0])])
+    L = P.lib()
+    for _ in range(3):
+        tr = P.StaticPSTGPU(d, len(pts), "f32", "u32")
+        num, ptr = ctypes.c_size_t(), ctypes.c_void_p()
+        P._check(L.pst_gpu_two_sided_left_search(tr.h, P.RET_ID, ctypes.byref(num), ctypes.byref(ptr), q.ctypes.data,
+                                                 q.ctypes.data))
+        assert np.array_equal(np.sort(P._d2h(ptr.value, num.value * 4).view(np.uint32)), want)
+        assert L.pst_free(ptr) == 0
+        assert L.pst_free(ptr) == 2  # PST_ERR_HIP
+        tr.set_level_index(True)
+        assert np.array_equal(np.sort(tr.twoSidedLeftSearch(q[0], q[0])), want)
+        tr.close()

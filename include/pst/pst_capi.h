@@ -104,7 +104,9 @@ int pst_free(void* res_arr_d);
 int pst_gpu_create(const void* pt_arr_d, size_t num_elems, int dtype, int id_dtype,
                    int warp_multiplier, int dev_ind, int num_devs, pst_stream_t stream,
                    pst_tree** out);
-/* Replaces ~StaticPSTGPU (pst/static-pst-gpu.h:80-88). */
+/* Replaces ~StaticPSTGPU (pst/static-pst-gpu.h:80-88). Waits for the device's
+ * work; allowed beside a stream capture wherever hipFree is. Where that is
+ * refused (PST_ERR_HIP), the handle stays as it is. */
 int pst_gpu_destroy(pst_tree* tree);
 /* Getters (pst/static-pst-gpu.h:96-98) and sizes; the dtype getters have
  * no counterpart (the reference's types are template parameters). */

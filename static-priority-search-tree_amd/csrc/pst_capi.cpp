@@ -407,15 +407,18 @@ int pst_gpu_destroy(pst_tree* t) {
   if (!t) return PST_OK;
   if (t->graphs > 0)
     return fail(PST_ERR_INVALID, "Error: the tree still has batch graphs; destroy them before the tree");
-  // one wait for the device's work, then every array goes back
-  hipError_t e = t->nodes ? pst::dev_wait(t->nodes) : hipSuccess;
-  const bool idle = e == hipSuccess;
-  for (void* p : {t->nodes, t->submin, t->ids, t->tree_bounds, t->lv_key, t->lv_id}) {
-    const hipError_t e2 = idle ? pst::dev_free_idle(p) : pst::dev_free(p);
+  // one wait for the device's work (refused: the handle stays as it is), then
+  // every other array goes back
+  hipError_t e = t->nodes ? pst::dev_free(t->nodes) : hipSuccess;
+  if (e != hipSuccess)
+    return fail(PST_ERR_HIP, "Error in freeing array storing priority search tree" + dev_suffix(t->dev_ind, t->num_devs) +
+                                 hipGetErrorString(e));
+  for (void* p : {t->submin, t->ids, t->tree_bounds, t->lv_key, t->lv_id}) {
+    const hipError_t e2 = pst::dev_free_idle(p);
     if (e == hipSuccess) e = e2;
   }
-  pst::scratch_release(t->sc, idle);
-  pst::level_scratch_release(t->lsc, idle);
+  pst::scratch_release(t->sc, true);
+  pst::level_scratch_release(t->lsc, true);
   pst::host_words_give(t->host);
   const int di = t->dev_ind, nd = t->num_devs;
   delete t;

@@ -24,8 +24,8 @@
 //     kept block that a caller could free behind the cache's back would be
 //     handed out unmapped.) Up to 2 MB that pair takes 1.4 us, 64 MB 24 us.
 //   - Safe over streams: a block enters the cache only when nothing on the
-//     device can use it any more: dev_free waits for the device, as hipFree
-//     does, and dev_free_idle is for callers that have waited themselves.
+//     device can use it any more: dev_free waits for the device, by a hipFree,
+//     and dev_free_idle is for callers that have waited themselves.
 //   - Safe over threads: one mutex guards the tables; no HIP call that waits
 //     is made under it.
 // Blocks hold what their last user left; no caller may expect zeros.
@@ -248,6 +248,10 @@ hipError_t dev_free_idle(void* p) {
   return hipSuccess;
 }
 
+// The wait is a hipFree of eight bytes, which waits for every stream of the
+// device and for running graphs. hipDeviceSynchronize would break a capture
+// that any thread has running, also a relaxed one; a free does not (1.4 us on
+// an idle device, with the allocation).
 hipError_t dev_wait(const void* p) {
   Cache& c = cache();
   int dev = -1, cur = 0;
@@ -259,16 +263,38 @@ hipError_t dev_wait(const void* p) {
   if (dev < 0) return hipSuccess;  // hipFree waits by itself
   hipError_t e = hipGetDevice(&cur);
   if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
-  if (e == hipSuccess) e = hipDeviceSynchronize();
+  void* token = nullptr;
+  if (e == hipSuccess) e = malloc_on(dev, &token, 8);
+  if (e == hipSuccess) e = hipFree(token);
   if (cur != dev) (void)hipSetDevice(cur);
+  if (e != hipSuccess) (void)hipGetLastError();
   return e;
 }
 
 hipError_t dev_free(void* p) {
   if (!p) return hipSuccess;
-  const hipError_t e = dev_wait(p);
-  if (e != hipSuccess) return e;
-  return dev_free_idle(p);
+  if (dev_wait(p) == hipSuccess) return dev_free_idle(p);
+  // no wait to be had: the block's own hipFree waits, or refuses, and then
+  // the block stays the caller's
+  Cache& c = cache();
+  Block b{};
+  bool known = false;
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    auto it = c.live.find(p);
+    known = it != c.live.end();
+    if (known) {
+      b = it->second;
+      c.live.erase(it);
+    }
+  }
+  const hipError_t e = hipFree(p);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lk(c.mu);
+    if (known) c.live[p] = b;
+  }
+  return e;
 }
 
 }  // namespace pst

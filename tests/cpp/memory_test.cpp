@@ -27,6 +27,7 @@ char* g_next = reinterpret_cast<char*>(size_t{1} << 40);
 int g_waits = 0;          // hipFree calls that worked: each waits for the device
 bool g_capturing = false;  // some stream is being captured (relaxed)
 bool g_capture_broken = false;
+bool g_refused = false;    // some stream is being captured in global mode: no call that may wait
 int g_fail_host = 0;       // hipHostMalloc calls that fail
 hipError_t g_last = hipSuccess;
 std::mutex g_mu;
@@ -42,6 +43,7 @@ hipError_t hipGetDevice(int* d) { return *d = g_cur, hipSuccess; }
 hipError_t hipSetDevice(int d) { return g_cur = d, hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) {
   std::lock_guard<std::mutex> lk(g_mu);
+  if (g_refused) return set_last(hipErrorStreamCaptureUnsupported);
   Dev& d = g_dev[g_cur];
   if (n > d.total - d.used) return set_last(hipErrorOutOfMemory);
   auto& f = g_free[g_cur][n];
@@ -56,6 +58,7 @@ hipError_t hipMalloc(void** p, size_t n) {
 hipError_t hipFree(void* p) {
   std::lock_guard<std::mutex> lk(g_mu);
   if (!p) return hipSuccess;
+  if (g_refused) return set_last(hipErrorStreamCaptureUnsupported);
   auto it = g_mem.find(static_cast<char*>(p));
   if (it == g_mem.end()) return set_last(hipErrorInvalidValue);
   g_dev[it->second.second].used -= it->second.first;
@@ -132,11 +135,47 @@ void results() {
   CHECK(g_mem[static_cast<char*>(big)].first == 2 * n);
   CHECK(pst::dev_free(big) == hipSuccess);
 }
+
+// Frees beside a capture neither break it nor lose the block; every block is
+// waited for before it can be handed out again.
+void captures() {
+  constexpr size_t n = 3 << 20;
+  void* a = take(n);
+  g_capturing = true;
+  const int before = g_waits;
+  CHECK(pst::dev_free(a) == hipSuccess);
+  CHECK(!g_capture_broken);
+  CHECK(g_waits > before);
+  void* b = take(n);
+  CHECK(b == a);  // it was kept
+  CHECK(pst::dev_wait(b) == hipSuccess);
+  CHECK(pst::dev_free_idle(b) == hipSuccess);
+  CHECK(!g_capture_broken);
+  g_capturing = false;
+  // refused outright: an error, the block stays the caller's and goes later
+  void* c = take(2 * n);
+  g_refused = true;
+  CHECK(pst::dev_wait(c) != hipSuccess);
+  CHECK(pst::dev_free(c) != hipSuccess);
+  g_refused = false;
+  CHECK(hipGetLastError() == hipSuccess);
+  CHECK(allocated(c));
+  void* d = take(2 * n);
+  CHECK(d != c);
+  CHECK(pst::dev_free(c) == hipSuccess && pst::dev_free(d) == hipSuccess);
+  // a block of another device is waited for there
+  g_cur = 1;
+  void* e = take(n);
+  g_cur = 0;
+  CHECK(pst::dev_free(e) == hipSuccess);
+  CHECK(g_cur == 0);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string only = argc > 1 ? argv[1] : "";
   if (only.empty() || only == "results") results();
+  if (only.empty() || only == "captures") captures();
   std::printf(g_bad ? "%d checks failed\n" : "MEMORY OK\n", g_bad);
   return g_bad != 0;
 }

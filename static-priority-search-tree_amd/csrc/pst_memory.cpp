@@ -106,7 +106,6 @@ constexpr int kHostSlots = 128, kHostWords = 4;
 struct HostPage {
   std::mutex mu;
   unsigned long long* page = nullptr;
-  bool failed = false;
   bool used[kHostSlots] = {};
 };
 HostPage& host_page() {
@@ -117,12 +116,12 @@ HostPage& host_page() {
 unsigned long long* host_words_take() {
   HostPage& h = host_page();
   std::lock_guard<std::mutex> lk(h.mu);
-  if (!h.page && !h.failed) {
+  if (!h.page) {
     void* p = nullptr;
     if (hipHostMalloc(&p, kHostSlots * kHostWords * 8, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess)
       h.page = static_cast<unsigned long long*>(p);
-    else
-      h.failed = true;
+    else  // refused for now (a capture in global mode, say): the caller copies its results
+      (void)hipGetLastError();
   }
   if (!h.page) return nullptr;
   for (int k = 0; k < kHostSlots; k++)

@@ -9,6 +9,7 @@
 #include <cstdlib>
 #include <map>
 #include <mutex>
+#include <set>
 #include <string>
 #include <thread>
 #include <vector>
@@ -170,12 +171,29 @@ void captures() {
   CHECK(pst::dev_free(e) == hipSuccess);
   CHECK(g_cur == 0);
 }
+
+// The pinned words: a failed allocation (as beside a global capture) leaves no
+// error for the next launch check and is tried again; slots are distinct,
+// bounded and given back.
+void host_words() {
+  g_fail_host = 1;
+  CHECK(pst::host_words_take() == nullptr);
+  CHECK(hipGetLastError() == hipSuccess);
+  std::set<unsigned long long*> got;
+  while (unsigned long long* w = pst::host_words_take()) got.insert(w);
+  CHECK(got.size() == 128);
+  for (auto it = got.begin(); it != got.end() && std::next(it) != got.end(); ++it) CHECK(*std::next(it) - *it >= 4);
+  pst::host_words_give(*got.begin());
+  CHECK(pst::host_words_take() == *got.begin());
+  for (unsigned long long* w : got) pst::host_words_give(w);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string only = argc > 1 ? argv[1] : "";
   if (only.empty() || only == "results") results();
   if (only.empty() || only == "captures") captures();
+  if (only.empty() || only == "host_words") host_words();
   std::printf(g_bad ? "%d checks failed\n" : "MEMORY OK\n", g_bad);
   return g_bad != 0;
 }

@@ -91,6 +91,11 @@ const char* pst_last_error(void);
 size_t pst_point_size(int dtype, int id_dtype);
 /* Releases a result array returned by a blocking search. */
 int pst_free(void* res_arr_d);
+/* Gives the device memory that the library keeps for later calls (blocks of
+ * destroyed trees and of construction, at most 1/32 of each device's memory)
+ * back to the runtime. The library does so itself when one of its own
+ * allocations fails; call it when another allocator needs the room. */
+int pst_release_cached_memory(void);
 
 /* ------------------------------------------------------------------ */
 /* StaticPSTGPU (pst/static-pst-gpu.h:72-477)                          */

@@ -90,7 +90,7 @@ unsigned long long* device_counter(int dev) {
   auto it = g_ctr.find(dev);
   if (it != g_ctr.end()) return it->second;
   unsigned long long* p = nullptr;
-  if (hipMalloc(&p, sizeof(unsigned long long)) != hipSuccess) return nullptr;
+  if (pst::result_alloc(&p, sizeof(unsigned long long)) != hipSuccess) return nullptr;
   g_ctr[dev] = p;
   return p;
 }
@@ -352,6 +352,11 @@ int pst_free(void* p) {
   if (!p) return PST_OK;
   hipError_t e = pst::result_free(p);
   if (e != hipSuccess) return fail(pst::hip_status(e, "Error in freeing search result array"));
+  return PST_OK;
+}
+
+int pst_release_cached_memory(void) {
+  pst::dev_release_kept();
   return PST_OK;
 }
 
@@ -1192,19 +1197,18 @@ int surface_blocking(IsoCountFn cfn, IsoWriteFn wfn, const void* vertex_arr_d, i
                          "Error in reading the triangle count");
   if (st.ok()) st = pst::hip_status(hipMemcpy(&bad, err, 8, hipMemcpyDeviceToHost), "Error in reading the error flag");
   if (st.ok() && bad) st = Status{PST_ERR_INVALID, "Error: a metacell ID lies past the metacell grid"};
-  void* tri = nullptr;
+  float* tri = nullptr;
   if (st.ok() && total)
     st = pst::hip_status(pst::result_alloc(&tri, total * 9 * sizeof(float)), "Error in allocating the triangle array");
   if (st.ok() && total)
-    st = wfn(dtype, id_dtype, vertex_arr_d, p32, m32, metacell_ids_d, num_ids, isovalue, offsets, total,
-             static_cast<float*>(tri), nullptr);
+    st = wfn(dtype, id_dtype, vertex_arr_d, p32, m32, metacell_ids_d, num_ids, isovalue, offsets, total, tri, nullptr);
   if (st.ok()) st = pst::hip_status(hipStreamSynchronize(nullptr), "Error in synchronising after isosurface extraction");
   pst::dev_free(counts);
   if (!st.ok()) {
     if (tri) pst::result_free(tri);
     return fail(st);
   }
-  *triangles_d = static_cast<float*>(tri);
+  *triangles_d = tri;
   *num_triangles = total;
   return PST_OK;
 }

@@ -122,9 +122,19 @@ hipError_t dev_alloc(U** p, size_t bytes) {
 hipError_t dev_free(void* p);
 // The same without waiting: the caller has waited for every use of p.
 hipError_t dev_free_idle(void* p);
-// Memory of results that go to the caller, who may free it by hipFree: never
-// from or into the cache.
-hipError_t result_alloc(void** p, size_t bytes);
+// Gives every kept block of every device back to the runtime.
+void dev_release_kept();
+// Memory that is never from or in the cache: results, which the caller may
+// free by hipFree, and a server's buffers. An allocation that finds too little
+// is tried again once the kept blocks are given back.
+hipError_t result_alloc_bytes(void** p, size_t bytes);
+template <typename U>
+hipError_t result_alloc(U** p, size_t bytes) {
+  void* v = nullptr;
+  const hipError_t e = result_alloc_bytes(&v, bytes);
+  *p = static_cast<U*>(v);
+  return e;
+}
 hipError_t result_free(void* p);
 // Waits for the work of the device that holds the block p.
 hipError_t dev_wait(const void* p);

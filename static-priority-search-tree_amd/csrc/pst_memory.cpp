@@ -18,7 +18,8 @@
 //     least recently freed blocks leave first, and larger blocks are never
 //     kept. When less than 1/8 of the device is free nothing large is kept.
 //   - Given back: every kept block of a device is freed when an allocation
-//     on it fails, before that allocation is tried once more.
+//     on it fails, before that allocation is tried once more, and all of them
+//     on request (dev_release_kept), for other allocators of the program.
 //   - Only the library's own blocks: results go to callers, who free them by
 //     pst_free or hipFree, so they come from hipMalloc and go by hipFree. (A
 //     kept block that a caller could free behind the cache's back would be
@@ -139,6 +140,16 @@ void host_words_give(unsigned long long* p) {
   h.used[(p - h.page) / kHostWords] = false;
 }
 
+void dev_release_kept() {
+  std::vector<int> devs;
+  {
+    Cache& c = cache();
+    std::lock_guard<std::mutex> lk(c.mu);
+    for (const auto& k : c.kept_bytes) devs.push_back(k.first);
+  }
+  for (int d : devs) free_all(take_kept(d));
+}
+
 namespace {
 // hipMalloc on device `dev`, the current one, once more without the kept
 // blocks where it finds too little.
@@ -157,7 +168,7 @@ hipError_t malloc_on(int dev, void** p, size_t bytes) {
 }
 }  // namespace
 
-hipError_t result_alloc(void** p, size_t bytes) {
+hipError_t result_alloc_bytes(void** p, size_t bytes) {
   *p = nullptr;
   int dev = 0;
   const hipError_t e = hipGetDevice(&dev);
@@ -165,6 +176,7 @@ hipError_t result_alloc(void** p, size_t bytes) {
 }
 
 hipError_t result_free(void* p) {
+  if (!p) return hipSuccess;
   const hipError_t e = hipFree(p);
   if (e != hipSuccess) (void)hipGetLastError();  // the caller's mistake, not the next launch's
   return e;

@@ -28,7 +28,7 @@ RET_ID, RET_POINT = 0, 1
 ERR_CAPACITY = 4
 
 EXPORTED = [
-    "pst_last_error", "pst_point_size", "pst_free",
+    "pst_last_error", "pst_point_size", "pst_free", "pst_release_cached_memory",
     "pst_gpu_create", "pst_gpu_destroy", "pst_gpu_num_elems", "pst_gpu_dev_ind",
     "pst_gpu_num_devs", "pst_gpu_three_sided_search", "pst_gpu_two_sided_left_search",
     "pst_gpu_two_sided_right_search", "pst_gpu_search_into", "pst_gpu_calc_global_mem_needed",
@@ -208,6 +208,12 @@ def to_device(arr: np.ndarray, device="cuda"):
     import torch
     b = np.ascontiguousarray(arr).view(np.uint8).reshape(-1)
     return torch.from_numpy(b.copy()).to(device)
+
+
+def release_cached_memory():
+    """Give the device memory that the library keeps for later calls back
+    (pst_release_cached_memory)."""
+    _check(lib().pst_release_cached_memory())
 
 
 class StaticPSTGPU:

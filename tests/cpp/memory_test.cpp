@@ -14,6 +14,7 @@
 #include <thread>
 #include <vector>
 
+#include "pst_capi.h"
 #include "pst_internal.hpp"
 
 namespace {
@@ -81,6 +82,23 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   if (g_fail_host > 0) return g_fail_host--, set_last(hipErrorOutOfMemory);
   *p = std::calloc(1, n);
   return hipSuccess;
+}
+hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = nullptr, hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = nullptr, hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
+// the tree calls that a server makes when it is created
+int pst_gpu_dtype(const pst_tree*) { return PST_F32; }
+int pst_gpu_id_dtype(const pst_tree*) { return PST_U32; }
+size_t pst_point_size(int, int) { return 12; }
+const char* pst_last_error(void) { return ""; }
+int pst_gpu_batch_count(pst_tree*, const void*, size_t, unsigned long long*, pst_stream_t) { return PST_OK; }
+int pst_gpu_batch_write(pst_tree*, const void*, size_t, int, const unsigned long long*, const unsigned long long*, void*,
+                        pst_stream_t) {
+  return PST_OK;
 }
 hipError_t hipGetLastError() {
   const hipError_t e = g_last;
@@ -187,6 +205,113 @@ void host_words() {
   CHECK(pst::host_words_take() == *got.begin());
   for (unsigned long long* w : got) pst::host_words_give(w);
 }
+
+size_t used(int dev) { return g_dev[dev].used; }
+
+// Kept blocks make room for a server's buffers where the device is full.
+void server() {
+  std::vector<void*> keep;
+  for (int k = 0; k < 8; k++) keep.push_back(take(3 << 20));
+  for (void* p : keep) CHECK(pst::dev_free(p) == hipSuccess);
+  void* rest = nullptr;
+  CHECK(hipMalloc(&rest, g_dev[0].total - used(0) - (4 << 20)) == hipSuccess);
+  int dummy = 0;
+  pst_tree* tree = reinterpret_cast<pst_tree*>(&dummy);
+  pst_server* s = nullptr;
+  CHECK(pst_server_create(&tree, 1, 10 << 20, 64, &s) == PST_OK);
+  if (s) CHECK(pst_server_destroy(s) == PST_OK);
+  CHECK(hipFree(rest) == hipSuccess);
+  (void)hipGetLastError();
+}
+
+// The cache's bounds: at most 1/32 of the device, the least recently freed
+// blocks leave first, larger blocks are never kept, nothing large on a nearly
+// full device, each device its own; everything given back on request and where
+// an allocation fails, which is then tried once more.
+void bounds() {
+  pst::dev_release_kept();
+  const size_t base = used(0), base1 = used(1), limit = g_dev[0].total / 32;
+  const size_t n = limit / 4 - 4096;  // four of them fit
+  std::vector<void*> p;
+  for (int k = 0; k < 6; k++) p.push_back(take(n + 16 * k));
+  for (void* x : p) {
+    CHECK(pst::dev_free(x) == hipSuccess);
+    size_t held = used(0) - base;
+    for (void* y : p) held -= allocated(y) && y > x ? g_mem[static_cast<char*>(y)].first : 0;
+    CHECK(held <= limit);
+  }
+  CHECK(!allocated(p[0]) && !allocated(p[1]));
+  for (int k = 2; k < 6; k++) CHECK(allocated(p[k]));
+  CHECK(take(n + 16 * 3) == p[3]);  // exactly its size
+  void* fresh = take(n + 16 * 3);
+  CHECK(fresh != p[2] && fresh != p[4] && fresh != p[5]);
+  CHECK(pst::dev_free(fresh) == hipSuccess && pst::dev_free(p[3]) == hipSuccess);
+  void* big = take(limit + 1);
+  CHECK(pst::dev_free(big) == hipSuccess);
+  CHECK(!allocated(big));
+  g_cur = 1;
+  void* other = take(n);
+  CHECK(pst::dev_free(other) == hipSuccess);
+  CHECK(allocated(other) && used(1) == base1 + n);
+  g_cur = 0;
+  // an allocation that fails gives back this device's blocks alone
+  void* rest = nullptr;
+  CHECK(used(0) > base);
+  CHECK(pst::dev_alloc(&rest, g_dev[0].total - base - 4096) == hipSuccess);
+  CHECK(used(0) == g_dev[0].total - 4096 && used(1) == base1 + n);
+  void* no = nullptr;
+  CHECK(pst::dev_alloc(&no, 1 << 20) == hipErrorOutOfMemory && no == nullptr);
+  CHECK(hipGetLastError() == hipErrorOutOfMemory);  // as hipMalloc leaves it
+  CHECK(pst::dev_free(rest) == hipSuccess);
+  CHECK(!allocated(rest));
+  // on request: every device's
+  void* a = take(n);
+  CHECK(pst::dev_free(a) == hipSuccess && allocated(a));
+  pst::dev_release_kept();
+  CHECK(used(0) == base && used(1) == base1);
+  // a block of 32 MB and more is not kept while less than 1/8 is free
+  g_dev[0].total = size_t{4} << 30;
+  void* fill = nullptr;
+  CHECK(hipMalloc(&fill, (size_t{4} << 30) - (size_t{300} << 20)) == hipSuccess);
+  g_dev[1].total = size_t{4} << 30;
+  void* l = take(size_t{32} << 20);
+  CHECK(pst::dev_free(l) == hipSuccess);
+  CHECK(!allocated(l));
+  CHECK(hipFree(fill) == hipSuccess);
+  l = take(size_t{32} << 20);
+  CHECK(pst::dev_free(l) == hipSuccess);
+  CHECK(allocated(l));
+  pst::dev_release_kept();
+  CHECK(used(0) == base);
+}
+
+// Threads take and free blocks of the same sizes: no block is held twice, and
+// all of them are given back.
+void threads() {
+  pst::dev_release_kept();
+  const size_t base = used(0);
+  std::mutex mu;
+  std::set<void*> held;
+  auto work = [&](unsigned seed) {
+    for (int r = 0; r < 3000; r++) {
+      seed = seed * 1664525u + 1013904223u;
+      void* p = nullptr;
+      const bool ok = pst::dev_alloc(&p, 4096u * (1 + (seed >> 28))) == hipSuccess;
+      {
+        std::lock_guard<std::mutex> lk(mu);
+        CHECK(ok && held.insert(p).second);
+      }
+      std::lock_guard<std::mutex> lk(mu);
+      held.erase(p);
+      CHECK(pst::dev_free(p) == hipSuccess);
+    }
+  };
+  std::vector<std::thread> ts;
+  for (unsigned k = 0; k < 4; k++) ts.emplace_back(work, k + 1);
+  for (auto& t : ts) t.join();
+  pst::dev_release_kept();
+  CHECK(used(0) == base);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -194,6 +319,9 @@ int main(int argc, char** argv) {
   if (only.empty() || only == "results") results();
   if (only.empty() || only == "captures") captures();
   if (only.empty() || only == "host_words") host_words();
+  if (only.empty() || only == "server") server();
+  if (only.empty() || only == "bounds") bounds();
+  if (only.empty() || only == "threads") threads();
   std::printf(g_bad ? "%d checks failed\n" : "MEMORY OK\n", g_bad);
   return g_bad != 0;
 }

@@ -30,3 +30,23 @@ def test_second_free_is_refused(torch, P):  # noqa: F811
         tr.set_level_index(True)
         assert np.array_equal(np.sort(tr.twoSidedLeftSearch(q[0], q[0])), want)
         tr.close()
+
+
+def test_cached_memory_is_given_back(torch, P):  # noqa: F811
+    import pst_data as D
+    n = 3_000_000
+    pts = D.interval_points(n, seed=8)
+    d = P.to_device(pts)
+    P.release_cached_memory()
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    for _ in range(2):
+        tr = P.StaticPSTGPU(d, n, "f32", "u32")
+        q = np.float32(0.3)
+        assert np.array_equal(np.sort(tr.twoSidedLeftSearch(q, q)), np.sort(pts["id"][O.brute_force(pts, O.LEFT, 0, q, q)]))
+        tr.close()
+        kept = free0 - torch.cuda.mem_get_info()[0]
+        P.release_cached_memory()
+        left = free0 - torch.cuda.mem_get_info()[0]
+        print(f"kept {kept}, left after the release {left}", flush=True)
+        assert kept > 24 * n and left < (8 << 20)

@@ -8,7 +8,7 @@ import pytest
 BIN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "_build", "memory_test")
 
 
-@pytest.mark.parametrize("part", ["results", "captures", "host_words"])
+@pytest.mark.parametrize("part", ["results", "captures", "host_words", "server", "bounds", "threads"])
 def test_memory_tables(part):
     assert os.path.exists(BIN), "tests/cpp/_build/memory_test is not built (run __graft_entry__.build())"
     r = subprocess.run([BIN, part], capture_output=True, text=True, timeout=60)

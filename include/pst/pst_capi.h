@@ -150,10 +150,10 @@ int pst_gpu_search_into(pst_tree* tree, int kind, int ret, const void* min_dim1_
 /* Replaces StaticPSTGPU::calcGlobalMemNeeded(num_elems)
  * (pst/static-pst-gpu.h:132, pst/static-pst-gpu.tu:646-671): bytes of
  * device memory a tree needs: its resident arrays (node records, subtree
- * minima, IDs), construction's buffers (kept, within 1/32 of the device's
- * memory, for the next construction of this size) and one blocking search
- * (the handle's search buffers, kept, and a result array of num_elems
- * points). A level index, built on request, adds
+ * minima, IDs) plus the larger of construction's buffers and one blocking
+ * search (the handle's search buffers, kept, and a result array of num_elems
+ * points) beside what the library keeps of construction's buffers (at most
+ * 1/32 of the device's memory). A level index, built on request, adds
  * pst_gpu_level_index_bytes on top. */
 size_t pst_gpu_calc_global_mem_needed(size_t num_elems, int dtype, int id_dtype);
 

@@ -591,7 +591,7 @@ size_t pst_gpu_calc_global_mem_needed(size_t n, int dtype, int id_dtype) {
   const size_t S = slots_for(n);
   // resident: node records, subtree minima and the per-slot ID array
   const size_t tree = S * (pst::node_size(dtype, id_dtype) + pst::dtype_size(dtype) + id_size(id_dtype));
-  // construction's buffers, kept for the next construction of this size
+  // construction's buffers
   const size_t construct = pst::build_scratch_bytes(dtype, id_dtype, n);
   // one blocking search: the handle's search buffers (kept) and a result
   // array of n points (the reference's allocation, pst/static-pst-gpu.tu:563)
@@ -599,7 +599,9 @@ size_t pst_gpu_calc_global_mem_needed(size_t n, int dtype, int id_dtype) {
   hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
   const size_t search = pst::search_scratch_bytes(n, dtype, cus) + n * pst::point_size(dtype, id_dtype);
-  return tree + construct + search;
+  // of construction's buffers a search finds kept what the library's cache
+  // holds at most (on a machine without a device, that of a 288 GB one)
+  return tree + std::max(construct, std::min(construct, pst::dev_keep_limit()) + search);
 }
 
 size_t pst_gpu_arr_calc_global_mem_needed(size_t n, unsigned threads_per_block, int dtype, int id_dtype) {

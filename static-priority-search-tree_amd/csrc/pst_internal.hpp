@@ -122,6 +122,8 @@ hipError_t dev_alloc(U** p, size_t bytes) {
 hipError_t dev_free(void* p);
 // The same without waiting: the caller has waited for every use of p.
 hipError_t dev_free_idle(void* p);
+// Bytes the cache keeps at most on the current device.
+size_t dev_keep_limit();
 // Gives every kept block of every device back to the runtime.
 void dev_release_kept();
 // Memory that is never from or in the cache: results, which the caller may

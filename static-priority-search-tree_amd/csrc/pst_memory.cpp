@@ -44,6 +44,7 @@ namespace pst {
 namespace {
 
 constexpr size_t kLargeBlock = size_t{32} << 20;
+constexpr size_t kKeepShare = 32;  // of a device's memory at most one part in so many is kept
 
 struct Block {
   void* p;
@@ -140,6 +141,12 @@ void host_words_give(unsigned long long* p) {
   h.used[(p - h.page) / kHostWords] = false;
 }
 
+size_t dev_keep_limit() {
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) total_b = size_t{288} << 30;
+  return total_b / kKeepShare;
+}
+
 void dev_release_kept() {
   std::vector<int> devs;
   {
@@ -234,7 +241,7 @@ hipError_t dev_free_idle(void* p) {
     if (ok) ok = hipMemGetInfo(&free_b, &total_b) == hipSuccess;
     if (cur != b.dev) (void)hipSetDevice(cur);
     if (!ok) return hipFree(p);
-    limit = total_b / 32;
+    limit = total_b / kKeepShare;
     if (b.bytes >= kLargeBlock && free_b < total_b / 8) return hipFree(p);
   }
   if (b.bytes > limit) return hipFree(p);

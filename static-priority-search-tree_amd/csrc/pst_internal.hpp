@@ -237,6 +237,14 @@ Status build_forest_bounds(int dtype, int id_dtype, size_t n, size_t slots_per_t
 // Device bytes of the index: bit_length(n) levels of n (key, ID) pairs,
 // each level padded to a multiple of 64 pairs.
 size_t level_index_bytes(int dtype, int id_dtype, size_t n);
+// Elements from one level to the next.
+inline size_t level_stride(size_t n) { return (n + 63) & ~size_t{63}; }
+// Construction's two slot arrays (4 B per point) in one block: the second's
+// first element, and the bytes of both.
+struct LevelSlots {
+  size_t second, bytes;
+};
+inline LevelSlots level_slots(size_t n) { return LevelSlots{level_stride(n), 2 * level_stride(n) * 4}; }
 // Builds the index of a deep tree with IDs (ids_d: ID per slot) into key_d
 // (unsigned keys of the tree's dtype width) and id_d (blocking).
 Status build_level_index(int dtype, int id_dtype, size_t n, const void* nodes_d, const void* ids_d, void* key_d,

@@ -74,11 +74,9 @@ constexpr uint32_t kFlat = 4096;  // positions per flat pass of the copy (16 per
 template <typename T>
 using key_of = decltype(ord_key(T{}));
 
-__host__ __device__ inline uint64_t level_stride(uint64_t n) { return (n + 63) & ~63ull; }
-
 // The kLvPer consecutive elements from a[base] (zeros past nt): aligned
 // 16-byte loads when all are in range (base is a multiple of kLvPer and
-// every level starts 256-byte aligned).
+// every level and slot array starts 256-byte aligned, level_stride).
 template <typename V>
 __device__ inline void load_run(const V* __restrict__ a, uint32_t base, uint32_t nt, V (&v)[kLvPer]) {
   if (base + kLvPer <= nt) {
@@ -948,16 +946,17 @@ Status build_level_index(int dtype, int id_dtype, size_t n, const void* nodes_d,
       // size used and gave back. The sort of level 0 works in the key array's
       // deeper levels, which are written after it, where they hold it.
       const size_t slots = build_arena_bytes(dtype, id_dtype, n);
-      const bool inside = H >= 2 && ns * sizeof(K) * (H - 2) >= tmp_bytes && n * 8 <= slots;
+      const LevelSlots ls = level_slots(n);
+      const bool inside = H >= 2 && ns * sizeof(K) * (H - 2) >= tmp_bytes && ls.bytes <= slots;
       uint32_t* slot_block = nullptr;
       void* sort_block = nullptr;
-      if (e == hipSuccess) e = dev_alloc(&slot_block, std::max(slots, n * 8));
+      if (e == hipSuccess) e = dev_alloc(&slot_block, std::max(slots, ls.bytes));
       if (e == hipSuccess) e = dev_alloc(&agg, 2 * (ntiles + 1) * 8ull);
       if (e == hipSuccess) e = dev_alloc(&pre, 2 * (ntiles + 2) * 8ull);
       const size_t kin_bytes = (n * sizeof(K) + 255) & ~size_t{255};
       if (e == hipSuccess && !inside) e = dev_alloc(&sort_block, kin_bytes + std::max<size_t>(tmp_bytes, 16));
       sa = slot_block;
-      sb = slot_block + n;
+      sb = slot_block + ls.second;
       kin = inside ? key + ns : static_cast<K*>(sort_block);
       tmp = inside ? static_cast<void*>(key + 2 * ns) : static_cast<unsigned char*>(sort_block) + kin_bytes;
       Status st = hip_status(e, "Error in allocating level index construction buffers");

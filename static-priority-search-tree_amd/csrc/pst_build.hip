@@ -34,7 +34,6 @@ namespace pst {
 namespace {
 
 constexpr int kFinishBlock = 512;      // threads per LDS subtree of the deep tree
-constexpr uint32_t kFinishTile = 2048;  // max points per LDS subtree
 constexpr int kForestBlock = 256;       // threads per forest tree
 // Levels of the forest trees that k_forest_reg builds (pst_forest_build.hip):
 // trees of 31 to 511 points, a wave each (2.99 -> 0.174 ms for 16.7M points
@@ -136,8 +135,6 @@ __global__ void k_scatter_rank(const uint32_t* __restrict__ perm2, uint32_t n, u
 // the levels above that lie in it (its holes, a sorted list of at most t
 // positions; one per segment on average, since a node lies in one segment).
 // ---------------------------------------------------------------------------
-constexpr uint32_t kFan = 64;        // values per block minimum, and per step of the hierarchy
-constexpr uint32_t kMaxHoles = 24;   // list entries per segment (levels above LDS size: at most 19)
 constexpr int kTopBlock = 256;
 
 // mins1[k]: minimum of values [64 k, 64 k + 64); mins2 of 64 such, one
@@ -291,49 +288,22 @@ __global__ __launch_bounds__(kTopBlock) void k_top_level(Src src, const typename
   const uint32_t b = in.b[j], e = j + 1 < nseg ? in.b[j + 1] : n;
   const uint32_t cnt = in.cnt[j];
   uint32_t hole = lane < cnt ? in.holes[static_cast<size_t>(j) * kMaxHoles + lane] : ~0u;
-  const uint32_t n1 = (n + kFan - 1) / kFan, n2 = (n1 + kFan - 1) / kFan;
+  const uint32_t n1 = blocks_of(n), n2 = blocks_of(n1);
   // the lane's best candidate: its value, step of the hierarchy and index
   V best = static_cast<V>(~V(0));
   uint32_t step = 0, at = ~0u;
-  auto take = [&](const V* arr, uint32_t i, uint32_t end, uint32_t st) {
-    if (i < end) {
-      const V v = arr[i];
-      if (v < best || at == ~0u) {
-        best = v;
-        step = st;
-        at = i;
-      }
+  auto take = [&](uint32_t st, uint32_t i) {
+    const V v = (st == 0 ? a : (st == 1 ? m1 : (st == 2 ? m2 : m3)))[i];
+    if (v < best || at == ~0u) {
+      best = v;
+      step = st;
+      at = i;
     }
   };
   for (uint32_t r = 0; r <= cnt; r++) {
     const uint32_t lo = r == 0 ? b : __builtin_amdgcn_readlane(hole, r - 1) + 1;
     const uint32_t hi = r == cnt ? e : static_cast<uint32_t>(__builtin_amdgcn_readlane(hole, r));
-    if (lo >= hi) continue;
-    const uint32_t lo1 = (lo + kFan - 1) / kFan, hi1 = hi / kFan;
-    if (lo1 >= hi1) {  // no whole block of 64 inside
-      take(a, lo + lane, hi, 0);
-      take(a, lo + kWave + lane, hi, 0);
-      continue;
-    }
-    take(a, lo + lane, lo1 * kFan, 0);
-    take(a, hi1 * kFan + lane, hi, 0);
-    const uint32_t lo2 = (lo1 + kFan - 1) / kFan, hi2 = hi1 / kFan;
-    if (lo2 >= hi2) {
-      take(m1, lo1 + lane, hi1, 1);
-      take(m1, lo1 + kWave + lane, hi1, 1);
-      continue;
-    }
-    take(m1, lo1 + lane, lo2 * kFan, 1);
-    take(m1, hi2 * kFan + lane, hi1, 1);
-    const uint32_t lo3 = (lo2 + kFan - 1) / kFan, hi3 = hi2 / kFan;
-    if (lo3 >= hi3) {
-      take(m2, lo2 + lane, hi2, 2);
-      take(m2, lo2 + kWave + lane, hi2, 2);
-      continue;
-    }
-    take(m2, lo2 + lane, lo3 * kFan, 2);
-    take(m2, hi3 * kFan + lane, hi2, 2);
-    for (uint32_t i = lo3; i < hi3; i += kWave) take(m3, i + lane, hi3, 3);
+    stretch_minima(lo, hi, lane, take);
   }
   V mn = best;
 #pragma unroll
@@ -1092,23 +1062,10 @@ struct BuildLayout {
 
 inline size_t al256(size_t b) { return (b + 255) & ~size_t{255}; }
 
-// Levels walked by global passes: every segment of level t0 fits in LDS.
-inline uint32_t finish_level(uint64_t M) {
-  uint32_t t0 = 0;
-  while (true) {
-    const uint64_t base = M >> t0;
-    const uint64_t r = M & ((1ull << t0) - 1ull);
-    const uint64_t mx = base - 1 + (r ? 1 : 0);
-    if (mx <= kFinishTile) break;
-    t0++;
-  }
-  return t0;
-}
-
 // Block minima of n values: steps 1, 2 and 3 of the hierarchy.
 inline size_t min_words(size_t n) {
-  const size_t n1 = (n + kFan - 1) / kFan, n2 = (n1 + kFan - 1) / kFan;
-  return n1 + n2 + (n2 + kFan - 1) / kFan;
+  const size_t n1 = blocks_of(n), n2 = blocks_of(n1);
+  return n1 + n2 + blocks_of(n2);
 }
 // One level's segment table, for levels up to t0.
 inline size_t segs_bytes(uint32_t t0) { return (size_t{1} << t0) * (2 + kMaxHoles) * 4; }
@@ -1167,7 +1124,7 @@ Status build_levels(Src src, const typename Src::V* A, uint32_t n, uint32_t t0, 
   Segs cur = segs_at(segs, t0), nxt = segs_at(segs + segs_bytes(t0), t0);
   k_segs_root<<<1, 1, 0, s>>>(cur);
   if (t0 > 0) {
-    const uint32_t n1 = (n + kFan - 1) / kFan, n2 = (n1 + kFan - 1) / kFan, n3 = (n2 + kFan - 1) / kFan;
+    const uint32_t n1 = blocks_of(n), n2 = blocks_of(n1), n3 = blocks_of(n2);
     V* m1 = reinterpret_cast<V*>(mins);
     V* m2 = m1 + n1;
     V* m3 = m2 + n2;

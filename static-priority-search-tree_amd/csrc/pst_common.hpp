@@ -200,6 +200,59 @@ __host__ __device__ inline uint64_t brev_below(uint32_t t, uint32_t j, uint64_t 
 }
 
 // ---------------------------------------------------------------------------
+// Construction's levels above LDS size (pst_build.hip): a static hierarchy of
+// minima, kFan values per entry and step, answers range minima of the
+// key1-ordered array.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kFinishTile = 2048;  // max points per LDS subtree
+constexpr uint32_t kFan = 64;           // values per block minimum, and per step of the hierarchy
+// Entries of a segment's hole list: at most one per level above LDS size.
+constexpr uint32_t kMaxHoles = 24;
+
+// Levels above LDS size of a tree of M - 1 points: every segment of the
+// returned level fits in LDS.
+constexpr uint32_t finish_level(uint64_t M) {
+  uint32_t t0 = 0;
+  while ((M >> t0) - 1 + ((M & ((1ull << t0) - 1ull)) ? 1 : 0) > kFinishTile) t0++;
+  return t0;
+}
+static_assert(finish_level((1ull << 32) - 1) <= kMaxHoles, "hole lists hold a node per level");
+
+// Blocks of kFan values, the last one partial (no sum that could wrap).
+template <typename N>
+__host__ __device__ constexpr N blocks_of(N n) {
+  return n / kFan + (n % kFan != 0 ? 1 : 0);
+}
+
+// Hands lane `lane` of a wave its entries of the hierarchy whose minima make
+// up that of values [lo, hi): take(step, index), step 0 the values, 1 their
+// block minima, 2 and 3 those above. At most 126 entries at each end of each
+// step, and the middle of step 3. Indices are formed only inside the range,
+// so that none wraps for arrays of up to 2^32 - 1 values.
+template <typename F>
+__host__ __device__ inline void stretch_minima(uint32_t lo, uint32_t hi, uint32_t lane, F&& take) {
+  auto part = [&](uint32_t step, uint32_t from, uint32_t skip, uint32_t end) {
+    if (from < end && lane + skip < end - from) take(step, from + lane + skip);
+  };
+  uint32_t f = lo, e = hi;  // the range in entries of the step
+#pragma unroll
+  for (uint32_t step = 0; step < 3; step++) {
+    if (f >= e) return;
+    const uint32_t f1 = blocks_of(f), e1 = e / kFan;
+    if (f1 >= e1) {  // no whole block inside
+      part(step, f, 0, e);
+      part(step, f, kFan, e);
+      return;
+    }
+    part(step, f, 0, f1 * kFan);
+    part(step, e1 * kFan, 0, e);
+    f = f1;
+    e = e1;
+  }
+  for (uint32_t i = f; i < e; i += kFan) part(3, i, 0, e);
+}
+
+// ---------------------------------------------------------------------------
 // Search state of a query at a node, as bits j of three masks for the G
 // queries of a group: `a` the query is walking this subtree, `l` its lower
 // dim1 bound still cuts the subtree, `h` its upper bound still does. These

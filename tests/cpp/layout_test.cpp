@@ -26,11 +26,55 @@ void level_slots() {
     CHECK(pst::level_stride(n) * 4 % 256 == 0 && pst::level_stride(n) >= n, n);
   }
 }
+
+// The entries that a range minimum reads, over all lanes: exactly the range,
+// each value once, also next to 2^32, at most two wave reads per end and step.
+void stretch() {
+  const uint32_t top = 0xfffffffeu;
+  auto one = [&](uint32_t lo, uint32_t hi) {
+    unsigned long long covered = 0;
+    bool inside = true;
+    uint32_t most = 0;
+    for (uint32_t lane = 0; lane < 64; lane++) {
+      uint32_t few = 0;
+      pst::stretch_minima(lo, hi, lane, [&](uint32_t step, uint32_t i) {
+        const unsigned long long w = 1ull << (6 * step);
+        inside &= i * w >= lo && i * w + w <= hi;
+        covered += w;
+        if (step < 3) few++;
+      });
+      most = few > most ? few : most;
+    }
+    CHECK(inside, lo);
+    CHECK(covered == (hi > lo ? hi - lo : 0), lo);
+    CHECK(most <= 6, lo);
+  };
+  for (uint32_t n : {1u, 63u, 64u, 65u, 128u, 4095u, 4096u, 4097u, 300007u, 0x10000000u, 0xffffff80u, 0xffffffbfu,
+                     0xffffffc0u, 0xffffffc1u, 0xfffffff0u, top}) {
+    one(0, n);
+    for (uint32_t d : {0u, 1u, 2u, 62u, 63u, 64u, 65u, 127u, 128u, 4000u, 4096u, 5000u, 270000u})
+      for (uint32_t w : {1u, 2u, 63u, 64u, 65u, 127u, 128u, 200u, 4097u, 262145u})
+        if (d + w <= n) {
+          one(n - d - w, n - d);  // ranges that end at or near the array's end
+          one(d, d + w);
+        }
+  }
+  for (uint32_t n : {1u, 64u, 65u, 0xffffffc0u, 0xffffffc1u, top}) {
+    CHECK(pst::blocks_of(n) == (n + 63ull) / 64, n);
+    CHECK(pst::blocks_of(static_cast<size_t>(n)) == (n + 63ull) / 64, n);
+  }
+  // hole lists: a level's segments hold at most one hole per level above it
+  for (unsigned long long n : {1ull, 2048ull, 2049ull, 1ull << 26, 1ull << 31, 0xfffffffeull}) {
+    CHECK(pst::finish_level(n + 1) <= pst::kMaxHoles, n);
+    CHECK(pst::level_size(n + 1, pst::finish_level(n + 1), 0) <= 2048, n);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string only = argc > 1 ? argv[1] : "";
   if (only.empty() || only == "level_slots") level_slots();
+  if (only.empty() || only == "stretch") stretch();
   std::printf(g_bad ? "%d checks failed\n" : "LAYOUT OK\n", g_bad);
   return g_bad != 0;
 }

@@ -357,6 +357,29 @@ __host__ __device__ inline StepOut node_step_report_above(T d2, int32_t m, const
 }
 
 // ---------------------------------------------------------------------------
+// How a round's list of work items is dealt to its waves: evenly, wave w
+// taking items [w c / W, (w + 1) c / W), one more or one fewer than any other;
+// or each wave c / W rounded down, at most `most`, and the rest in grabs of as
+// many from a counter, which gives it to the waves that are done first. The
+// counter serves grabs one by one, 34 ns each on MI355X, so the rest is grabbed
+// where that takes at most `grabs` of them, or the list is too long to deal.
+// ---------------------------------------------------------------------------
+struct Deal {
+  uint64_t base;  // the wave's first item
+  uint64_t dyn;   // first item that is grabbed (the list's length: none is)
+  uint32_t cnt;   // items of the wave
+  uint32_t unit;  // items per grab
+};
+__host__ __device__ inline Deal deal_items(uint64_t count, uint32_t waves, uint32_t wave, uint32_t most, uint32_t grabs) {
+  const uint64_t per = count / waves, rest = count - per * waves;
+  if (per >= most || (per > 0 && rest <= grabs * per)) {
+    const uint32_t unit = per < most ? static_cast<uint32_t>(per) : most;
+    return Deal{static_cast<uint64_t>(wave) * unit, static_cast<uint64_t>(waves) * unit, unit, unit};
+  }
+  return Deal{wave * per + (wave < rest ? wave : rest), count, static_cast<uint32_t>(per) + (wave < rest ? 1u : 0u), 0u};
+}
+
+// ---------------------------------------------------------------------------
 // Wave64 helpers (gfx950 wavefront = 64 lanes).
 // ---------------------------------------------------------------------------
 constexpr int kWave = 64;

@@ -139,6 +139,7 @@ struct Params {
   unsigned long long* task_ctr;
   uint32_t total_waves;
   uint32_t budget_small, budget_large;
+  uint32_t grabs;      // most grabs of a round whose list could be dealt evenly
   uint32_t few_items;  // lists shorter than this take the small budget
 };
 
@@ -376,15 +377,13 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
   const Entry* list_in = P.list[round & 1];
   Entry* list_out = P.list[(round + 1) & 1];
 
-  unsigned long long chunk = count_in / P.total_waves;
-  chunk = chunk < 1 ? 1 : (chunk > kWave ? kWave : chunk);
+  const Deal share = deal_items(count_in, P.total_waves, blockIdx.x, kWave, P.grabs);
   const uint32_t budget =
       last ? 0xffffffffu : (count_in < P.few_items ? P.budget_small : P.budget_large);
 
-  // The first chunk of each wave is fixed by its index; later chunks are
+  // The wave's share of the list is fixed by its index; the rest, if any, is
   // grabbed from a shared counter, which is read first so that waves with
   // nothing left to take leave without an atomic update.
-  const unsigned long long dyn0 = static_cast<unsigned long long>(P.total_waves) * chunk;
   bool fixed_done = false;
   uint32_t npend = 0;  // uniform: valid pending entries are pend[0..npend) with group != kEmpty
   while (true) {
@@ -393,19 +392,21 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
     const uint64_t have = __ballot(mine_g != kEmpty);
     if (have == 0) {
       unsigned long long base = 0;
+      uint32_t cnt = 0;
       if (!fixed_done) {
         fixed_done = true;
-        base = static_cast<unsigned long long>(blockIdx.x) * chunk;
-        if (base >= count_in) continue;
+        base = share.base;
+        cnt = share.cnt;
+        if (cnt == 0) continue;
       } else {
-        if (dyn0 >= count_in ||
-            dyn0 + __hip_atomic_load(grab, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= count_in)
+        if (share.dyn >= count_in ||
+            share.dyn + __hip_atomic_load(grab, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= count_in)
           break;
-        if (lane == 0) base = dyn0 + atomicAdd(grab, chunk);
+        if (lane == 0) base = share.dyn + atomicAdd(grab, static_cast<unsigned long long>(share.unit));
         base = __shfl(base, 0, kWave);
         if (base >= count_in) break;
+        cnt = count_in - base < share.unit ? static_cast<uint32_t>(count_in - base) : share.unit;
       }
-      const unsigned long long cnt = min(chunk, count_in - base);
       Entry e{0, kEmpty};
       if (lane < cnt) {
         e.group = __hip_atomic_load(&list_in[base + lane].group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -419,8 +420,8 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
         e.group = kEmpty;
       }
       pend[lane] = e;
-      npend = static_cast<uint32_t>(cnt);
-      if (P.dbg && lane == 0) atomicAdd(&P.dbg[round * 8 + 2], cnt);
+      npend = cnt;
+      if (P.dbg && lane == 0) atomicAdd(&P.dbg[round * 8 + 2], static_cast<unsigned long long>(cnt));
       __builtin_amdgcn_wave_barrier();
       continue;
     }
@@ -1167,20 +1168,32 @@ TreeShape tree_shape(const SearchArgs& a) {
 // step after that doubles what a round hands on: many groups on few points
 // have enough items after one round, and a second would only move them through
 // memory; few groups on many points need it for balance. By points per group,
-// count / write passes in us on MI355X, at 2 rounds (9 steps), 3 (7), 3 (8):
-//   1396 queries on 4,183,215 (24k)  350/ 965   276/ 846   475/1063
-//   2500 on 4,183,215         (13k)  403/1227   443/1210  1115/1898
-//   2500 on 2,000,003          (6k)  232/ 817   331/ 887   887/1468
-//   1000 on 2,000,003         (16k)  129/ 595   199/ 586   219/ 630
-//   256 on 2^20               (33k)   66/ 181   189/ 284   143/ 213
-//   2000 on 2^23              (34k)  793/1605   577/1477  1096/1828
-//   3000 on 2^25              (89k)      3368       2728       3159
-//   4096 on 2^26             (131k)      9016       6562       5391
-//   2048 on 2^26             (262k)      4788       4368       3462
-//   256 on 2^23              (262k)  247/ 675   167/ 447   165/ 445
-//   32 on 2^20               (262k)   74/ 175   244/ 237   136/ 193
-// 4 rounds of 6 and 384 steps take 309/1540, 466/1884, 327/1555, 216/1263,
-// 256/345, 637/1659, 3432, 6387, 4135, 435/718 and 228/318.
+// count / write passes in us on MI355X, at 2 rounds (9 steps), 3 (7), 3 (8) and
+// 4 rounds of 6 and 384:
+//   1396 queries on 4,183,215 (24k)  275/1017   268/ 858   483/1096   260/ 885
+//   2500 on 4,183,215         (13k)  388/1304   447/1248   773/1553   394/1205
+//   2500 on 2,000,003          (6k)  222/ 819   326/ 886   568/1169   258/ 802
+//   1000 on 2,000,003         (16k)  140/ 613   181/ 608   236/ 648   158/ 601
+//   600 on 1,300,003          (17k)   97/ 458   138/ 458   144/ 454   363/ 721
+//   256 on 2^20               (33k)   78/ 194   105/ 202   110/ 200   255/ 363
+//   2000 on 2^23              (34k)  586/1841   575/1517   902/1725   551/1514
+//   3000 on 2^25              (89k)      3420       2731       2413       3292
+//   200 on 3,000,000         (120k)  125/ 426   118/ 372   130/ 369   270/ 527
+//   4096 on 2^26             (131k)      9451       6221       6107       6210
+//   2048 on 2^26             (262k)      5882       4490       3669       4064
+//   256 on 2^23              (262k)  250/ 688   155/ 449   173/ 453   343/ 657
+//   32 on 2^20               (262k)   86/ 192   113/ 176   118/ 182   206/ 275
+// A pass walks some 4.5M pairs of a group and a point per microsecond. One grab
+// per 2^22 pairs is a fraction of its time, and giving a list's rest to the
+// waves that are done first is worth more than that: count passes in us, all
+// lists dealt evenly / one grab per 2^22 pairs / all rests grabbed, 4096 mixed
+// queries on 2^26 points 6252 / 5393 / 5374, 3000 stabbing 6507 / 5838 / 5754.
+// On smaller walks the grabs are the time: 1600 stabbing queries on 2^21 points
+// 209 / 209 / 543, 3000 on 400,003 126 / 126 / 391, 2048 mixed on 2.5M
+// 244 / 238 / 551, 4096 stabbing on 2^23 1486 / 1499 / 1971. (2^21 pairs: 1989
+// instead of 1745 for 4096 mixed on 2^24; 2^23: 5053 instead of 4599 for 3000
+// stabbing on 50,000,017.)
+constexpr int kGrabShift = 22;
 constexpr uint64_t kSmallWalk = 1ull << 25;    // groups x points
 constexpr uint64_t kSmallTree = 1ull << 21;    // points
 constexpr uint64_t kGroupPoints = 1ull << 14;  // points per group below which groups alone fill the rounds
@@ -1196,17 +1209,20 @@ int search_rounds(const SearchArgs& a) {
 namespace {
 
 // Steps per batch in the rounds before the last, while lists are short. Of two
-// rounds, 9 steps lose to 8 on small trees between 128 and 384 groups, where
-// the longer list of the second round is dealt to the waves less evenly: count
-// passes in us, 9 / 8 steps (4 rounds of 6: last)
-//   2000 queries on 65536 122 / 65 (131), on 200,000 217 / 74 (227), on
-//   1,000,003 326 / 127 (199); 3000 on 100,000 357 / 101 (253);
-//   beyond: 4096 on 65536 140 / 213 (334), 1000 on 2,000,003 127 / 165 (216),
-//   640 on 2^20 79 / 96 (165), 3400 on 2^20 265 / 318 (356).
+// rounds, 9 steps, but 8 on trees that leave the second round little work:
+// count passes in us, 8 / 9 steps, 64, 400, 1000, 1600 and 3064 queries on
+//   20,001   46/46  52/53   58/61   63/69   83/84
+//   65,536   48/49  53/55   61/68   69/74   90/91
+//   150,001  53/51  59/59   67/73   77/82   98/105
+//   262,144  56/53  63/61   74/76   82/85  105/111
+//   400,003  62/55  71/64   85/81   92/90  116/115
+//   2^20     83/67  96/83  122/104 134/119 188/163
+constexpr uint64_t kFewPoints = 1ull << 17, kFewPointsGroups = 1ull << 18;
+constexpr uint64_t kManyGroups = 128;
 int search_budget(const SearchArgs& a, int group, int rounds) {
   if (group == 1) return 6;
   const uint64_t groups = (a.nq + kGroup - 1) / kGroup;
-  if (rounds <= 2) return groups >= 128 && groups < 384 && a.n <= kSmallTree / 2 ? 8 : 9;
+  if (rounds <= 2) return a.n <= (groups >= kManyGroups ? kFewPointsGroups : kFewPoints) ? 8 : 9;
   return a.n >= groups * kWidePoints ? 8 : 7;
 }
 
@@ -1285,6 +1301,7 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
   const uint32_t grid = static_cast<uint32_t>(cus * occ);
   P.total_waves = grid;
   P.few_items = G == 1 ? grid : 4 * grid;
+  P.grabs = static_cast<uint32_t>(std::min<uint64_t>(a.n * P.ngroups >> kGrabShift, grid));
   const size_t gbytes = static_cast<size_t>(grid) * P.gcap * sizeof(Items::type);
   if (sc.gstack_bytes < gbytes) {
     if (sc.pinned) return Status{1, kPinnedScratchMsg};

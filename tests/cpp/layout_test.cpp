@@ -69,12 +69,43 @@ void stretch() {
     CHECK(pst::level_size(n + 1, pst::finish_level(n + 1), 0) <= 2048, n);
   }
 }
+
+// A round's list over its waves: every item once, shares within one of each
+// other, and no more grabs than allowed where the list could be dealt evenly.
+void deal() {
+  for (uint32_t waves : {1u, 3u, 256u, 8192u})
+    for (uint32_t most : {1u, 4u, 64u})
+      for (uint32_t grabs : {0u, 1u, 100u, 8192u})
+        for (unsigned long long per : {0ull, 1ull, 2ull, 3ull, 17ull, 63ull, 64ull, 200ull})
+          for (unsigned long long more : {0ull, 1ull, waves / 2ull, waves - 1ull}) {
+            const unsigned long long count = per * waves + (more < waves ? more : 0);
+            unsigned long long at = 0, low = ~0ull, high = 0, dyn = 0;
+            uint32_t unit = 0;
+            bool ok = true;
+            for (uint32_t w = 0; w < waves; w++) {
+              const pst::Deal d = pst::deal_items(count, waves, w, most, grabs);
+              ok &= (w == 0 || (d.dyn == dyn && d.unit == unit)) && d.base == at && d.cnt <= most;
+              dyn = d.dyn;
+              unit = d.unit;
+              at += d.cnt;
+              low = d.cnt < low ? d.cnt : low;
+              high = d.cnt > high ? d.cnt : high;
+            }
+            CHECK(ok, count);
+            CHECK(at == dyn && dyn <= count, count);
+            CHECK(high - low <= 1, count);
+            const unsigned long long left = count - dyn;
+            CHECK(left == 0 || unit > 0, count);
+            CHECK(left == 0 || per >= most || (left + unit - 1) / unit <= grabs, count);
+          }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string only = argc > 1 ? argv[1] : "";
   if (only.empty() || only == "level_slots") level_slots();
   if (only.empty() || only == "stretch") stretch();
+  if (only.empty() || only == "deal") deal();
   std::printf(g_bad ? "%d checks failed\n" : "LAYOUT OK\n", g_bad);
   return g_bad != 0;
 }

@@ -1183,6 +1183,14 @@ TreeShape tree_shape(const SearchArgs& a) {
 //   2048 on 2^26             (262k)      5882       4490       3669       4064
 //   256 on 2^23              (262k)  250/ 688   155/ 449   173/ 453   343/ 657
 //   32 on 2^20               (262k)   86/ 192   113/ 176   118/ 182   206/ 275
+// Few groups on a large tree need three rounds most: what two rounds hand on
+// to the last one is a few hundred subtrees per group, each a wave's. 2 (9) /
+// 3 (7) / 3 (8): 8 queries on 2^21 points 123/221, 122/144, 146/167; on 2^22
+// 204/389, 131/186, 149/197; on 2^25 1342/2701, 166/564, 169/579; 48 on 2^22
+// 175/353, 128/247, 129/253; 100 on 2^21 98/209, 117/205, 121/212. 8 steps pay
+// on large walks alone, 3 (7) / 3 (8): 1024 on 2^24 712/1730, 907/1703; 640 on
+// 2^25 885/2151, 887/2092; 1024 on 2^25 1339/3354, 1405/2875; 256 on 2^26
+// 839/2632, 835/2633; 400 on 2^26 1196/3170, 1138/3154; 2048 on 2^26 4926, 3877.
 // A pass walks some 4.5M pairs of a group and a point per microsecond. One grab
 // per 2^22 pairs is a fraction of its time, and giving a list's rest to the
 // waves that are done first is worth more than that: count passes in us, all
@@ -1194,16 +1202,16 @@ TreeShape tree_shape(const SearchArgs& a) {
 // instead of 1745 for 4096 mixed on 2^24; 2^23: 5053 instead of 4599 for 3000
 // stabbing on 50,000,017.)
 constexpr int kGrabShift = 22;
-constexpr uint64_t kSmallWalk = 1ull << 25;    // groups x points
 constexpr uint64_t kSmallTree = 1ull << 21;    // points
 constexpr uint64_t kGroupPoints = 1ull << 14;  // points per group below which groups alone fill the rounds
-constexpr uint64_t kWidePoints = 1ull << 17;   // and from which a round hands on one more doubling
+constexpr uint64_t kWidePoints = 1ull << 17;   // and from which a round hands on one more doubling,
+constexpr uint64_t kWideWalk = 1ull << 31;     // on walks of more pairs of a group and a point than this
 
 int search_rounds(const SearchArgs& a) {
   if (a.rounds > 0) return std::min(a.rounds, kMaxRounds);
   if (group_size(a) == 1) return 4;
   const uint64_t n = a.n, groups = (a.nq + kGroup - 1) / kGroup;
-  return n <= kSmallTree || groups * n <= kSmallWalk || n < groups * kGroupPoints ? 2 : 3;
+  return n <= kSmallTree || n < groups * kGroupPoints ? 2 : 3;
 }
 
 namespace {
@@ -1223,7 +1231,7 @@ int search_budget(const SearchArgs& a, int group, int rounds) {
   if (group == 1) return 6;
   const uint64_t groups = (a.nq + kGroup - 1) / kGroup;
   if (rounds <= 2) return a.n <= (groups >= kManyGroups ? kFewPointsGroups : kFewPoints) ? 8 : 9;
-  return a.n >= groups * kWidePoints ? 8 : 7;
+  return a.n >= groups * kWidePoints && a.n * groups > kWideWalk ? 8 : 7;
 }
 
 

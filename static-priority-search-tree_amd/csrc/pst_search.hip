@@ -1228,7 +1228,7 @@ namespace {
 constexpr uint64_t kFewPoints = 1ull << 17, kFewPointsGroups = 1ull << 18;
 constexpr uint64_t kManyGroups = 128;
 int search_budget(const SearchArgs& a, int group, int rounds) {
-  if (group == 1) return 6;
+  if (group == 1 || rounds > 3) return 6;
   const uint64_t groups = (a.nq + kGroup - 1) / kGroup;
   if (rounds <= 2) return a.n <= (groups >= kManyGroups ? kFewPointsGroups : kFewPoints) ? 8 : 9;
   return a.n >= groups * kWidePoints && a.n * groups > kWideWalk ? 8 : 7;
@@ -1308,7 +1308,7 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
   hipError_t e = hipSuccess;
   const uint32_t grid = static_cast<uint32_t>(cus * occ);
   P.total_waves = grid;
-  P.few_items = G == 1 ? grid : 4 * grid;
+  P.few_items = few_items(a, G, grid);
   P.grabs = static_cast<uint32_t>(std::min<uint64_t>(a.n * P.ngroups >> kGrabShift, grid));
   const size_t gbytes = static_cast<size_t>(grid) * P.gcap * sizeof(Items::type);
   if (sc.gstack_bytes < gbytes) {

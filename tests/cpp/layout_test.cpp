@@ -99,6 +99,25 @@ void deal() {
             CHECK(left == 0 || per >= most || (left + unit - 1) / unit <= grabs, count);
           }
 }
+
+// Which lists of a round count as short: forests and budgets set by the caller
+// as ever, the default schedule of group walks on a deep tree four times that.
+void few() {
+  pst::SearchArgs a{};
+  a.n = 1 << 24;
+  CHECK(pst::few_items(a, 8, 8192) == 4 * 8192, 0);
+  CHECK(pst::few_items(a, 1, 8192) == 8192, 0);
+  a.budget_small = 6;
+  CHECK(pst::few_items(a, 8, 8192) == 8192, 0);
+  a.budget_small = 0;
+  a.rounds = 4;
+  CHECK(pst::few_items(a, 8, 8192) == 8192, 0);
+  a.rounds = 2;
+  CHECK(pst::few_items(a, 8, 8192) == 4 * 8192, 0);
+  a.rounds = 0;
+  a.slots_per_tree = 1023;
+  CHECK(pst::few_items(a, 8, 8192) == 8192, 0);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -106,6 +125,7 @@ int main(int argc, char** argv) {
   if (only.empty() || only == "level_slots") level_slots();
   if (only.empty() || only == "stretch") stretch();
   if (only.empty() || only == "deal") deal();
+  if (only.empty() || only == "few") few();
   std::printf(g_bad ? "%d checks failed\n" : "LAYOUT OK\n", g_bad);
   return g_bad != 0;
 }

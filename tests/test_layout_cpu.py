@@ -8,7 +8,7 @@ import pytest
 BIN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "_build", "layout_test")
 
 
-@pytest.mark.parametrize("part", ["level_slots", "stretch", "deal"])
+@pytest.mark.parametrize("part", ["level_slots", "stretch", "deal", "few"])
 def test_layout(part):
     assert os.path.exists(BIN), "tests/cpp/_build/layout_test is not built (run __graft_entry__.build())"
     r = subprocess.run([BIN, part], capture_output=True, text=True, timeout=120)

@@ -90,7 +90,7 @@ unsigned long long* device_counter(int dev) {
   auto it = g_ctr.find(dev);
   if (it != g_ctr.end()) return it->second;
   unsigned long long* p = nullptr;
-  if (pst::result_alloc(&p, sizeof(unsigned long long)) != hipSuccess) return nullptr;
+  if (pst::plain_alloc(&p, sizeof(unsigned long long)) != hipSuccess) return nullptr;
   g_ctr[dev] = p;
   return p;
 }

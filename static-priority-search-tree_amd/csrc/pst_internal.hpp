@@ -126,9 +126,19 @@ hipError_t dev_free_idle(void* p);
 size_t dev_keep_limit();
 // Gives every kept block of every device back to the runtime.
 void dev_release_kept();
-// Memory that is never from or in the cache: results, which the caller may
-// free by hipFree, and a server's buffers. An allocation that finds too little
-// is tried again once the kept blocks are given back.
+// Memory that is never from or in the cache (a server's buffers), freed by
+// hipFree. An allocation that finds too little is tried again once the kept
+// blocks are given back.
+hipError_t plain_alloc_bytes(void** p, size_t bytes);
+template <typename U>
+hipError_t plain_alloc(U** p, size_t bytes) {
+  void* v = nullptr;
+  const hipError_t e = plain_alloc_bytes(&v, bytes);
+  *p = static_cast<U*>(v);
+  return e;
+}
+// Results for the caller, who may free them by hipFree: large ones through the
+// cache, which result_free (it waits as hipFree does) puts them back into.
 hipError_t result_alloc_bytes(void** p, size_t bytes);
 template <typename U>
 hipError_t result_alloc(U** p, size_t bytes) {

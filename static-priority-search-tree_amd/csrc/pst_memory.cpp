@@ -20,10 +20,12 @@
 //   - Given back: every kept block of a device is freed when an allocation
 //     on it fails, before that allocation is tried once more, and all of them
 //     on request (dev_release_kept), for other allocators of the program.
-//   - Only the library's own blocks: results go to callers, who free them by
-//     pst_free or hipFree, so they come from hipMalloc and go by hipFree. (A
-//     kept block that a caller could free behind the cache's back would be
-//     handed out unmapped.) Up to 2 MB that pair takes 1.4 us, 64 MB 24 us.
+//   - Results go to callers, who may free them by pst_free, which keeps them,
+//     or by hipFree, of which the cache learns nothing. So a result is known
+//     by the runtime's ID of its allocation, and every use of a kept one
+//     (handing it out, freeing it) first checks that the address still holds
+//     that allocation; a second pst_free is refused. Results of up to 1 MB
+//     come from hipMalloc and go by hipFree (1.4 us for both; 4 to 64 MB 24).
 //   - Safe over streams: a block enters the cache only when nothing on the
 //     device can use it any more: dev_free waits for the device, by a hipFree,
 //     and dev_free_idle is for callers that have waited themselves.
@@ -32,6 +34,7 @@
 // Blocks hold what their last user left; no caller may expect zeros.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <unordered_map>
@@ -45,19 +48,35 @@ namespace {
 
 constexpr size_t kLargeBlock = size_t{32} << 20;
 constexpr size_t kKeepShare = 32;  // of a device's memory at most one part in so many is kept
+constexpr size_t kSmallResult = size_t{1} << 20;  // results up to here are not kept
 
 struct Block {
   void* p;
   size_t bytes;
   int dev;
+  unsigned long long id = 0;  // the runtime's ID of an allocation that was a result (0: never one)
 };
+
+// ID of the allocation that starts at p (0: none, or none to be had).
+unsigned long long allocation_id(void* p) {
+  unsigned long long id = 0;
+  if (hipPointerGetAttribute(&id, HIP_POINTER_ATTRIBUTE_BUFFER_ID, p) == hipSuccess) return id;
+  (void)hipGetLastError();
+  return 0;
+}
+bool still_there(const Block& b) { return b.id == 0 || allocation_id(b.p) == b.id; }
 
 struct Cache {
   std::mutex mu;
   std::unordered_map<void*, Block> live;
+  // results that callers hold, and how many entries it takes to look for
+  // those that were freed by hipFree
+  std::unordered_map<void*, Block> results;
+  size_t sweep_at = 256;
   // kept blocks in the order they were freed, and per (device, size) which
   std::map<unsigned long long, Block> kept;
   std::multimap<std::pair<int, size_t>, unsigned long long> by_size;
+  std::unordered_map<void*, unsigned long long> kept_at;
   std::map<int, size_t> kept_bytes, limit;
   unsigned long long tick = 0;
 
@@ -69,7 +88,20 @@ struct Cache {
         break;
       }
     kept_bytes[it->second.dev] -= it->second.bytes;
+    kept_at.erase(it->second.p);
     kept.erase(it);
+  }
+  // A kept block of exactly this size, out of the tables; blocks that are no
+  // longer the library's are dropped on the way.
+  bool take(int dev, size_t bytes, Block* out) {
+    for (;;) {
+      auto r = by_size.equal_range({dev, bytes});
+      if (r.first == r.second) return false;
+      auto k = kept.find(r.first->second);
+      *out = k->second;
+      forget(k);
+      if (still_there(*out)) return true;
+    }
   }
 };
 
@@ -79,19 +111,20 @@ Cache& cache() {
   return *c;
 }
 
-void free_all(const std::vector<void*>& ps) {
-  for (void* p : ps) (void)hipFree(p);
+void free_all(const std::vector<Block>& bs) {
+  for (const Block& b : bs)
+    if (still_there(b)) (void)hipFree(b.p);
 }
 
 // Takes every kept block of `dev` out of the cache.
-std::vector<void*> take_kept(int dev) {
+std::vector<Block> take_kept(int dev) {
   Cache& c = cache();
-  std::vector<void*> out;
+  std::vector<Block> out;
   std::lock_guard<std::mutex> lk(c.mu);
   for (auto it = c.kept.begin(); it != c.kept.end();) {
     auto next = std::next(it);
     if (it->second.dev == dev) {
-      out.push_back(it->second.p);
+      out.push_back(it->second);
       c.forget(it);
     }
     it = next;
@@ -163,7 +196,7 @@ namespace {
 hipError_t malloc_on(int dev, void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e == hipErrorOutOfMemory) {
-    const std::vector<void*> back = take_kept(dev);
+    const std::vector<Block> back = take_kept(dev);
     if (!back.empty()) {
       free_all(back);
       (void)hipGetLastError();  // the failed attempt's
@@ -175,15 +208,119 @@ hipError_t malloc_on(int dev, void** p, size_t bytes) {
 }
 }  // namespace
 
-hipError_t result_alloc_bytes(void** p, size_t bytes) {
+namespace {
+// Puts an idle block into the cache, within its bounds, or frees it.
+hipError_t keep(const Block& b) {
+  Cache& c = cache();
+  size_t limit = 0;
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    auto l = c.limit.find(b.dev);
+    if (l != c.limit.end()) limit = l->second;
+  }
+  if (limit == 0 || b.bytes >= kLargeBlock) {
+    int cur = 0;
+    size_t free_b = 0, total_b = 0;
+    bool ok = hipGetDevice(&cur) == hipSuccess;
+    if (ok && cur != b.dev) ok = hipSetDevice(b.dev) == hipSuccess;
+    if (ok) ok = hipMemGetInfo(&free_b, &total_b) == hipSuccess;
+    if (cur != b.dev) (void)hipSetDevice(cur);
+    if (!ok) return hipFree(b.p);
+    limit = total_b / kKeepShare;
+    if (b.bytes >= kLargeBlock && free_b < total_b / 8) return hipFree(b.p);
+  }
+  if (b.bytes > limit) return hipFree(b.p);
+  std::vector<Block> out;
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    c.limit[b.dev] = limit;
+    for (auto it = c.kept.begin(); it != c.kept.end() && c.kept_bytes[b.dev] + b.bytes > limit;) {
+      auto next = std::next(it);
+      if (it->second.dev == b.dev) {
+        out.push_back(it->second);
+        c.forget(it);
+      }
+      it = next;
+    }
+    // an entry of this address is of an allocation that a caller freed
+    auto old = c.kept_at.find(b.p);
+    if (old != c.kept_at.end()) c.forget(c.kept.find(old->second));
+    const unsigned long long t = c.tick++;
+    c.kept[t] = b;
+    c.by_size.insert({{b.dev, b.bytes}, t});
+    c.kept_at[b.p] = t;
+    c.kept_bytes[b.dev] += b.bytes;
+  }
+  free_all(out);
+  return hipSuccess;
+}
+
+// Waits for the work of device `dev` by a hipFree of eight bytes, which waits
+// for every stream of the device and for running graphs. hipDeviceSynchronize
+// would break a capture that any thread has running, also a relaxed one; a
+// free does not (1.4 us on an idle device, with the allocation).
+hipError_t wait_on(int dev) {
+  int cur = 0;
+  hipError_t e = hipGetDevice(&cur);
+  if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
+  void* token = nullptr;
+  if (e == hipSuccess) e = malloc_on(dev, &token, 8);
+  if (e == hipSuccess) e = hipFree(token);
+  if (cur != dev) (void)hipSetDevice(cur);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+}  // namespace
+
+hipError_t plain_alloc_bytes(void** p, size_t bytes) {
   *p = nullptr;
   int dev = 0;
   const hipError_t e = hipGetDevice(&dev);
   return e == hipSuccess ? malloc_on(dev, p, bytes ? bytes : 1) : e;
 }
 
+hipError_t result_alloc_bytes(void** p, size_t bytes) {
+  if (bytes <= kSmallResult) return plain_alloc_bytes(p, bytes);
+  *p = nullptr;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  Cache& c = cache();
+  Block b{};
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    if (c.take(dev, bytes, &b)) *p = b.p;
+  }
+  if (!*p) {
+    e = malloc_on(dev, p, bytes);
+    if (e != hipSuccess) return e;
+  }
+  const unsigned long long id = allocation_id(*p);
+  if (id == 0) return hipSuccess;  // freed by hipFree
+  std::lock_guard<std::mutex> lk(c.mu);
+  c.results[*p] = Block{*p, bytes, dev, id};
+  if (c.results.size() >= c.sweep_at) {
+    for (auto it = c.results.begin(); it != c.results.end();) it = still_there(it->second) ? std::next(it) : c.results.erase(it);
+    c.sweep_at = std::max<size_t>(256, 2 * c.results.size());
+  }
+  return hipSuccess;
+}
+
 hipError_t result_free(void* p) {
   if (!p) return hipSuccess;
+  Cache& c = cache();
+  Block b{};
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    auto k = c.kept_at.find(p);
+    if ((k != c.kept_at.end() && still_there(c.kept[k->second])) || c.live.count(p)) return hipErrorInvalidValue;
+    auto it = c.results.find(p);
+    if (it != c.results.end()) {
+      b = it->second;
+      c.results.erase(it);
+    }
+  }
+  if (b.p && still_there(b) && wait_on(b.dev) == hipSuccess) return keep(b);
   const hipError_t e = hipFree(p);
   if (e != hipSuccess) (void)hipGetLastError();  // the caller's mistake, not the next launch's
   return e;
@@ -198,11 +335,8 @@ hipError_t dev_alloc_bytes(void** p, size_t bytes) {
   Cache& c = cache();
   {
     std::lock_guard<std::mutex> lk(c.mu);
-    auto it = c.by_size.find({dev, bytes});
-    if (it != c.by_size.end()) {
-      auto k = c.kept.find(it->second);
-      const Block b = k->second;
-      c.forget(k);
+    Block b{};
+    if (c.take(dev, bytes, &b)) {
       c.live[b.p] = b;
       *p = b.p;
       return hipSuccess;
@@ -219,74 +353,26 @@ hipError_t dev_free_idle(void* p) {
   if (!p) return hipSuccess;
   Cache& c = cache();
   Block b{};
-  size_t limit = 0;
-  bool known = false;
   {
     std::lock_guard<std::mutex> lk(c.mu);
     auto it = c.live.find(p);
     if (it != c.live.end()) {
       b = it->second;
       c.live.erase(it);
-      known = true;
-      auto l = c.limit.find(b.dev);
-      if (l != c.limit.end()) limit = l->second;
     }
   }
-  if (!known) return hipFree(p);
-  if (limit == 0 || b.bytes >= kLargeBlock) {
-    int cur = 0;
-    size_t free_b = 0, total_b = 0;
-    bool ok = hipGetDevice(&cur) == hipSuccess;
-    if (ok && cur != b.dev) ok = hipSetDevice(b.dev) == hipSuccess;
-    if (ok) ok = hipMemGetInfo(&free_b, &total_b) == hipSuccess;
-    if (cur != b.dev) (void)hipSetDevice(cur);
-    if (!ok) return hipFree(p);
-    limit = total_b / kKeepShare;
-    if (b.bytes >= kLargeBlock && free_b < total_b / 8) return hipFree(p);
-  }
-  if (b.bytes > limit) return hipFree(p);
-  std::vector<void*> out;
-  {
-    std::lock_guard<std::mutex> lk(c.mu);
-    c.limit[b.dev] = limit;
-    for (auto it = c.kept.begin(); it != c.kept.end() && c.kept_bytes[b.dev] + b.bytes > limit;) {
-      auto next = std::next(it);
-      if (it->second.dev == b.dev) {
-        out.push_back(it->second.p);
-        c.forget(it);
-      }
-      it = next;
-    }
-    const unsigned long long t = c.tick++;
-    c.kept[t] = b;
-    c.by_size.insert({{b.dev, b.bytes}, t});
-    c.kept_bytes[b.dev] += b.bytes;
-  }
-  free_all(out);
-  return hipSuccess;
+  return b.p ? keep(b) : hipFree(p);
 }
 
-// The wait is a hipFree of eight bytes, which waits for every stream of the
-// device and for running graphs. hipDeviceSynchronize would break a capture
-// that any thread has running, also a relaxed one; a free does not (1.4 us on
-// an idle device, with the allocation).
 hipError_t dev_wait(const void* p) {
   Cache& c = cache();
-  int dev = -1, cur = 0;
+  int dev = -1;
   {
     std::lock_guard<std::mutex> lk(c.mu);
     auto it = c.live.find(const_cast<void*>(p));
     if (it != c.live.end()) dev = it->second.dev;
   }
-  if (dev < 0) return hipSuccess;  // hipFree waits by itself
-  hipError_t e = hipGetDevice(&cur);
-  if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
-  void* token = nullptr;
-  if (e == hipSuccess) e = malloc_on(dev, &token, 8);
-  if (e == hipSuccess) e = hipFree(token);
-  if (cur != dev) (void)hipSetDevice(cur);
-  if (e != hipSuccess) (void)hipGetLastError();
-  return e;
+  return dev < 0 ? hipSuccess : wait_on(dev);  // hipFree waits by itself
 }
 
 hipError_t dev_free(void* p) {

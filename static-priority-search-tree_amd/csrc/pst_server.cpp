@@ -287,7 +287,7 @@ int pst_server_create(pst_tree* const* trees, int num_trees, size_t out_budget_b
   pst_server* s = new pst_server();
   s->max_batch = max_batch;
   s->pool_bytes = out_budget_bytes;
-  hipError_t e = pst::result_alloc(&s->pool_dev, out_budget_bytes);
+  hipError_t e = pst::plain_alloc(&s->pool_dev, out_budget_bytes);
   if (e != hipSuccess) {
     delete s;
     return sfail(PST_ERR_HIP, std::string("Error in allocating the output pool: ") + hipGetErrorString(e));
@@ -305,9 +305,9 @@ int pst_server_create(pst_tree* const* trees, int num_trees, size_t out_budget_b
     e = hipStreamCreateWithFlags(&tq.stream, hipStreamNonBlocking);
     for (int k = 0; k < kSlots && e == hipSuccess; k++) {
       Slot& sl = tq.slots[k];
-      e = pst::result_alloc(&sl.q_dev, max_batch * tq.qrec);
-      if (e == hipSuccess) e = pst::result_alloc(&sl.cnt_dev, (max_batch + 1) * 8);
-      if (e == hipSuccess) e = pst::result_alloc(&sl.off_dev, (max_batch + 1) * 8);
+      e = pst::plain_alloc(&sl.q_dev, max_batch * tq.qrec);
+      if (e == hipSuccess) e = pst::plain_alloc(&sl.cnt_dev, (max_batch + 1) * 8);
+      if (e == hipSuccess) e = pst::plain_alloc(&sl.off_dev, (max_batch + 1) * 8);
       if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&sl.q_host), max_batch * tq.qrec);
       if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&sl.cnt_host), (max_batch + 1) * 8);
       if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&sl.off_host), (max_batch + 1) * 8);
@@ -361,9 +361,9 @@ int pst_server_destroy(pst_server* s) {
   for (auto& tq : s->trees) {
     if (tq.stream) hipStreamSynchronize(tq.stream);
     for (auto& sl : tq.slots) {
-      pst::result_free(sl.q_dev);
-      pst::result_free(sl.cnt_dev);
-      pst::result_free(sl.off_dev);
+      if (sl.q_dev) hipFree(sl.q_dev);
+      if (sl.cnt_dev) hipFree(sl.cnt_dev);
+      if (sl.off_dev) hipFree(sl.off_dev);
       if (sl.q_host) hipHostFree(sl.q_host);
       if (sl.cnt_host) hipHostFree(sl.cnt_host);
       if (sl.off_host) hipHostFree(sl.off_host);
@@ -371,7 +371,7 @@ int pst_server_destroy(pst_server* s) {
     }
     if (tq.stream) hipStreamDestroy(tq.stream);
   }
-  pst::result_free(s->pool_dev);
+  if (s->pool_dev) hipFree(s->pool_dev);
   delete s->pool;
   delete s;
   return PST_OK;

@@ -24,6 +24,9 @@ struct Dev {
 Dev g_dev[2];
 int g_cur = 0;
 std::map<char*, std::pair<size_t, int>> g_mem;  // allocations: bytes, device
+std::map<char*, unsigned long long> g_id;        // and the runtime's ID of each
+unsigned long long g_ids = 0;
+int g_mallocs = 0;
 std::map<size_t, std::vector<char*>> g_free[2];  // freed addresses by size, reused last first
 char* g_next = reinterpret_cast<char*>(size_t{1} << 40);
 int g_waits = 0;          // hipFree calls that worked: each waits for the device
@@ -53,6 +56,8 @@ hipError_t hipMalloc(void** p, size_t n) {
   if (!f.empty()) a = f.back(), f.pop_back();
   else g_next += n + 4096;
   g_mem[a] = {n, g_cur};
+  g_id[a] = ++g_ids;
+  g_mallocs++;
   d.used += n;
   *p = a;
   return hipSuccess;
@@ -67,6 +72,12 @@ hipError_t hipFree(void* p) {
   g_free[it->second.second][it->second.first].push_back(it->first);
   g_mem.erase(it);
   g_waits++;
+  return hipSuccess;
+}
+hipError_t hipPointerGetAttribute(void* data, hipPointer_attribute what, hipDeviceptr_t p) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  if (what != HIP_POINTER_ATTRIBUTE_BUFFER_ID || !g_mem.count(static_cast<char*>(p))) return set_last(hipErrorInvalidValue);
+  *static_cast<unsigned long long*>(data) = g_id[static_cast<char*>(p)];
   return hipSuccess;
 }
 hipError_t hipDeviceSynchronize() {
@@ -123,28 +134,39 @@ void* take(size_t n) {
   return p;
 }
 
-// A result freed twice, or by hipFree and then pst_free, is refused as hipFree
-// refuses it, and the memory handed out afterwards is allocated.
+// A result freed twice by pst_free, or by hipFree and then pst_free, is refused
+// as hipFree refuses it; whatever a caller frees by hipFree, before or after,
+// the memory handed out afterwards is allocated and nobody else's.
 void results() {
-  constexpr size_t n = 1 << 20;
-  for (int how = 0; how < 4; how++) {
-    void* r = nullptr;
-    CHECK(pst::result_alloc(&r, n) == hipSuccess);
-    const hipError_t first = how & 1 ? hipFree(r) : pst::result_free(r);
-    const hipError_t second = how & 2 ? hipFree(r) : pst::result_free(r);
-    CHECK(first == hipSuccess);
-    CHECK(second != hipSuccess);
-    CHECK((how & 2) || hipGetLastError() == hipSuccess);
-    void* a = take(n);
-    void* b = take(n);
-    CHECK(a != b);
-    CHECK(pst::dev_free(a) == hipSuccess && pst::dev_free(b) == hipSuccess);
-    (void)hipGetLastError();
+  for (size_t n : {size_t{1} << 16, size_t{1} << 21}) {
+    for (int how = 0; how < 4; how++) {
+      void* r = nullptr;
+      CHECK(pst::result_alloc(&r, n) == hipSuccess && allocated(r));
+      const hipError_t first = how & 1 ? hipFree(r) : pst::result_free(r);
+      const hipError_t second = how & 2 ? hipFree(r) : pst::result_free(r);
+      CHECK(first == hipSuccess);
+      CHECK((how & 2) || second != hipSuccess);
+      CHECK((how & 2) || hipGetLastError() == hipSuccess);
+      void* other = nullptr;  // may get the address that is free now
+      CHECK(hipMalloc(&other, n) == hipSuccess);
+      void* a = take(n);
+      void* b = nullptr;
+      CHECK(pst::result_alloc(&b, n) == hipSuccess && allocated(b));
+      CHECK(a != b && a != other && b != other);
+      CHECK(pst::dev_free(a) == hipSuccess && pst::result_free(b) == hipSuccess);
+      CHECK(allocated(other));
+      pst::dev_release_kept();
+      CHECK(allocated(other));
+      CHECK(hipFree(other) == hipSuccess);
+      (void)hipGetLastError();
+    }
   }
+  constexpr size_t n = 1 << 20;
   // another owner's block of another size at a freed result's address
   void* r = nullptr;
   CHECK(pst::result_alloc(&r, 2 * n) == hipSuccess);
   CHECK(hipFree(r) == hipSuccess);
+  g_free[0].clear();
   g_free[0][n / 2].push_back(static_cast<char*>(r));
   void* other = nullptr;
   CHECK(hipMalloc(&other, n / 2) == hipSuccess && other == r);
@@ -152,7 +174,34 @@ void results() {
   CHECK(!allocated(other));
   void* big = take(2 * n);
   CHECK(g_mem[static_cast<char*>(big)].first == 2 * n);
+  CHECK(pst::result_free(big) != hipSuccess && allocated(big));  // not the caller's
   CHECK(pst::dev_free(big) == hipSuccess);
+  // a large result that pst_free took is used again, waits included; a block
+  // that was a result stays one that callers may have kept the address of
+  pst::dev_release_kept();
+  CHECK(pst::result_alloc(&r, 2 * n) == hipSuccess);
+  int w = g_waits, m = g_mallocs;
+  CHECK(pst::result_free(r) == hipSuccess && allocated(r) && g_waits > w);
+  m = g_mallocs;
+  void* again = nullptr;
+  CHECK(pst::result_alloc(&again, 2 * n) == hipSuccess && again == r && g_mallocs == m);
+  CHECK(pst::result_free(again) == hipSuccess);
+  void* own = take(2 * n);
+  CHECK(own == r && pst::dev_free(own) == hipSuccess);
+  CHECK(hipFree(r) == hipSuccess);  // by its old address
+  void* fresh = take(2 * n);
+  CHECK(allocated(fresh));
+  CHECK(pst::dev_free(fresh) == hipSuccess);
+  // results that callers free by hipFree do not pile up in the tables' way
+  for (int k = 0; k < 2000; k++) {
+    CHECK(pst::result_alloc(&r, 2 * n + 4096 * (k % 7)) == hipSuccess);
+    CHECK(hipFree(r) == hipSuccess);
+  }
+  std::vector<void*> held(600);
+  for (void*& h : held) CHECK(pst::result_alloc(&h, n + 16) == hipSuccess);
+  for (void* h : held) CHECK(allocated(h) && pst::result_free(h) == hipSuccess);
+  pst::dev_release_kept();
+  for (void* h : held) CHECK(!allocated(h));
 }
 
 // Frees beside a capture neither break it nor lose the block; every block is

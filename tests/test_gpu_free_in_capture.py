@@ -1,4 +1,4 @@
-"""Closing a tree, dropping its level index and freeing a result while another
+"""Closing a tree and dropping its level index while another
 stream is being captured (relaxed or thread-local mode) leaves the capture
 whole and frees what it should: the captured work replays, and a tree built
 afterwards answers."""

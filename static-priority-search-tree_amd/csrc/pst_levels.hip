@@ -47,26 +47,26 @@ constexpr int kLvPer = 16;
 constexpr uint32_t kLvTile = kLvBlock * kLvPer;  // points per partition tile
 constexpr uint32_t kTaskCap = 128;               // ranges per query: <= 4 per level, <= 31 levels
 constexpr uint32_t kFewQueries = 64;             // write plans of up to this many queries probe wider
-// Copy chunks and workgroups. Queries of kLongQuery IDs and more on average,
-// in a large batch, copy best in large chunks by three workgroups per CU (4, 6,
-// 8 are 1 to 3% slower on 1.84G IDs of 1024 queries). Other batches spend
-// their time moving between queries and ranges, where the hardware's own
-// balancing of one chunk per workgroup hides each other's waits: 8192 queries
-// of 14,500 IDs take 342 us with three per CU and chunks of 32768, 273 with
-// eight and 16384, 234 with sixteen, 209 with 64 and 8192 (4.6 TB/s). Small batches are cut into about eight chunks per CU, at least
-// 1024 IDs each (one query of 1.5M IDs 33 us in chunks of 32768, which leave
-// most CUs idle, now 11). 64 bytes of loads in flight per lane: with 256 the
-// registers held the CU to half the waves (2785 instead of 2681 us on the
-// large batch). The IDs are stored as streaming: 2687 -> 2480 us on the large
-// batch and 209 -> 193 (5.0 TB/s) on the short one; loads stay ordinary, since
-// queries share ranges (3154 us with both, the short one 222).
-constexpr uint64_t kLongQuery = 65536, kLongBatch = 1ull << 26;
-constexpr uint64_t kMinChunk = 1024, kChunkShort = 8192, kChunkLong = 32768;
+// Copy chunks and workgroups. Copies spend their time moving between queries
+// and ranges, where the hardware's own balancing of one chunk per workgroup
+// hides each other's waits: 64 workgroups per CU and chunks of 8192 IDs. Small
+// batches are cut into about eight chunks per CU, at least 1024 IDs each (one
+// query of 1.5M IDs 33 us in chunks of 32768, which leave most CUs idle, now
+// 11). us of write calls on MI355X with three workgroups per CU and chunks of
+// 32768 / 64 and 8192 (2^26 points): 32768 queries of 8192 IDs 970 / 753, 2048
+// of 65,636 299 / 231, 512 of 264,712 265 / 218, 256 of 1.0M 426 / 367, 1024
+// mixed ones of 1.8M 2250 / 2140. 64 bytes of loads in flight per lane: with
+// 256 the registers held the CU to half the waves (2785 instead of 2681 us on
+// the last). The IDs are stored as streaming (2687 -> 2480 us there); loads
+// stay ordinary, since queries share ranges (3154 us with both).
+constexpr uint64_t kMinChunk = 1024, kMaxChunk = 8192;
 constexpr uint64_t kChunkSpread = 2048;
 constexpr uint64_t kChunkCap = 1u << 20;  // chunk table entries
-constexpr uint32_t kCopyPerCu = 64, kCopyPerCuLong = 3, kCopyPerCuFew = 8;
-constexpr uint32_t kFewCopies = 16;  // queries that rarely fill more than kCopyPerCuFew workgroups per CU
-__host__ __device__ inline bool long_copies(uint64_t W, uint64_t nq) { return W >= kLongBatch && W >= nq * kLongQuery; }
+// Up to 16 queries rarely fill more than eight workgroups per CU, and the idle
+// ones of 64 cost 2 to 4 us: 8 / 64 per CU take 42 / 46 us for 8 queries of
+// 335,000 IDs, 47 / 49 for 16, 48 / 48 for 24, 54 / 55 for 32, 73 / 67 for 64.
+constexpr uint32_t kCopyPerCu = 64, kCopyPerCuFew = 8;
+constexpr uint32_t kFewCopies = 16;
 constexpr int kCopyBlock = 256;
 constexpr int kCopyBytes = 64;  // bytes of loads in flight per lane in the copy
 constexpr uint32_t kFlat = 4096;  // positions per flat pass of the copy (16 per lane)
@@ -458,14 +458,13 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_scatter2(const uint32_t* __rest
   }
 }
 
-// IDs per chunk of a batch of nq queries that writes W IDs.
-__host__ __device__ inline uint64_t chunk_len(uint64_t W, uint64_t nq) {
+// IDs per chunk of a batch that writes W IDs.
+__host__ __device__ inline uint64_t chunk_len(uint64_t W) {
   uint64_t c = (W + kChunkCap - 1) / kChunkCap;
   c = (c + 255) & ~255ull;
-  const uint64_t most = long_copies(W, nq) ? kChunkLong : kChunkShort;
-  if (c >= most) return c;
+  if (c >= kMaxChunk) return c;
   uint64_t f = (W / kChunkSpread + 255) & ~255ull;
-  f = f < kMinChunk ? kMinChunk : (f > most ? most : f);
+  f = f < kMinChunk ? kMinChunk : (f > kMaxChunk ? kMaxChunk : f);
   return f > c ? f : c;
 }
 
@@ -712,7 +711,7 @@ __global__ __launch_bounds__(kWave) void k_lv_plan(LvParams<T, IS> P) {
           if (P.host)
             __hip_atomic_store(P.host, static_cast<unsigned long long>(total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
-        const uint32_t L = static_cast<uint32_t>(chunk_len(clip, 1));
+        const uint32_t L = static_cast<uint32_t>(chunk_len(clip));
         auto mark = [&](bool keep, uint32_t at, uint32_t pre, uint32_t c) {
           const uint32_t end = keep ? (pre + c < cw ? pre + c : cw) : 0u;
           mark_chunks(P.chunk_task, at, keep ? (pre + L - 1) / L : 0u, (end + L - 1) / L, lane);
@@ -763,7 +762,7 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_mark(const unsigned long long* 
   const uint32_t q = blockIdx.x * (kLvBlock / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
   if (q >= nq) return;
   const uint32_t nt = ntask[q];
-  const uint64_t L = chunk_len(woff[nq], nq);
+  const uint64_t L = chunk_len(woff[nq]);
   const uint64_t base = woff[q];
   const uint64_t qb = static_cast<uint64_t>(q) * kTaskCap;
   for (uint32_t i0 = 0; i0 < nt; i0 += kWave) {
@@ -807,16 +806,14 @@ __global__ __launch_bounds__(kCopyBlock) void k_lv_copy(const IS* __restrict__ i
                                                         const unsigned long long* __restrict__ woff,
                                                         const unsigned long long* __restrict__ offsets,
                                                         const uint32_t* __restrict__ chunk_task, uint32_t nq,
-                                                        uint32_t long_grid, IS* __restrict__ out) {
+                                                        IS* __restrict__ out) {
   __shared__ uint32_t s_pre[kTaskCap + 1];
   __shared__ uint64_t s_src[kTaskCap];
   const uint64_t W = woff[nq];
-  const uint64_t L = chunk_len(W, nq);
+  const uint64_t L = chunk_len(W);
   const uint64_t nch = (W + L - 1) / L;
   const uint32_t tid = threadIdx.x;
-  const uint32_t grid = long_copies(W, nq) ? long_grid : gridDim.x;
-  if (blockIdx.x >= grid) return;
-  for (uint64_t c = blockIdx.x; c < nch; c += grid) {
+  for (uint64_t c = blockIdx.x; c < nch; c += gridDim.x) {
     const uint32_t e = chunk_task[c];
     uint32_t q = e >> 7, i = e & 127u;
     uint64_t x = c * L;
@@ -1106,7 +1103,7 @@ Status level_search(const SearchArgs& a, const void* key_d, const void* id_d, Le
       const uint32_t per = P.nq <= kFewCopies ? kCopyPerCuFew : kCopyPerCu;
       hipLaunchKernelGGL((k_lv_copy<IS>), dim3(static_cast<unsigned>(cus) * per), dim3(kCopyBlock), 0, s, P.id, sc.tsrc,
                          sc.tpre, sc.ntask, sc.woff, a.offsets, sc.chunk_task, P.nq,
-                         static_cast<uint32_t>(cus) * kCopyPerCuLong, static_cast<IS*>(a.out));
+                         static_cast<IS*>(a.out));
       return hip_status(hipGetLastError(), "Error in launching level search");
     });
   });

@@ -153,13 +153,8 @@ int single_search(pst_tree* t, int kind, int ret, const void* a, const void* b, 
   args.out = out;
   const bool via_index = t->lv_key && ret != PST_RET_POINT;
   if (!t->host) t->host = pst::host_words_take();
-  // a deep tree's walk starts as one workgroup that most searches end in; on
-  // larger trees what that leaves to the rounds outweighs it (us per search,
-  // rounds only / workgroup first, 64 three-sided and 64 stabbing queries:
-  // 2^20 points 135/74 and 194/128, 2^23 170/132 and 255/262, 2^26 177/173
-  // and 253/340)
-  constexpr uint64_t kFrontPoints = 1ull << 23;
-  const bool front = !via_index && t->host && !t->slots_per_tree && !t->debug && t->n <= kFrontPoints;
+  // a deep tree's walk starts as one workgroup that most searches end in
+  const bool front = !via_index && t->host && !t->slots_per_tree && !t->debug;
   unsigned long long host[2] = {0, 0};
   hipError_t e = hipSuccess;
   bool read = true;  // results are copied from the device

@@ -787,8 +787,9 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
 // ---------------------------------------------------------------------------
 // One search on a deep tree, first launch: a workgroup of 1024 threads walks
 // from the root with a stack in LDS, up to 1024 items per step. Small
-// searches end here; a search whose stack outgrows LDS, or that is still
-// walking after kFrontSteps steps, hands its stack to the round kernels. Full
+// searches end here; a search whose stack outgrows LDS, that is still walking
+// after kFrontSteps steps or has filled all threads `wide` times hands its
+// stack to the round kernels. Full
 // subtrees become copy tasks with their output position, which k_front_copy
 // writes in parts of kFrontPart positions.
 //
@@ -804,6 +805,16 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
 constexpr int kFrontBlock = 1024;
 constexpr uint32_t kFrontStack = 7168;  // 56 KB of LDS
 constexpr uint32_t kFrontSteps = 40;
+// Steps of a full workgroup before the rest is handed on: a search that fills
+// the threads once goes on for long on a large tree, and the whole chip does it
+// faster, while on a small tree the rounds cost more than its end. us per
+// search, wide limits 1 / 4 / 16, stabbing searches: 131,075 points 90/39/38,
+// 524,288 104/111/57, 2^20 109/124/125, 2^21 130/148/158, 2^22 179/187/203,
+// 2^23 193/220/238, 2^26 256/319/343 (the rounds alone 93, 120, 151, 165, 167,
+// 180, 239; for a mix of searches 172 on 2^26 points, with this 136, three-sided
+// ones 112 and 43).
+constexpr uint64_t kFrontWidePoints = 1ull << 20;
+constexpr uint32_t kFrontWideSmall = 16, kFrontWideLarge = 1;
 constexpr uint32_t kFrontTasks = 16384;
 constexpr uint32_t kFrontPart = 4096;   // positions per part of a copy
 constexpr uint32_t kFrontParts = 16;    // parts that take turns on a task
@@ -817,7 +828,8 @@ struct FrontTask {
 template <typename T, typename IS, bool RET_POINT>
 __global__ __launch_bounds__(kFrontBlock) void k_front(Params<T, IS> P, FrontTask* __restrict__ tasks,
                                                        uint32_t task_cap, unsigned long long* __restrict__ task_count,
-                                                       uint32_t nctr, unsigned long long* __restrict__ host) {
+                                                       uint32_t nctr, uint32_t wide,
+                                                       unsigned long long* __restrict__ host) {
   using Rec = typename OutRec<T, IS, RET_POINT>::type;
   using It = Items;
   __shared__ uint64_t stack[kFrontStack];
@@ -836,8 +848,9 @@ __global__ __launch_bounds__(kFrontBlock) void k_front(Params<T, IS> P, FrontTas
   }
   uint32_t sp = 1;
   __syncthreads();
-  for (uint32_t step = 0; sp > 0 && sp <= kFrontStack - kFrontBlock && step < kFrontSteps; step++) {
+  for (uint32_t step = 0; sp > 0 && sp <= kFrontStack - kFrontBlock && step < kFrontSteps && wide > 0; step++) {
     const uint32_t n = sp < kFrontBlock ? sp : kFrontBlock;
+    if (n == kFrontBlock) wide--;
     const uint32_t base = sp - n;
     const bool act = tid < n;
     const uint64_t item = act ? stack[base + tid] : 0ull;
@@ -1537,7 +1550,8 @@ Status front_typed(const SearchArgs& a, SearchScratch& sc, bool rounds, unsigned
   const uint32_t cap = a.copy_tasks > 0 ? static_cast<uint32_t>(std::min<size_t>(a.copy_tasks, kFrontTasks)) : kFrontTasks;
   auto* tasks = static_cast<FrontTask*>(sc.front);
   auto* count = reinterpret_cast<unsigned long long*>(tasks + kFrontTasks);
-  k_front<T, IS, RP><<<1, kFrontBlock, 0, s>>>(P, tasks, cap, count, 2 * kMaxRounds + 2, host);
+  const uint32_t wide = a.n >= kFrontWidePoints ? kFrontWideLarge : kFrontWideSmall;
+  k_front<T, IS, RP><<<1, kFrontBlock, 0, s>>>(P, tasks, cap, count, 2 * kMaxRounds + 2, wide, host);
   if (P.copy_max > 0) k_front_copy<T, IS, RP><<<kFrontCopyWaves, kWave, 0, s>>>(P, tasks, count);
   return hip_status(hipGetLastError(), "Error in launching search kernel");
 }

@@ -295,7 +295,7 @@ hipError_t result_alloc_bytes(void** p, size_t bytes) {
     e = malloc_on(dev, p, bytes);
     if (e != hipSuccess) return e;
   }
-  const unsigned long long id = allocation_id(*p);
+  const unsigned long long id = b.id ? b.id : allocation_id(*p);
   if (id == 0) return hipSuccess;  // freed by hipFree
   std::lock_guard<std::mutex> lk(c.mu);
   c.results[*p] = Block{*p, bytes, dev, id};

@@ -787,11 +787,10 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
 // ---------------------------------------------------------------------------
 // One search on a deep tree, first launch: a workgroup of 1024 threads walks
 // from the root with a stack in LDS, up to 1024 items per step. Small
-// searches end here; a search whose stack outgrows LDS, that is still walking
-// after kFrontSteps steps or has filled all threads `wide` times hands its
-// stack to the round kernels. Full
-// subtrees become copy tasks with their output position, which k_front_copy
-// writes in parts of kFrontPart positions.
+// searches end here; a search whose stack grows beyond `most` items, or that is
+// still walking after kFrontSteps steps, hands its stack to the round kernels.
+// Full subtrees become copy tasks with their output position, which
+// k_front_copy writes in parts of kFrontPart positions.
 //
 // Bound by latency: a step is a node load, and the tree's depth in steps is
 // the least a search takes. The four rounds of 7168 one-wave workgroups that
@@ -805,16 +804,16 @@ __global__ __launch_bounds__(kWave) void k_search_round(Params<T, IS> P, uint32_
 constexpr int kFrontBlock = 1024;
 constexpr uint32_t kFrontStack = 7168;  // 56 KB of LDS
 constexpr uint32_t kFrontSteps = 40;
-// Steps of a full workgroup before the rest is handed on: a search that fills
-// the threads once goes on for long on a large tree, and the whole chip does it
-// faster, while on a small tree the rounds cost more than its end. us per
-// search, wide limits 1 / 4 / 16, stabbing searches: 131,075 points 90/39/38,
-// 524,288 104/111/57, 2^20 109/124/125, 2^21 130/148/158, 2^22 179/187/203,
-// 2^23 193/220/238, 2^26 256/319/343 (the rounds alone 93, 120, 151, 165, 167,
-// 180, 239; for a mix of searches 172 on 2^26 points, with this 136, three-sided
-// ones 112 and 43).
-constexpr uint64_t kFrontWidePoints = 1ull << 20;
-constexpr uint32_t kFrontWideSmall = 16, kFrontWideLarge = 1;
+// Stacks that are handed on: on a large tree those that no longer fit the
+// threads, since such a search goes on for long and the whole chip does it
+// faster; on a small one those that LDS does not hold, since the rounds cost
+// more than the search's end. us per stabbing search, stacks of up to 1024 /
+// 3072 / 6144 items: 524,288 points 104/-/57, 2^20 100/122/131, 2^22 172/178/
+// 208, 2^23 180/210/250, 2^26 241/271/348 (rounds alone 120, 151, 167, 180,
+// 239; a mix of searches on 2^26 points 172, with this 129, three-sided ones
+// 112 and 42).
+constexpr uint64_t kFrontLargeTree = 1ull << 20;
+constexpr uint32_t kFrontMost = kFrontStack - kFrontBlock, kFrontMostLarge = kFrontBlock;
 constexpr uint32_t kFrontTasks = 16384;
 constexpr uint32_t kFrontPart = 4096;   // positions per part of a copy
 constexpr uint32_t kFrontParts = 16;    // parts that take turns on a task
@@ -828,7 +827,7 @@ struct FrontTask {
 template <typename T, typename IS, bool RET_POINT>
 __global__ __launch_bounds__(kFrontBlock) void k_front(Params<T, IS> P, FrontTask* __restrict__ tasks,
                                                        uint32_t task_cap, unsigned long long* __restrict__ task_count,
-                                                       uint32_t nctr, uint32_t wide,
+                                                       uint32_t nctr, uint32_t most,
                                                        unsigned long long* __restrict__ host) {
   using Rec = typename OutRec<T, IS, RET_POINT>::type;
   using It = Items;
@@ -848,9 +847,8 @@ __global__ __launch_bounds__(kFrontBlock) void k_front(Params<T, IS> P, FrontTas
   }
   uint32_t sp = 1;
   __syncthreads();
-  for (uint32_t step = 0; sp > 0 && sp <= kFrontStack - kFrontBlock && step < kFrontSteps && wide > 0; step++) {
+  for (uint32_t step = 0; sp > 0 && sp <= most && step < kFrontSteps; step++) {
     const uint32_t n = sp < kFrontBlock ? sp : kFrontBlock;
-    if (n == kFrontBlock) wide--;
     const uint32_t base = sp - n;
     const bool act = tid < n;
     const uint64_t item = act ? stack[base + tid] : 0ull;
@@ -1550,8 +1548,8 @@ Status front_typed(const SearchArgs& a, SearchScratch& sc, bool rounds, unsigned
   const uint32_t cap = a.copy_tasks > 0 ? static_cast<uint32_t>(std::min<size_t>(a.copy_tasks, kFrontTasks)) : kFrontTasks;
   auto* tasks = static_cast<FrontTask*>(sc.front);
   auto* count = reinterpret_cast<unsigned long long*>(tasks + kFrontTasks);
-  const uint32_t wide = a.n >= kFrontWidePoints ? kFrontWideLarge : kFrontWideSmall;
-  k_front<T, IS, RP><<<1, kFrontBlock, 0, s>>>(P, tasks, cap, count, 2 * kMaxRounds + 2, wide, host);
+  const uint32_t most = a.n >= kFrontLargeTree ? kFrontMostLarge : kFrontMost;
+  k_front<T, IS, RP><<<1, kFrontBlock, 0, s>>>(P, tasks, cap, count, 2 * kMaxRounds + 2, most, host);
   if (P.copy_max > 0) k_front_copy<T, IS, RP><<<kFrontCopyWaves, kWave, 0, s>>>(P, tasks, count);
   return hip_status(hipGetLastError(), "Error in launching search kernel");
 }

@@ -1202,8 +1202,8 @@ TreeShape tree_shape(const SearchArgs& a) {
 // on large walks alone, 3 (7) / 3 (8): 1024 on 2^24 712/1730, 907/1703; 640 on
 // 2^25 885/2151, 887/2092; 1024 on 2^25 1339/3354, 1405/2875; 256 on 2^26
 // 839/2632, 835/2633; 400 on 2^26 1196/3170, 1138/3154; 2048 on 2^26 4926, 3877.
-// A pass walks some 4.5M pairs of a group and a point per microsecond. One grab
-// per 2^22 pairs is a fraction of its time, and giving a list's rest to the
+// A count pass walks some 4.5M pairs of a group and a point per microsecond, a
+// write pass half as many. One grab per 2^22 pairs (2^21 of a write pass) is a fraction of its time, and giving a list's rest to the
 // waves that are done first is worth more than that: count passes in us, all
 // lists dealt evenly / one grab per 2^22 pairs / all rests grabbed, 4096 mixed
 // queries on 2^26 points 6252 / 5393 / 5374, 3000 stabbing 6507 / 5838 / 5754.
@@ -1211,8 +1211,11 @@ TreeShape tree_shape(const SearchArgs& a) {
 // 209 / 209 / 543, 3000 on 400,003 126 / 126 / 391, 2048 mixed on 2.5M
 // 244 / 238 / 551, 4096 stabbing on 2^23 1486 / 1499 / 1971. (2^21 pairs: 1989
 // instead of 1745 for 4096 mixed on 2^24; 2^23: 5053 instead of 4599 for 3000
-// stabbing on 50,000,017.)
-constexpr int kGrabShift = 22;
+// stabbing on 50,000,017.) Write passes at one grab per 2^22 / 2^21 / 2^20
+// pairs: 2048 mixed on 2^26 10132 / 9165 / 9192, 2048 stabbing on it 10014 /
+// 8987 / 9021, 4096 stabbing on 2^24 5088 / 5033 / 5711, 4096 mixed on it 4803 /
+// 4711 / 5161, on 2^25 9217 / 9958 / 9883.
+constexpr int kGrabShift = 22, kGrabShiftWrite = 21;
 constexpr uint64_t kSmallTree = 1ull << 21;    // points
 constexpr uint64_t kGroupPoints = 1ull << 14;  // points per group below which groups alone fill the rounds
 constexpr uint64_t kWidePoints = 1ull << 17;   // and from which a round hands on one more doubling,
@@ -1320,7 +1323,7 @@ Status launch_rounds(const SearchArgs& a, SearchScratch& sc, hipStream_t s) {
   const uint32_t grid = static_cast<uint32_t>(cus * occ);
   P.total_waves = grid;
   P.few_items = few_items(a, G, grid);
-  P.grabs = static_cast<uint32_t>(std::min<uint64_t>(a.n * P.ngroups >> kGrabShift, grid));
+  P.grabs = static_cast<uint32_t>(std::min<uint64_t>(a.n * P.ngroups >> (W ? kGrabShiftWrite : kGrabShift), grid));
   const size_t gbytes = static_cast<size_t>(grid) * P.gcap * sizeof(Items::type);
   if (sc.gstack_bytes < gbytes) {
     if (sc.pinned) return Status{1, kPinnedScratchMsg};

@@ -28,11 +28,13 @@
 // Construction: level 0 is one stable radix sort of all points by key (the
 // input in slot order, last-level slots in bit-reversed position order);
 // level t+1 is the stable partition of every level-t run into the runs of
-// the root's left and right children (the root itself dropped). Each
-// point's destination is its child run's closed-form start plus its rank
-// among the points of its run going the same way, from a global prefix
-// count of left- and right-going points (per 4096-point tile, then
-// scanned) less the closed-form count of same-way points in earlier runs.
+// the root's left and right children (the root itself dropped), and level
+// t+2 that of level t+1. One pass over level t writes both (the last level of
+// an odd number takes a pass of its own). A point's destination is its child
+// run's closed-form start plus its rank among the points of its run going the
+// same way, from a global prefix count of the points of each way (per
+// 4096-point tile, then scanned) less the closed-form count of same-way points
+// in earlier runs.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -22,8 +22,9 @@
  *  - Results of the blocking searches are returned as a device array the
  *    library allocates with hipMalloc, of num_elems * sizeof(RetType) bytes
  *    as the reference does (pst/static-pst-gpu.tu:563); release it with
- *    pst_free() or hipFree(). Only the first *num_res_elems entries are
- *    valid; their order is unspecified.
+ *    pst_free() or hipFree(), once; pst_free() keeps arrays of more than
+ *    1 MB for the next result of that size. Only the first *num_res_elems
+ *    entries are valid; their order is unspecified.
  *  - An empty tree prints "Tree is empty; nothing to search" and returns
  *    *num_res_elems = 0, *res_arr_d = NULL (pst/static-pst-gpu.tu:504-510).
  *  - Handles are not shared between threads without external locking; each
